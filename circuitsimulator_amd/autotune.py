@@ -1,22 +1,11 @@
-"""Autotuner for the engine's persistent sweep: the knobs that change how the
-work is cut and which kernel runs it, never the results.
+"""Autotuner for the engine's persistent sweep: the knob that changes how the
+work is cut, never the results.
 
-Exact mode (cse_batch_exact): the sweep's occupancy and the claim cap.
-Kernel 1 runs the exact sweep at seven waves per SIMD, kernel 2 at eight
-(more latency hidden, more values spilled): long launches gain a few percent
-at eight, short ones (a few slices per wave) lose a few, and the engine's
-rule (kernel 0) takes eight from 16 slices per resident wave.  The sweep hands out slices of 64 j, a static first claim per wave
-and then guided self-scheduling from eight counters; `chunk` caps a claim.
-Larger caps cut the per-segment cost (the record load, the lane tables) on
-launches with many slices per wave; the guided claims shrink at the end of
-the queue whatever the cap.
-
-Sampled mode (cse_batch_sampled): the sweep kernel and the item size.  Kernel
-1 is the eight-wave sweep whose hand-scheduled path takes records of at most
-two non-pivot columns (others run compiled code), kernel 2 the eight-wave
-sweep with the general restriction loop (cse_set_sweep_kernel); the item size
-trades per-item cost (record load, tables, flush of the per-record sums)
-against balance.
+`chunk` bounds the terms that one lane takes (cse_sweep.h): deeper trees share
+more of their elimination, shallower ones give more lanes.  The engine's rule
+(0) prices both for the launch at hand; the candidates bound it further.  The
+sweep kernels that a call may name (cse_set_sweep_kernel) are one per mode and
+width, so the kernel half of a candidate changes nothing.
 
 Every setting gives the same terms and the same exact results (integer sums,
 independent of order), so the choice is a timing question only.
@@ -38,16 +27,15 @@ import threading
 
 import numpy as np
 
-# sampled mode: item sizes in j (terms); 64 terms run per asm block, so
-# multiples of 64
+# sampled mode: bounds on a lane's terms
 CANDIDATES = (128, 192, 256, 384, 512, 1024)
 # the sweep kernels of either mode (cse_set_sweep_kernel)
 KERNELS = (1, 2)
-# exact mode: claim caps in j (multiples of the 64-j slice)
+# exact mode: bounds on a lane's terms
 EXACT_CAPS = (256, 512, 1024, 2048, 4096)
-# resident waves per CU of the two packed sweep kernels (4 waves per block)
+# waves per CU that a launch is sized by for the proxy
 _WAVES_PER_CU = {"exact": 7 * 4, "sampled": 8 * 4}
-# packed layout (D in the J rows) up to this width
+# widths up to this share a cache key
 _PACKED_MAX_T = 60
 
 _cache = {}

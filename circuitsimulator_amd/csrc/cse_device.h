@@ -65,13 +65,6 @@ DEV unsigned row_xor32(unsigned v) {
     v ^= dpp_mov<0x128>(v);
     return v;
 }
-DEV unsigned row_or32(unsigned v) {
-    v |= dpp_mov<0xB1>(v);
-    v |= dpp_mov<0x4E>(v);
-    v |= dpp_mov<0x124>(v);
-    v |= dpp_mov<0x128>(v);
-    return v;
-}
 // XOR of v over all lanes, wave-uniform: rows reduced with DPP, the four
 // rows' results (lanes 0, 16, 32, 48) combined in scalar registers
 DEV u64 wave_xor(u64 v) {
@@ -80,14 +73,6 @@ DEV u64 wave_xor(u64 v) {
     const unsigned h = (unsigned)(rl32(hi, 0) ^ rl32(hi, 16) ^ rl32(hi, 32) ^ rl32(hi, 48));
     return ((u64)h << 32) | l;
 }
-// OR of v over all lanes, wave-uniform (as wave_xor)
-DEV u64 wave_or(u64 v) {
-    const int lo = (int)row_or32((unsigned)v), hi = (int)row_or32((unsigned)(v >> 32));
-    const unsigned l = (unsigned)(rl32(lo, 0) | rl32(lo, 16) | rl32(lo, 32) | rl32(lo, 48));
-    const unsigned h = (unsigned)(rl32(hi, 0) | rl32(hi, 16) | rl32(hi, 32) | rl32(hi, 48));
-    return ((u64)h << 32) | l;
-}
-
 // ------------------------------------------------------------------ Philox
 // Philox4x32-10 (Salmon, Moraes, Dror, Shaw, SC'11).
 struct P4 { uint32_t x[4]; };
@@ -401,67 +386,12 @@ template <bool PK> DEV bool as_restrict(AState &s, u64 xi, int alpha) {
     return true;
 }
 
-// Adds 4 x_u x_v (as a function of the affine coordinates) to the form:
-// the coupling of an |00>+|01>+|10>-|11> pair (stateprep.c:45-50).
-template <bool PK> DEV void as_add_coupling(AState &s, int u, int v) {
-    const int gu = (int)((s.G >> u) & 1ull), gv = (int)((s.G >> v) & 1ull);
-    const u64 cu = ballot(lane_in(s.act) && gu), cv = ballot(lane_in(s.act) && gv);
-    const int hu = (int)((s.h >> u) & 1ull), hv = (int)((s.h >> v) & 1ull);
-    s.Q = (s.Q + 4 * (hu & hv)) & 7;
-    // linear part: 4 z_a (hu g_va + hv g_ua + g_ua g_va)
-    const u64 lin = (cv & allmask(hu)) ^ (cu & allmask(hv)) ^ (cu & cv);
-    d_add4<PK>(s, lin);
-    // quadratic part: J_ab ^= g_ua g_vb + g_ub g_va
-    if (lane_in(cu)) s.J ^= cv;
-    if (lane_in(cv)) s.J ^= cu;
-}
-
 // sum_{z in F2^act} w^{q(z)} by eliminating one variable at a time:
 //  D_a in {2,6}: sum over z_a gives sqrt2 w^{s(1-2l)}, l = parity of the
 //    J-row; expanding the parity to second order updates D and J (rank 1);
 //  D_a in {0,4}: sum over z_a gives 2 [l = D_a/4]; a non-empty J-row makes
 //    that a linear constraint, solved by as_eliminate on its last member.
 // Returns eps; p is the exponent of sqrt2, m the phase (mod 8, includes Q).
-// Packed layout, branch-free on the lanes: basis change of pivot i over Sp
-// (as as_basis_change), then z_i = c.  Rows b in Sp: J_b ^= Jc,
-// D_b += D_i + 4 J_bi (and G_b ^= G_i when WITHG); rows x in M: J_x ^= Sp;
-// c = 1 adds D_i to Q, 4 to D_x on M (and G_i to h when WITHG).  The caller
-// retires row i.
-template <bool WITHG> DEV void pk_eliminate(AState &s, int i, u64 Sp, unsigned c) {
-    const u64 Jr = rl64(s.J, i);
-    const unsigned di = (unsigned)(Jr >> 61);
-    const u64 jii = (u64)((di >> 1) & 1u);
-    const u64 Jc = (Jr & CSE_ROWMASK & ~bit(i)) | (jii << i);
-    const u64 M = Jc ^ (Sp & (0ull - jii));
-    const bool inS = lane_in(Sp), inSJ = lane_in(Sp & Jc), inM = lane_in(M);
-    const unsigned jlo = (unsigned)s.J, jhi = (unsigned)(s.J >> 32);
-    const u64 X = (inS ? Jc : 0ull) ^ (inM ? Sp : 0ull);
-    unsigned nhi = (jhi ^ (unsigned)(X >> 32)) + (inS ? (di << 29) : 0u);
-    nhi ^= (inSJ ? 0x80000000u : 0u) ^ ((inM && c) ? 0x80000000u : 0u);
-    s.J = ((u64)nhi << 32) | (jlo ^ (unsigned)X);
-    s.Q = (s.Q + (int)(di & (0u - c))) & 7;
-    if (WITHG) {
-        const u64 Gi = rl64(s.G, i);
-        s.G = inS ? (s.G ^ Gi) : s.G;
-        s.h ^= Gi & (0ull - (u64)c);
-    }
-}
-
-// as_restrict on the packed layout for xi = e_q: {x : x_q = alpha}.  The
-// rows in B (variables fixed to 1 and retired beforehand, never modified
-// since) still contribute to x_q: their part of h is the parity of column q
-// over B, taken from the same ballot as the pivot set.
-DEV bool pk_restrict_coord(AState &s, int q, unsigned alpha, u64 B) {
-    const u64 col = ballot((s.G >> q) & 1ull);
-    const u64 S = col & s.act;
-    const unsigned beta = (alpha ^ (unsigned)(s.h >> q) ^ (unsigned)__popcll(col & B)) & 1u;
-    if (!S) return beta == 0;
-    const int i = __builtin_ctzll(S);
-    pk_eliminate<true>(s, i, S & ~bit(i), beta);
-    s.act &= ~bit(i);
-    return true;
-}
-
 //
 // Packed layout (D_x in bits 61..63 of J_x), the elimination loop scheduled
 // by hand: the compiler's lowering of this loop spends most of its scalar
@@ -470,7 +400,7 @@ DEV bool pk_restrict_coord(AState &s, int q, unsigned alpha, u64 B) {
 //  D_a in {2,6} (bit 62 of J_a): factor sqrt2 w^{s}, s = +1 for 2, -1 for 6;
 //    rows b in eta = J_a & act get J_b ^= eta and D_b -= D_a;
 //  D_a in {0,4}, eta != 0: factor 2 and the constraint eta . z = D_a/4,
-//    solved for i = min(eta) with Sp = eta \ {i} (pk_eliminate, c = D_a/4);
+//    solved for i = min(eta) with Sp = eta \ {i} and c = D_a/4;
 //  D_a in {0,4}, eta = 0: factor 2 (D_a = 0) or the sum vanishes (D_a = 4).
 // Column i and row i are dead after a step, so Jc keeps the stored diagonal
 // bit of row i, M may contain i, and eta (which contains i) stands for Sp.

@@ -36,9 +36,9 @@ struct HostBuf {
 // buffer address its nodes hold.  A call whose key matches replays the graph.
 struct GraphKey {
     int mode, ninst, kernel;
-    long long nrec, nitems, take_max;
+    long long nrec, nitems, stack_words;
     size_t plan_bytes, out_bytes;
-    const void *ptr[8];
+    const void *ptr[9];
 };
 
 struct GraphEntry {
@@ -54,7 +54,7 @@ struct cse_ctx {
     int cus = 0;
     char name[128] = {0};
     char err[512] = {0};
-    DevBuf s1, s2, out, recs, terms, queue, thr, sexp, L, idx, errflag, lsh;
+    DevBuf s1, s2, out, recs, terms, queue, thr, sexp, L, idx, errflag, lsh, stack;
     // a batch's plan: instance descriptors, item and record offsets and
     // projectors in one allocation, laid out as the pinned staging buffer
     DevBuf plan;
@@ -76,6 +76,7 @@ struct cse_ctx {
     // the static scratch array (cse_exact_projector_noalloc)
     char *b_plan = nullptr, *b_out = nullptr, *b_hup = nullptr, *b_hstage = nullptr;
     uint64_t *b_recs = nullptr;
+    uint32_t *b_stack = nullptr;
     unsigned long long *b_queue = nullptr;
     int32_t *b_sexp1 = nullptr, *b_terms = nullptr;
     // batched calls replayed from captured HIP graphs (cse_set_graphs)
@@ -87,7 +88,6 @@ struct cse_ctx {
     char *scratch = nullptr;
     char scratch_err[160] = {0};
     bool thr_ready = false;
-    int blocks_per_cu = 8;  // persistent grid: blocks of 4 waves per CU
     int sweep_kernel[2] = {0, 0};  // per mode (cse_set_sweep_kernel)
     // exact mode: terms of one instance after which a wave flushes its
     // partial histogram (CSE_FLUSH_TERMS in the environment, at most and by
@@ -104,14 +104,14 @@ struct cse_ctx {
 // that device is created, and host code only ever uses that address.
 constexpr int kStaticMaxLogChi = 13;
 constexpr long long kStaticMaxChi = 1ll << kStaticMaxLogChi;
-constexpr size_t kStaticPlanBytes = 4096;  // one instance's plan: 2,816 B
+constexpr size_t kStaticPlanBytes = 4096;  // one instance: 3,072 B
 constexpr size_t kStaticOutBytes = 8448;   // one instance's results block: 8,288 B
 constexpr size_t kScratchQueue = 0;
-constexpr size_t kScratchPlan = 8 * CSE_QUEUE_WORDS;
+constexpr size_t kScratchPlan = 256;
 constexpr size_t kScratchOut = kScratchPlan + kStaticPlanBytes;
 constexpr size_t kScratchSexp = kScratchOut + kStaticOutBytes;
 constexpr size_t kScratchRecs = kScratchSexp + 4 * (size_t)kStaticMaxChi;
-constexpr size_t kScratchBytes = kScratchRecs + (size_t)REC_WORDS * 8 * (size_t)kStaticMaxChi;  // 8,762,624 B
+constexpr size_t kScratchBytes = kScratchRecs + (size_t)REC_WORDS * 8 * (size_t)kStaticMaxChi;  // 4,502,016 B
 static_assert(kScratchOut % 256 == 0 && kScratchSexp % 256 == 0 && kScratchRecs % 256 == 0, "scratch parts aligned");
 
 static __device__ __align__(256) unsigned char scratch[kScratchBytes];
@@ -254,37 +254,6 @@ double elapsed(hipEvent_t a, hipEvent_t b) {
     return (double)ms;
 }
 
-int default_chunk(long long chi, int size = 256) {
-    long long c = size;
-    if (chi < c) c = chi;
-    return (int)(c < 1 ? 1 : c);
-}
-
-// Exact mode's default largest claim: 512 j when the launch still has eight
-// items of that size per resident wave of k_sweep_packed_all (seven waves per
-// SIMD), else 256.  Larger claims halve the per-segment record load, table
-// set-up and histogram flush; the guided self-scheduling of the sweep shrinks
-// the claims at the end of the queue in any case.
-int exact_chunk(cse_ctx *ctx, const cse_instance *in, int ninst) {
-    long long items = 0;
-    for (int i = 0; i < ninst; i++) {
-        const long long chi = in[i].exact ? (1ll << ((in[i].P.nqubits + 1) / 2)) : (1ll << in[i].k);
-        // items of record r that reach the diagonal or beyond
-        const long long per = (chi + 511) / 512;
-        items += chi * (per + 1) / 2;
-    }
-    const long long waves = (long long)ctx->cus * CSE_EXACT_BLOCKS_PER_CU * 4;
-    return items >= 8 * waves ? 512 : 256;
-}
-
-// Persistent grid for k_sweep: bpc resident blocks of 4 waves per CU
-int sweep_grid(cse_ctx *ctx, long long nitems, int bpc) {
-    long long g = (long long)ctx->cus * bpc;
-    long long need = (nitems + 3) / 4;
-    if (need < g) g = need;
-    return (int)(g < 1 ? 1 : g);
-}
-
 // Records for instances [0, ninst): mode 0 random states (sample indices
 // first + i), mode 1 projected decomposition states.  Then the sweep.
 struct Plan {
@@ -294,7 +263,9 @@ struct Plan {
     long long *item_off = nullptr;  // ninst + 1
     DevProjector *projs = nullptr;
     long long nrec = 0, nitems = 0, nterms = 0;
-    long long take_max = 1;  // exact mode: largest claim, in slices of 64 j
+    long long stack_words = 0;  // per lane and wave, beyond LDS
+    int nmax = 0;
+    bool anyH = false;
     // appends an instance of nr records, ni work items and nt terms (its
     // record and term offsets are set here)
     void add(InstDesc d, const DevProjector &p, long long nr, long long ni, long long nt) {
@@ -307,6 +278,9 @@ struct Plan {
         nitems += ni;
         nterms += nt;
         ninst++;
+        nmax = std::max(nmax, d.n);
+        anyH = anyH || d.exact;
+        stack_words = std::max(stack_words, (long long)d.spare);
         rec_off[ninst] = nrec;
         item_off[ninst] = nitems;
     }
@@ -412,6 +386,32 @@ OutLayout out_layout(const Plan &pl, int mode) {
     return o;
 }
 
+// The sweep kernel of a launch, by its widest state (slots beyond 32 cost
+// registers: 128 VGPRs, four waves per SIMD, up to 48 slots, three waves
+// beyond) and whether some instance has |H^t> terms (their signs cost four
+// instructions a step).
+typedef void (*SweepFn)(SweepArgs);
+struct SweepKernel {
+    int id;
+    SweepFn fn;
+    int blocks_per_cu;
+};
+SweepKernel sweep_choice(const Plan &pl, int mode) {
+    static const SweepFn fn[2][2][3] = {{{k_sweep_s32, k_sweep_s48, k_sweep_s64}, {k_sweep_sh32, k_sweep_sh48, k_sweep_sh64}},
+                                        {{k_sweep_e32, k_sweep_e48, k_sweep_e64}, {k_sweep_eh32, k_sweep_eh48, k_sweep_eh64}}};
+    const int w = pl.nmax <= 32 ? 0 : pl.nmax <= 48 ? 1 : 2, h = pl.anyH ? 1 : 0;
+    SweepKernel k;
+    k.id = (mode * 2 + h) * 3 + w;
+    k.fn = fn[mode][h][w];
+    k.blocks_per_cu = w == 2 ? 3 : 4;
+    return k;
+}
+
+// persistent grid: the resident blocks, or the items if they are fewer
+int sweep_grid(const cse_ctx *ctx, const Plan &pl, const SweepKernel &k) {
+    return (int)std::max(1ll, std::min((long long)ctx->cus * k.blocks_per_cu, pl.nitems));
+}
+
 // Binds a batch to the context's own buffers, grown on demand (device memory
 // and pinned host stages).
 int bind_ctx_mem(cse_ctx *ctx, const Plan &pl, int mode, bool want_terms) {
@@ -421,7 +421,8 @@ int bind_ctx_mem(cse_ctx *ctx, const Plan &pl, int mode, bool want_terms) {
     ENSURE(plan, pbytes);
     ENSURE(outb, o.total);
     ENSURE(recs, (size_t)REC_WORDS * 8 * (size_t)pl.nrec);
-    ENSURE(queue, 8 * CSE_QUEUE_WORDS);
+    ENSURE(queue, 8);
+    ENSURE(stack, (size_t)pl.stack_words * 64 * 4 * 4 * (size_t)sweep_grid(ctx, pl, sweep_choice(pl, mode)));
     if (mode == 1) ENSURE(sexp, 4 * (size_t)pl.nrec);
     if (want_terms) ENSURE(terms, 4 * (size_t)(pl.nterms > 0 ? pl.nterms : 1));
     int rc = ensure_host(ctx, ctx->hup, pbytes);
@@ -431,6 +432,7 @@ int bind_ctx_mem(cse_ctx *ctx, const Plan &pl, int mode, bool want_terms) {
     ctx->b_out = (char *)ctx->outb.p;
     ctx->b_recs = dp<uint64_t>(ctx->recs);
     ctx->b_queue = dp<unsigned long long>(ctx->queue);
+    ctx->b_stack = dp<uint32_t>(ctx->stack);
     ctx->b_sexp1 = mode == 1 ? dp<int32_t>(ctx->sexp) : nullptr;
     ctx->b_terms = want_terms ? dp<int32_t>(ctx->terms) : nullptr;
     ctx->b_hup = (char *)ctx->hup.p;
@@ -455,6 +457,7 @@ int bind_static_mem(cse_ctx *ctx, const Plan &pl, char *hup, char *hstage) {
     ctx->b_out = ctx->scratch + kScratchOut;
     ctx->b_sexp1 = (int32_t *)(ctx->scratch + kScratchSexp);
     ctx->b_recs = (uint64_t *)(ctx->scratch + kScratchRecs);
+    ctx->b_stack = nullptr;  // its trees stay in LDS
     ctx->b_terms = nullptr;
     ctx->b_hup = hup;
     ctx->b_hstage = hstage;
@@ -476,77 +479,29 @@ int prep_batch(cse_ctx *ctx, const Plan &pl, int mode) {
     ZeroList zl;
     memset(&zl, 0, sizeof(zl));
     zl_add(zl, b, (long long)(o.total / 8));
-    zl_add(zl, ctx->b_queue, CSE_QUEUE_WORDS);
+    zl_add(zl, ctx->b_queue, 1);
     return zero_list(ctx, zl);
 }
 
-enum SweepKernel { SK_GENERIC, SK_PACKED, SK_PACKED_GEN, SK_ALL, SK_ALL8 };
-
-// The sweep kernel of a launch.  Exact mode takes k_sweep_packed_all (seven
-// waves per SIMD) or k_sweep_packed_all8 (eight) as set, and by the engine's
-// rule the eight-wave kernel when the launch holds at least
-// CSE_ALL8_SLICES_PER_WAVE slices for each of its waves: a long launch gains
-// from the extra wave's latency hiding (the uneven batch 2.5%, the t=30 |H^t>
-// projector 2.6%), a short one loses more to its spills than it gains (one
-// projector of 2,048 records, 4.6 slices per wave: 4.5%).  Sampled launches take
-// k_sweep_packed (eight waves, the two-column asm path for |L> terms), or
-// k_sweep_packed_gen when set or when every term is an |H^t> term: that
-// kernel runs an aligned batch of |H^t> terms as eight groups of 8 that share
-// the pair operations of bits 3..5 of j.  Records of n > 60 take k_sweep.
-SweepKernel sweep_choice(const cse_ctx *ctx, const Plan &pl, int mode) {
-    bool packed = true, allH = true;
-    for (int i = 0; i < pl.ninst; i++) {
-        packed = packed && pl.inst[i].n <= CSE_END_ROW;
-        allH = allH && pl.inst[i].exact;
-    }
-    if (!packed) return SK_GENERIC;
-    if (mode == 1) {
-        const int k = ctx->sweep_kernel[1];
-        if (k) return k == 2 ? SK_ALL8 : SK_ALL;
-        return pl.nitems >= CSE_ALL8_SLICES_PER_WAVE * 32ll * ctx->cus ? SK_ALL8 : SK_ALL;
-    }
-    const int k = ctx->sweep_kernel[0];
-    return k == 2 || (k == 0 && allH) ? SK_PACKED_GEN : SK_PACKED;
-}
-
 int run_sweep(cse_ctx *ctx, const Plan &pl, int mode, bool want_terms) {
-    const int ninst = pl.ninst;
     SweepArgs A;
-    A.mode = mode;
-    A.ninst = ninst;
+    memset(&A, 0, sizeof(A));
+    A.ninst = pl.ninst;
     A.nitems = pl.nitems;
     A.item_off = ctx->d_itemoff;
+    A.flush_terms = ctx->flush_terms;
     A.inst = ctx->d_inst;
     A.recs = ctx->b_recs;
     A.queue = ctx->b_queue;
+    A.stack = ctx->b_stack;
+    A.stack_words = pl.stack_words;
     A.terms = want_terms ? ctx->b_terms : nullptr;
     A.zsum = ctx->d_zsum;
     A.kahan = ctx->d_kahan;
     A.hist = ctx->d_hist;
-    A.hist_stride = HIST_STRIDE;
     A.ips = ctx->d_ips;
-    A.err = ctx->d_err;
-    const SweepKernel sk = sweep_choice(ctx, pl, mode);
-    const int grid = sweep_grid(ctx, pl.nitems, sk == SK_ALL8 ? 8 : sk == SK_ALL ? CSE_EXACT_BLOCKS_PER_CU
-                                                                                 : ctx->blocks_per_cu);
-    A.take_max = pl.take_max;
-    A.flush_terms = ctx->flush_terms;
-    // the static first claims cover about 1 / CSE_STATIC_DIV of the slices
-    // (at most take_max per wave); the rest is cut into CSE_NQUEUES parts
-    const long long waves = 4ll * grid;
-    A.first_take = pl.nitems / (CSE_STATIC_DIV * waves);
-    if (A.first_take > A.take_max) A.first_take = A.take_max;
-    if (A.first_take < 1) A.first_take = 1;
-    A.static_end = A.first_take * waves < pl.nitems ? A.first_take * waves : pl.nitems;
-    A.part = (pl.nitems - A.static_end + CSE_NQUEUES - 1) / CSE_NQUEUES;
-    A.waves_per_part = (waves + CSE_NQUEUES - 1) / CSE_NQUEUES;
-    switch (sk) {
-    case SK_ALL8: hipLaunchKernelGGL(k_sweep_packed_all8, dim3(grid), dim3(256), 0, ctx->stream, A); break;
-    case SK_ALL: hipLaunchKernelGGL(k_sweep_packed_all, dim3(grid), dim3(256), 0, ctx->stream, A); break;
-    case SK_PACKED_GEN: hipLaunchKernelGGL(k_sweep_packed_gen, dim3(grid), dim3(256), 0, ctx->stream, A); break;
-    case SK_PACKED: hipLaunchKernelGGL(k_sweep_packed, dim3(grid), dim3(256), 0, ctx->stream, A); break;
-    default: hipLaunchKernelGGL(k_sweep, dim3(grid), dim3(256), 0, ctx->stream, A); break;
-    }
+    const SweepKernel k = sweep_choice(pl, mode);
+    hipLaunchKernelGGL(k.fn, dim3(sweep_grid(ctx, pl, k)), dim3(256), 0, ctx->stream, A);
     HIPCHK(hipGetLastError());
     return CSE_OK;
 }
@@ -582,13 +537,13 @@ int run_batch(cse_ctx *ctx, const Plan &pl, int mode, bool want_terms, size_t pl
     memset(&key, 0, sizeof(key));
     key.mode = mode;
     key.ninst = pl.ninst;
-    key.kernel = (int)sweep_choice(ctx, pl, mode);
+    key.kernel = sweep_choice(pl, mode).id;
     key.nrec = pl.nrec;
     key.nitems = pl.nitems;
-    key.take_max = pl.take_max;
+    key.stack_words = pl.stack_words;
     key.plan_bytes = plan_bytes;
     key.out_bytes = out_layout(pl, mode).total;
-    const void *ptr[8] = {ctx->b_plan, ctx->b_out, ctx->b_recs, ctx->b_queue,
+    const void *ptr[9] = {ctx->b_plan, ctx->b_out, ctx->b_recs, ctx->b_queue, ctx->b_stack,
                           ctx->b_sexp1, ctx->b_hup, ctx->b_hstage, mode == 0 ? ctx->thr.p : nullptr};
     memcpy(key.ptr, ptr, sizeof(ptr));
     GraphEntry *hit = nullptr;
@@ -635,18 +590,103 @@ int run_batch(cse_ctx *ctx, const Plan &pl, int mode, bool want_terms, size_t pl
     return CSE_OK;
 }
 
-InstDesc make_inst(int t, int k, int exact, const uint64_t *L, int chunk) {
+// Cost model of a lane's tree, in VALU instructions: a step of slot c takes
+// about 31 for its own state (a signed one, |H^t>, 4 more) and 6 for every
+// slot below it, a slot beyond 32 twice that; a term's sums take about 70.
+double step_cost(int c, bool h) {
+    return c < 32 ? 31.0 + (h ? 4 : 0) + 6.0 * c : 60.0 + (h ? 6 : 0) + 6.0 * 32 + 11.0 * (c - 32);
+}
+
+// G, the slot order and the stack of an instance.  G takes the largest share
+// of the work off the terms as long as the launch keeps the chip busy: with W
+// the instructions of one lane's tree, the launch takes about 4 W cycles for
+// its last wave plus 4 W per wave that each SIMD runs, and the G of the least
+// sum is taken (an instance of a batch bears its share of the last wave).
+// max_words: LDS words when the stack has to stay there.
+void plan_tree(InstDesc &d, int mode, int simds, int ninst, bool lds_only, int max_terms) {
+    const int lds = mode == 0 ? TREE_LDS_WORDS0 : TREE_LDS_WORDS1;
+    double best = 0.0, path[TREE_MAXG + 1];
+    // path[g]: steps of the slots from ub[g] up to ub[g + 1]
+    auto steps = [&](int lo, int hi) {
+        double w = 0;
+        for (int c = lo; c < hi; c++) w += step_cost(c, d.exact);
+        return w;
+    };
+    const int top = std::min(d.k, TREE_MAXG);
+    int words = 0;
+    d.G = 0;
+    double below = 0.0;  // steps of the slots below ub[g], per term
+    for (int g = 0; g <= top; g++) {
+        if (g > 0) {
+            if (d.ub[g] > 32 || (1ll << g) > max_terms) break;
+            words += TREE_STATE_WORDS + d.ub[g];
+            if (lds_only && words > lds) break;
+            path[g - 1] = steps(d.ub[g - 1], d.ub[g]);
+            below += path[g - 1] / (double)(1ll << (g - 1));
+        }
+        const double terms = (double)(1ll << g);
+        const double W = (below + 70.0) * terms + steps(d.ub[g], d.n) + 500.0;
+        const double nrec = mode == 0 ? (double)d.lanes : (double)d.chi;
+        const double lanes = nrec * (double)(d.chi >> g) * (mode == 0 ? 1.0 : 0.5);
+        const double f = W / ninst + W * std::max(lanes / 64.0, 1.0) / simds;
+        if (g == 0 || f < best) {
+            best = f;
+            d.G = g;
+        }
+    }
+    words = 0;
+    d.nlds = 0;
+    int beyond = 0;
+    for (int g = 1; g <= d.G; g++) {
+        const int w = TREE_STATE_WORDS + d.ub[g];
+        if (d.nlds == g - 1 && words + w <= lds) {
+            d.soff[g] = (uint16_t)words;
+            words += w;
+            d.nlds = g;
+        } else {
+            d.soff[g] = (uint16_t)beyond;
+            beyond += w;
+        }
+    }
+    d.spare = beyond;
+}
+
+// mode 0: nsamp records; mode 1: chi records.  max_terms > 0 bounds the terms
+// of a lane (the calls' chunk).
+InstDesc make_inst(const cse_ctx *ctx, int mode, int t, int k, int exact, const uint64_t *L, long long nsamp,
+                   int ninst, bool lds_only, int max_terms) {
     InstDesc d;
     memset(&d, 0, sizeof(d));
     d.n = t;
-    d.k = exact ? 0 : k;
+    d.k = exact ? (t + 1) / 2 : k;
     d.exact = exact ? 1 : 0;
-    d.chi = exact ? (1ll << ((t + 1) / 2)) : (1ll << k);
-    d.chunk = default_chunk(d.chi, chunk > 0 ? chunk : 256);
-    if (d.chunk > d.chi) d.chunk = (int)d.chi;
-    d.nchunks = (d.chi + d.chunk - 1) / d.chunk;
-    if (!exact)
-        for (int r = 0; r < k; r++) d.L[r] = L[r];
+    d.chi = 1ll << d.k;
+    uint8_t col[64];
+    if (exact) {
+        // bit b of j is pair size-1-b; its slots are u = x_2q (signed) below
+        // s = x_2q + x_2q+1, and the lone qubit of odd t is slot 0
+        const int odd = t & 1;
+        for (int b = 0; b < d.k; b++) {
+            const int q = d.k - 1 - b, u = 2 * b - odd, s = u + 1;
+            col[s] = (uint8_t)(odd && b == 0 ? t - 1 : 2 * q + 1);
+            if (u >= 0) col[u] = (uint8_t)(2 * q);
+            d.LP[b] = 1ull << s;
+            d.L[b] = u >= 0 ? 1ull << u : 0ull;
+            d.jmap[b] = 1u << b;
+            if (b < TREE_MAXG) d.ub[b + 1] = (uint8_t)(s + 1);
+        }
+    } else {
+        cse_chain_basis(t, k, L, TREE_MAXG, d.L, d.jmap, d.ub, col);
+        uint8_t pos[64];
+        for (int p = 0; p < t; p++) pos[col[p]] = (uint8_t)p;
+        for (int b = 0; b < k; b++)
+            for (uint64_t r = d.L[b]; r; r &= r - 1) d.LP[b] |= 1ull << pos[__builtin_ctzll(r)];
+    }
+    for (int p = 0; p < 64; p++) d.inv[p] = p < t ? col[p] : (uint8_t)p;
+    d.lanes = nsamp;
+    plan_tree(d, mode, 4 * ctx->cus, ninst, lds_only, max_terms > 0 ? max_terms : 1 << 30);
+    const long long per = d.chi >> d.G;
+    d.lanes = mode == 0 ? nsamp * per : tri_before(1ll << d.G, per, per);
     return d;
 }
 
@@ -766,7 +806,7 @@ void cse_destroy(cse_ctx *ctx) {
         if (g.exec) (void)hipGraphExecDestroy(g.exec);
     ctx->graphs.clear();
     DevBuf *bufs[] = {&ctx->s1, &ctx->s2, &ctx->out, &ctx->recs, &ctx->terms, &ctx->queue, &ctx->thr,
-                      &ctx->sexp, &ctx->L, &ctx->idx, &ctx->errflag, &ctx->lsh, &ctx->plan, &ctx->outb};
+                      &ctx->sexp, &ctx->L, &ctx->idx, &ctx->errflag, &ctx->lsh, &ctx->plan, &ctx->outb, &ctx->stack};
     for (DevBuf *b : bufs)
         if (b->p) (void)hipFree(b->p);
     if (ctx->hstage.p) (void)hipHostFree(ctx->hstage.p);
@@ -952,10 +992,10 @@ static int sampled_batch(cse_ctx *ctx, const cse_sampled_instance *in, int ninst
     Plan pl = store.plan();
     bool want_terms = false;
     for (int i = 0; i < ninst; i++) {
-        InstDesc d = make_inst(in[i].P.nqubits, in[i].k, in[i].exact, in[i].L, chunk);
+        InstDesc d = make_inst(ctx, 0, in[i].P.nqubits, in[i].k, in[i].exact, in[i].L, in[i].count, ninst, false, chunk);
         d.seed = in[i].seed;
         d.first = in[i].first;
-        pl.add(d, to_dev(&in[i].P), in[i].count, in[i].count * d.nchunks, in[i].count * d.chi);
+        pl.add(d, to_dev(&in[i].P), in[i].count, (d.lanes + 255) / 256, in[i].count * d.chi);
         want_terms = want_terms || res[i].terms != nullptr;
     }
     if (pl.nrec > kMaxSamples) return fail(ctx, CSE_ERR_ARG, "%lld samples above 2^24 per call", pl.nrec);
@@ -983,7 +1023,6 @@ static int sampled_batch(cse_ctx *ctx, const cse_sampled_instance *in, int ninst
     HIPCHK(hipStreamSynchronize(ctx->stream));
     const int errv = *errp;
     if (errv & 1) return fail(ctx, CSE_ERR_RNG, "random state draw exceeded its shrink cap");
-    if (errv & 2) return fail(ctx, CSE_ERR_HIP, "internal: an inner product exponent left [-64, 0]");
     // a replayed graph is timed as a whole (records and sweep together)
     const double pms = graphed ? 0.0 : elapsed(ctx->e0, ctx->e1);
     const double kms = graphed ? elapsed(ctx->e0, ctx->e2) : elapsed(ctx->e1, ctx->e2);
@@ -1067,7 +1106,6 @@ int cse_batch_sampled(cse_ctx *ctx, const cse_sampled_instance *inst, int ninst,
 static int exact_batch(cse_ctx *ctx, const cse_instance *in, int ninst, int chunk, cse_exact_result *res,
                        int32_t *terms_out, double *kernel_ms, bool use_static = false, char *hup = nullptr,
                        char *hstage = nullptr) {
-    if (chunk <= 0) chunk = exact_chunk(ctx, in, ninst);
     // the static path keeps its one-instance plan on the stack
     InstDesc s_inst[1];
     long long s_ro[2], s_io[2];
@@ -1081,11 +1119,10 @@ static int exact_batch(cse_ctx *ctx, const cse_instance *in, int ninst, int chun
         pl.item_off = s_io;
         pl.projs = s_pj;
     }
-    // items are slices of CSE_SLICE_J j; a claim takes at most chunk / CSE_SLICE_J of them
-    pl.take_max = chunk / CSE_SLICE_J > 1 ? chunk / CSE_SLICE_J : 1;
     for (int i = 0; i < ninst; i++) {
-        const InstDesc d = make_inst(in[i].P.nqubits, in[i].k, in[i].exact, in[i].L, CSE_SLICE_J);
-        pl.add(d, to_dev(&in[i].P), d.chi, tri_items(d.chi, d.chunk, d.nchunks), d.chi * (d.chi + 1) / 2);
+        const InstDesc d =
+            make_inst(ctx, 1, in[i].P.nqubits, in[i].k, in[i].exact, in[i].L, 0, ninst, use_static, chunk);
+        pl.add(d, to_dev(&in[i].P), d.chi, (d.lanes + 255) / 256, d.chi * (d.chi + 1) / 2);
     }
     if (terms_out && pl.nterms > (1ll << 31)) return fail(ctx, CSE_ERR_ARG, "per-term output too large");
     int rc = use_static ? bind_static_mem(ctx, pl, hup, hstage) : bind_ctx_mem(ctx, pl, 1, terms_out != nullptr);
@@ -1105,11 +1142,9 @@ static int exact_batch(cse_ctx *ctx, const cse_instance *in, int ninst, int chun
     const unsigned long long *hist = (const unsigned long long *)(hs + o.hist);
     const double *kz = (const double *)(hs + o.kahan);
     const unsigned long long *nips = (const unsigned long long *)(hs + o.ips);
-    int *errp = (int *)(hs + o.err);
     if (terms_out)
         HIPCHK(hipMemcpyAsync(terms_out, ctx->b_terms, 4 * (size_t)pl.nterms, hipMemcpyDeviceToHost, ctx->stream));
     HIPCHK(hipStreamSynchronize(ctx->stream));
-    if (*errp & 2) return fail(ctx, CSE_ERR_HIP, "internal: an inner product exponent left [-64, 0]");
     const double tms = elapsed(ctx->e0, ctx->e2);
     const double kms = graphed ? tms : elapsed(ctx->e1, ctx->e2);
     if (kernel_ms) *kernel_ms = kms;

@@ -265,6 +265,103 @@ void cse_sampled_estimators(int t, int64_t count, const long long *z, const int3
     cse_est_finish(&part, 1, t, count, mean, mean_kahan);
 }
 
+/* The row of least weight outside U among the nonzero combinations of the m
+ * rows w, by Gray code: *best gets the combination's mask. */
+#if defined(__x86_64__) && defined(__GNUC__) && !defined(__clang__)
+__attribute__((target_clones("popcnt", "default")))
+#endif
+static uint64_t lightest(const uint64_t *w, int m, uint64_t U, uint32_t *best) {
+    uint64_t x = 0, bx = 0;
+    int bw = 65;
+    uint32_t at = 1;
+    for (uint32_t i = 1; i < (1u << m); i++) {
+        x ^= w[__builtin_ctz(i)];
+        const int c = __builtin_popcountll(x & ~U);
+        if (c < bw) {
+            bw = c;
+            bx = x;
+            at = i;
+        }
+    }
+    *best = at ^ (at >> 1);
+    return bx;
+}
+
+/* Combinations are searched among at most this many rows at a time. */
+#define CHAIN_SEARCH 12
+
+void cse_chain_basis(int t, int k, const uint64_t *L, int levels, uint64_t *rows, uint32_t *jmap, uint8_t *ub,
+                     uint8_t *col) {
+    uint64_t w[32], U = 0;
+    uint32_t m[32];
+    int left = k, nc = 0;
+    for (int b = 0; b < k; b++) {
+        w[b] = L[k - 1 - b];
+        m[b] = 1u << b;
+    }
+    ub[0] = 0;
+    for (int g = 0; g < k; g++) {
+        uint32_t pick = 1;
+        uint64_t x = w[0];
+        if (g < levels) {
+            if (left > CHAIN_SEARCH) {
+                /* reduced row echelon form outside U: the lightest rows of a
+                 * systematic basis first */
+                int done = 0;
+                for (int q = 0; q < t && done < left; q++) {
+                    if ((U >> q) & 1) continue;
+                    int p = done;
+                    while (p < left && !((w[p] >> q) & 1)) p++;
+                    if (p == left) continue;
+                    uint64_t tw = w[p];
+                    uint32_t tm = m[p];
+                    w[p] = w[done];
+                    m[p] = m[done];
+                    w[done] = tw;
+                    m[done] = tm;
+                    for (p = 0; p < left; p++)
+                        if (p != done && ((w[p] >> q) & 1)) {
+                            w[p] ^= tw;
+                            m[p] ^= tm;
+                        }
+                    done++;
+                }
+                for (int a = 1; a < left; a++) {
+                    const uint64_t tw = w[a];
+                    const uint32_t tm = m[a];
+                    const int c = __builtin_popcountll(tw & ~U);
+                    int b = a;
+                    for (; b > 0 && __builtin_popcountll(w[b - 1] & ~U) > c; b--) {
+                        w[b] = w[b - 1];
+                        m[b] = m[b - 1];
+                    }
+                    w[b] = tw;
+                    m[b] = tm;
+                }
+            }
+            x = lightest(w, left < CHAIN_SEARCH ? left : CHAIN_SEARCH, U, &pick);
+        }
+        uint32_t jm = 0;
+        for (int b = 0; b < left; b++)
+            if (b < 32 && ((pick >> b) & 1)) jm ^= m[b];
+        rows[g] = x;
+        jmap[g] = jm;
+        for (int q = 0; q < t; q++)
+            if (((x & ~U) >> q) & 1) col[nc++] = (uint8_t)q;
+        U |= x;
+        if (g < levels) ub[g + 1] = (uint8_t)nc;
+        /* one row of the combination makes room (the rest still spans) */
+        const int out = __builtin_ctz(pick);
+        for (int b = out; b + 1 < left; b++) {
+            w[b] = w[b + 1];
+            m[b] = m[b + 1];
+        }
+        left--;
+    }
+    for (int q = 0; q < t; q++)
+        if (!((U >> q) & 1)) col[nc++] = (uint8_t)q;
+}
+
 /* ------------------------------------------------------------- rank */
 int cse_gf2_rank(const uint64_t *rows, int k)
 {

@@ -38,6 +38,15 @@ void cse_est_accumulate(cse_est_part *part, int t, int64_t lo, int64_t hi, const
 void cse_est_finish(const cse_est_part *parts, int nparts, int t, int64_t count, double *mean,
                     double *mean_kahan);
 
+/* A basis of the row combinations x_j = sum_b j_b L[k-1-b] of L (k <= 30 rows
+ * of t bits) in which the first rows move few columns: rows[i] and the index
+ * mask jmap[i] it stands for, each of the first `levels` rows the combination
+ * (of those left) that adds the fewest columns to the ones moved so far;
+ * ub[g] = columns moved by rows 0 .. g - 1 (ub[0] = 0), col[] = all t columns
+ * in the order in which the rows reach them. */
+void cse_chain_basis(int t, int k, const uint64_t *L, int levels, uint64_t *rows, uint32_t *jmap, uint8_t *ub,
+                     uint8_t *col);
+
 /* GF(2) rank of k rows of t bits (matrix.c:676-724 semantics) */
 int cse_gf2_rank(const uint64_t *rows, int k);
 

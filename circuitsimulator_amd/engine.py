@@ -183,12 +183,9 @@ class Engine:
         self._check(self._L.cse_set_graphs(self.h, 1 if enable else 0))
 
     def set_sweep_kernel(self, kernel, mode=0):
-        """sweep kernel of one mode (cse_set_sweep_kernel): sampled (mode 0):
-        0 the engine's choice (2 for calls of |H^t> instances only, else 1),
-        1 the eight-wave kernel with the two-column asm path, 2 the general
-        one; exact (mode 1): 0 the engine's choice (2 for launches of at
-        least 16 slices per resident wave, else 1), 1 seven waves per SIMD,
-        2 eight"""
+        """sweep kernel of one mode (cse_set_sweep_kernel), 0 sampled, 1
+        exact: 0 the engine's choice; 1 and 2 are accepted and run the same
+        kernel"""
         self._check(self._L.cse_set_sweep_kernel(self.h, int(mode), int(kernel)))
         self.sweep_kernels[int(mode)] = int(kernel)
 
@@ -286,8 +283,8 @@ class Engine:
 
     def batch_exact(self, instances, chunk=0, want_terms=False, nterms=0):
         """instances: a list of Instance or an instance_array.  chunk: the
-        claim cap in j (0: the engine's default; "auto": the autotuner's
-        choice of kernel and cap for this call)."""
+        most terms that one lane takes (0: the engine's rule; "auto": the
+        autotuner's choice for this call)."""
         res, terms, ms = self._batch_exact(instances, chunk, want_terms, nterms)
         return list(res), terms, ms
 
@@ -332,8 +329,8 @@ class Engine:
         """instances: a contiguous sampled_instance_array -> (means, results,
         kernel ms, samples); means[i] is cse_sampled_projector's mean for
         instance i; samples[i] (want_samples) its per-sample zsum and sexp.
-        chunk: the item size in j (0: the engine's default; "auto": the
-        autotuner's choice of kernel and item size for this call)."""
+        chunk: the most terms that one lane takes (0: the engine's rule;
+        "auto": the autotuner's choice for this call)."""
         if instances.dtype != SAMPLED_INSTANCE_DTYPE or not instances.flags["C_CONTIGUOUS"]:
             raise ValueError("instances must be a contiguous sampled_instance_array")
         kernel = None

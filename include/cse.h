@@ -54,7 +54,7 @@ typedef struct {
 
 /* A context on a gfx950 device.  It reads CSE_FLUSH_TERMS from the
  * environment when set: the number of terms of one instance after which a
- * wave of the exact-mode sweep flushes its partial histogram (1 to 2^30;
+ * block of the exact-mode sweep flushes its partial histogram (1 to 2^30;
  * default 2^30, which keeps the sweep's 32-bit partial bins from wrapping).
  * Results do not depend on it; a value outside that range fails the call. */
 int cse_create(int device, cse_ctx **ctx);
@@ -78,18 +78,11 @@ int cse_device_info(cse_ctx *ctx, int *cus, char *name, int name_len);
 int cse_set_graphs(cse_ctx *ctx, int enable);
 
 /*
- * The sweep kernel of the context's calls of one mode, a tuning knob (the
- * results are identical).  mode 0 (sampled calls): kernel 0 the engine's
- * choice (2 when every instance of the call uses the |H^t> decomposition,
- * else 1), 1 the eight-wave sweep whose hand-scheduled path takes records
- * of at most two non-pivot columns (others run compiled code), 2 the
- * eight-wave sweep whose hand-scheduled path takes any number of non-pivot
- * columns and, for |H^t> terms, retires uncoupled variables in one batch
- * and runs each aligned batch of 64 terms as eight groups of 8.  mode 1
- * (exact calls): kernel 0 the engine's choice (2 for launches of at least 16
- * slices of 64 j per resident wave, else 1), 1 the exact sweep at seven
- * waves per SIMD, 2 the same at eight.  No reference counterpart (the
- * reference has one CPU code path).
+ * The sweep kernel of the context's calls of one mode (0 sampled, 1 exact): a
+ * tuning knob that never changes a result.  kernel 0 is the engine's choice.
+ * Each mode and width has one sweep kernel, so 1 and 2, which used to select
+ * among several, are accepted and run the same one.  No reference counterpart
+ * (the reference has one CPU code path).
  */
 int cse_set_sweep_kernel(cse_ctx *ctx, int mode, int kernel);
 
@@ -161,7 +154,7 @@ int cse_exact_projector(cse_ctx *ctx, const cse_projector *P, const uint64_t *L,
  * capture, tight serving loops, harnesses that forbid hipMalloc).  It calls
  * no hipMalloc, hipFree, host allocator or other allocating routine: every
  * device buffer the call needs (work queue, plan, results block, records)
- * lives in a static device array of 8,762,624 bytes that each GPU holds
+ * lives in a static device array of 4,502,016 bytes that each GPU holds
  * until the process ends, and the host stages are on the stack.  Results
  * equal cse_exact_projector's.  chi <= 2^13 (|H^t> with t <= 26, or k <= 13);
  * larger chi returns CSE_ERR_ARG.  Every call on one GPU shares that GPU's
@@ -191,8 +184,8 @@ typedef struct {
  * states theta_s (replaces sampledProjector / singleProjectorSample,
  * innerprod.c:45-144; the median over bins of multiSampledProjector,
  * innerprod.c:23-41, is taken by the caller over disjoint sample ranges).
- * Persistent launch over a device work queue of (sample, chunk) items;
- * chunk = 0 picks the tuned default.
+ * Persistent launch over a device work queue; chunk > 0 bounds the terms that
+ * one lane takes, chunk = 0 leaves them to the engine's rule.
  */
 int cse_sampled_projector(cse_ctx *ctx, const cse_projector *P, const uint64_t *L, int k,
                           int exact, uint64_t seed, int64_t first, int64_t count, int chunk,
