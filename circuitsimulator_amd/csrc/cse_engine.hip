@@ -651,6 +651,9 @@ void plan_tree(InstDesc &d, int mode, int simds, int ninst, bool lds_only, int m
     d.spare = beyond;
 }
 
+// the bit of a slot in a record's words
+uint64_t slot_word(int x) { return x < 32 ? 1ull << (31 - x) : 1ull << (95 - x); }
+
 // mode 0: nsamp records; mode 1: chi records.  max_terms > 0 bounds the terms
 // of a lane (the calls' chunk).
 InstDesc make_inst(const cse_ctx *ctx, int mode, int t, int k, int exact, const uint64_t *L, long long nsamp,
@@ -670,8 +673,8 @@ InstDesc make_inst(const cse_ctx *ctx, int mode, int t, int k, int exact, const 
             const int q = d.k - 1 - b, u = 2 * b - odd, s = u + 1;
             col[s] = (uint8_t)(odd && b == 0 ? t - 1 : 2 * q + 1);
             if (u >= 0) col[u] = (uint8_t)(2 * q);
-            d.LP[b] = 1ull << s;
-            d.L[b] = u >= 0 ? 1ull << u : 0ull;
+            d.LP[b] = slot_word(s);
+            d.L[b] = u >= 0 ? slot_word(u) : 0ull;
             d.jmap[b] = 1u << b;
             if (b < TREE_MAXG) d.ub[b + 1] = (uint8_t)(s + 1);
         }
@@ -680,7 +683,7 @@ InstDesc make_inst(const cse_ctx *ctx, int mode, int t, int k, int exact, const 
         uint8_t pos[64];
         for (int p = 0; p < t; p++) pos[col[p]] = (uint8_t)p;
         for (int b = 0; b < k; b++)
-            for (uint64_t r = d.L[b]; r; r &= r - 1) d.LP[b] |= 1ull << pos[__builtin_ctzll(r)];
+            for (uint64_t r = d.L[b]; r; r &= r - 1) d.LP[b] |= slot_word(pos[__builtin_ctzll(r)]);
     }
     for (int p = 0; p < 64; p++) d.inv[p] = p < t ? col[p] : (uint8_t)p;
     d.lanes = nsamp;

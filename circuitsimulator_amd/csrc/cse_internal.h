@@ -20,6 +20,8 @@ struct DevProjector {
 //   w[0] = n << 8 | Q << 16 | sexp << 24 | vanished << 40
 //   w[1] = F, the slots that hold multipliers; w[2], w[3] = d1, d2
 //   w[4 .. 68)   rows of J (symmetric, no diagonal), zero beyond n
+// A word's slot x is bit 31 - x of its low half (x < 32), slot 32 + x bit
+// 31 - x of its high half.
 #define REC_ROWS 4
 #define REC_WORDS 68
 
@@ -64,8 +66,8 @@ struct InstDesc {
     uint8_t inv[64];    // column of each slot
     uint8_t ub[TREE_MAXG + 4];    // ub[g]: slots that index bits below g move
     uint16_t soff[TREE_MAXG + 4]; // first word of level g's part of its stack
-    // per index bit: the slots it toggles (LP), and by columns (|L>) or the
-    // slots whose sign it toggles (|H^t>)
+    // per index bit: the slots it toggles (LP, bits as in a record), and by
+    // columns (|L>) or the slots whose sign it toggles (|H^t>, as LP)
     uint64_t LP[TREE_MAXLOG];
     uint64_t L[TREE_MAXLOG];
     uint32_t jmap[TREE_MAXLOG];   // the reference's index j of each bit

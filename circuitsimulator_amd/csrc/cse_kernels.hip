@@ -334,6 +334,9 @@ DEV u64 transpose64(u64 v) {
     return v;
 }
 
+// slot x at bit 31 - x of each half, as the sweep keeps its words
+DEV u64 brev32x2(u64 v) { return (u64)__brev((unsigned)v) | (u64)__brev((unsigned)(v >> 32)) << 32; }
+
 // The record of a state in reduced row echelon form, rows at their pivot
 // lanes: its form on the instance's slots (cse_tree.h).
 //  * the slot of a pivot column is the coordinate x_a = h_a + z_a itself, so
@@ -370,11 +373,11 @@ DEV void store_form(const AState &s, const InstDesc &D, int sexp, uint64_t *rec)
     const u64 d1 = ballot(d & 2), d2 = ballot(d & 4), F = ballot(f);
     if (x == 0) {
         rec[0] = ((uint64_t)n << 8) | ((uint64_t)(Q & 7) << 16) | ((uint64_t)sexp << 24);
-        rec[1] = F;
-        rec[2] = d1;
-        rec[3] = d2;
+        rec[1] = brev32x2(F);
+        rec[2] = brev32x2(d1);
+        rec[3] = brev32x2(d2);
     }
-    rec[REC_ROWS + x] = M;
+    rec[REC_ROWS + x] = brev32x2(M);
 }
 
 // Reduced row echelon basis of the active rows (basis changes of the form,

@@ -105,7 +105,7 @@ template <int NH> DEV void form_save(const tree::Form<NH> &f, unsigned a, int c,
     p[64] = f.d2;
     p[128] = a;
     p[192] = f.x2;
-    p[256] = (f.z & 0x80000000u) | ((unsigned)f.q1 << 8) | (unsigned)f.nb;
+    p[256] = (f.z & 0x80000000u) | (f.q1 << 8) | f.nb;
 #pragma unroll
     for (int x = 0; x < 32; x += 2)
         if (c > x) {
@@ -120,8 +120,8 @@ template <int NH> DEV void form_load(tree::Form<NH> &f, int c, const uint32_t *p
     f.x2 = p[192];
     const unsigned w = p[256];
     f.z = w & 0x80000000u;
-    f.q1 = (int)((w >> 8) & 0xffu);
-    f.nb = (int)(w & 0xffu);
+    f.q1 = (w >> 8) & 0xffu;
+    f.nb = w & 0xffu;
 #pragma unroll
     for (int x = 0; x < 32; x += 2)
         if (c > x) {
@@ -227,7 +227,8 @@ template <int NH, bool HT, int MODE> DEV void sweep_body(const SweepArgs &A) {
         tree::Form<NH> f;
         {
             const u64 F = rec[1], d1 = rec[2], d2 = rec[3];
-            u64 xj = D->exact ? lowmask(n) : 0ull, T = 0;
+            u64 xj = D->exact ? brev32x2(lowmask(n)) : 0ull;
+            u64 T = 0;
             for (int b = G; b < k; b++) {
                 const u64 on = 0ull - (u64)((jh >> (b - G)) & 1);
                 xj ^= D->LP[b] & on;
@@ -291,8 +292,8 @@ template <int NH, bool HT, int MODE> DEV void sweep_body(const SweepArgs &A) {
             }
             int ph = ph0, cnt = cnt0;
             tree::fold<HT>(f.d1, f.d2, f.A, f.T, ph, cnt);
-            const int p = cnt - f.nb;
-            const int m = (ph + 2 * f.q1 + 4 * __popc(f.x2)) & 7;
+            const int p = cnt - (int)f.nb;
+            const int m = (ph + 2 * (int)f.q1 + 4 * __popc(f.x2)) & 7;
             const bool nz = valid && (int)f.z >= 0;
             float vr, vi;
             if (MODE == 0) {

@@ -25,29 +25,177 @@
 //
 // |H^t> terms add a sign per slot (T): a summed slot is summed with
 // (-1)^{T z}, a dropped one is taken at z = T.
+//
+// Slot x < 32 is bit 31 - x of a word, slot 32 + x bit 31 - x of the next one.
+//
+// Instructions.  gfx950 issues and, xor, or, bitop3, add, sub, right shifts
+// and fma at twice the rate of the other VALU instructions (4.4-4.6 against
+// 2.2 wave instructions per ns and CU, two or more waves per SIMD), but only
+// in stretches without a single one of the others: one v_bfe_i32 or v_bcnt in
+// 64 brings all of them down to 2.4 until a scalar instruction shifts the
+// waves' phases again.  So a step is written in the fast ones alone: a mask
+// from a bit is and, sub, ashr (not v_bfe_i32), successive row masks are ashr
+// and add (not v_bfe_i32 at each bit), the row of a slot that differs from
+// lane to lane is picked by a tree of bitop3 selects, and counts are sums of
+// masks (not v_bcnt).  With v_bfe_i32 masks a step of slot 10 takes 93
+// instructions at 2.4 per ns and CU, this way 125 at 4.4.
 #pragma once
 #include <stdint.h>
-
-#ifdef __HIPCC__
-#define TREE_DEV __device__ __forceinline__
-#define TREE_BFE(v, i) ((u32)__builtin_amdgcn_sbfe((int)(v), (unsigned)(i), 1u))
-// x ^ (a & b) as the one instruction that it is (left to itself the compiler
-// splits the sums below into three per term)
-#define TREE_XA(x, a, b) ((u32)__builtin_amdgcn_bitop3_b32((x), (a), (b), 0x78))
-#define TREE_POP(v) __popc(v)
-#define TREE_FFS(v) ((u32)(__ffs((int)(v)) - 1))
-#else
-#define TREE_DEV inline
-#define TREE_BFE(v, i) ((u32)((int32_t)((uint32_t)(v) << (31 - ((i) & 31))) >> 31))
-#define TREE_XA(x, a, b) ((x) ^ ((a) & (b)))
-#define TREE_POP(v) __builtin_popcount(v)
-#define TREE_FFS(v) ((u32)(__builtin_ffs((int)(v)) - 1))
-#endif
 
 namespace cse {
 namespace tree {
 
 typedef uint32_t u32;
+
+// truth tables of the three operands
+constexpr unsigned TA = 0xF0, TB = 0xCC, TC = 0xAA;
+
+#ifdef __HIPCC__
+#define TREE_DEV __device__ __forceinline__
+// the three-operand boolean function of truth table F in one instruction
+#define TREE_B3(a, b, c, F) ((cse::tree::u32)__builtin_amdgcn_bitop3_b32((a), (b), (c), (F) & 0xffu))
+#define TREE_POP(v) __popc(v)
+template <u32 K> TREE_DEV u32 andk(u32 v) {
+    u32 r;
+    asm("v_and_b32 %0, %2, %1" : "=v"(r) : "v"(v), "n"(K));
+    return r;
+}
+// all ones if t, a single bit or zero, is set
+#define TREE_NZ(r) "v_sub_u32 " r ", 0, " r "\n\tv_ashrrev_i32 " r ", 31, " r "\n\t"
+TREE_DEV u32 nz1(u32 t) {
+    asm(TREE_NZ("%0") : "+&v"(t));
+    return t;
+}
+TREE_DEV void nz2(u32 &t, u32 &u) { asm(TREE_NZ("%0") TREE_NZ("%1") : "+&v"(t), "+&v"(u)); }
+// all ones if the single bit K of v is set
+template <u32 K> TREE_DEV u32 bitk(u32 v) {
+    u32 r;
+    asm("v_and_b32 %0, %2, %1\n\t" TREE_NZ("%0") : "=v"(r) : "v"(v), "n"(K));
+    return r;
+}
+template <u32 K> TREE_DEV void bitk2(u32 v, u32 w, u32 &r, u32 &q) {
+    asm("v_and_b32 %0, %4, %2\n\tv_and_b32 %1, %4, %3\n\t" TREE_NZ("%0") TREE_NZ("%1")
+        : "=&v"(r), "=&v"(q)
+        : "v"(v), "v"(w), "n"(K));
+}
+// mask of the top bit, and the next bit moved up
+TREE_DEV u32 pop_mask(u32 &t) {
+    u32 m;
+    asm("v_ashrrev_i32 %0, 31, %1\n\tv_add_u32 %1, %1, %1" : "=&v"(m), "+&v"(t));
+    return m;
+}
+// the sign bit of 0 - t put in at the top of w, the others moved down (t a
+// single bit or zero)
+TREE_DEV u32 push_nz(u32 w, u32 t) {
+    asm("v_lshrrev_b32 %0, 1, %0\n\tv_sub_u32 %1, 0, %1\n\tv_and_b32 %1, 0x80000000, %1\n\tv_or_b32 %0, %0, %1"
+        : "+&v"(w), "+&v"(t));
+    return w;
+}
+// (Operands that a block writes before its last read are early clobbers: tv
+// and b start as the same value.)
+// N rows r: r ^= a where tv's next bit is set, ^= b where tw's is.  One asm
+// block for several rows: between blocks the compiler pads with s_nop.
+#define TREE_ROW(r)                                                                        \
+    "v_ashrrev_i32 %[m], 31, %[tv]\n\tv_add_u32 %[tv], %[tv], %[tv]\n\t"                  \
+    "v_bitop3_b32 " r ", " r ", %[m], %[a] bitop3:0x78\n\t"                                \
+    "v_ashrrev_i32 %[m], 31, %[tw]\n\tv_add_u32 %[tw], %[tw], %[tw]\n\t"                  \
+    "v_bitop3_b32 " r ", " r ", %[m], %[b] bitop3:0x78\n\t"
+#define TREE_ROWS_IO [tv] "+&v"(tv), [tw] "+&v"(tw), [m] "=&v"(m) : [a] "v"(a), [b] "v"(b)
+template <int N> TREE_DEV void rows(u32 *r, u32 &tv, u32 &tw, u32 a, u32 b) {
+    u32 m;
+    if constexpr (N >= 8) {
+        asm(TREE_ROW("%0") TREE_ROW("%1") TREE_ROW("%2") TREE_ROW("%3") TREE_ROW("%4") TREE_ROW("%5") TREE_ROW("%6")
+                TREE_ROW("%7")
+            : "+&v"(r[0]), "+&v"(r[1]), "+&v"(r[2]), "+&v"(r[3]), "+&v"(r[4]), "+&v"(r[5]), "+&v"(r[6]), "+&v"(r[7]),
+              TREE_ROWS_IO);
+        rows<N - 8>(r + 8, tv, tw, a, b);
+    } else if constexpr (N >= 4) {
+        asm(TREE_ROW("%0") TREE_ROW("%1") TREE_ROW("%2") TREE_ROW("%3")
+            : "+&v"(r[0]), "+&v"(r[1]), "+&v"(r[2]), "+&v"(r[3]), TREE_ROWS_IO);
+        rows<N - 4>(r + 4, tv, tw, a, b);
+    } else if constexpr (N >= 2) {
+        asm(TREE_ROW("%0") TREE_ROW("%1") : "+&v"(r[0]), "+&v"(r[1]), TREE_ROWS_IO);
+        rows<N - 2>(r + 2, tv, tw, a, b);
+    } else if constexpr (N == 1) {
+        asm(TREE_ROW("%0") : "+&v"(r[0]), TREE_ROWS_IO);
+    }
+}
+// the same for rows of two words
+TREE_DEV void row2(u32 &r, u32 &q, u32 &tv, u32 &tw, u32 a, u32 b, u32 c, u32 d) {
+    u32 m;
+    asm("v_ashrrev_i32 %[m], 31, %[tv]\n\tv_add_u32 %[tv], %[tv], %[tv]\n\t"
+        "v_bitop3_b32 %[r], %[r], %[m], %[a] bitop3:0x78\n\tv_bitop3_b32 %[q], %[q], %[m], %[c] bitop3:0x78\n\t"
+        "v_ashrrev_i32 %[m], 31, %[tw]\n\tv_add_u32 %[tw], %[tw], %[tw]\n\t"
+        "v_bitop3_b32 %[r], %[r], %[m], %[b] bitop3:0x78\n\tv_bitop3_b32 %[q], %[q], %[m], %[d] bitop3:0x78"
+        : [r] "+&v"(r), [q] "+&v"(q), [tv] "+&v"(tv), [tw] "+&v"(tw), [m] "=&v"(m)
+        : [a] "v"(a), [b] "v"(b), [c] "v"(c), [d] "v"(d));
+}
+// masks of the bits of a slot's number: w[k] starts as o with the slots that
+// have bit k, and becomes all ones if that is not empty
+template <int K> TREE_DEV void picked(u32 o, u32 *w) {
+#define TREE_PK(i, mask) "v_and_b32 %" #i ", " #mask ", %[o]\n\t" TREE_NZ("%" #i)
+    if constexpr (K == 5)
+        asm(TREE_PK(0, 0x55555555) TREE_PK(1, 0x33333333) TREE_PK(2, 0x0f0f0f0f) TREE_PK(3, 0x00ff00ff)
+                TREE_PK(4, 0x0000ffff)
+            : "=&v"(w[0]), "=&v"(w[1]), "=&v"(w[2]), "=&v"(w[3]), "=&v"(w[4])
+            : [o] "v"(o));
+    if constexpr (K == 4)
+        asm(TREE_PK(0, 0x55555555) TREE_PK(1, 0x33333333) TREE_PK(2, 0x0f0f0f0f) TREE_PK(3, 0x00ff00ff)
+            : "=&v"(w[0]), "=&v"(w[1]), "=&v"(w[2]), "=&v"(w[3])
+            : [o] "v"(o));
+    if constexpr (K == 3)
+        asm(TREE_PK(0, 0x55555555) TREE_PK(1, 0x33333333) TREE_PK(2, 0x0f0f0f0f)
+            : "=&v"(w[0]), "=&v"(w[1]), "=&v"(w[2])
+            : [o] "v"(o));
+    if constexpr (K == 2)
+        asm(TREE_PK(0, 0x55555555) TREE_PK(1, 0x33333333) : "=&v"(w[0]), "=&v"(w[1]) : [o] "v"(o));
+    if constexpr (K == 1) asm(TREE_PK(0, 0x55555555) : "=&v"(w[0]) : [o] "v"(o));
+}
+#else
+#define TREE_DEV inline
+#define TREE_POP(v) __builtin_popcount(v)
+inline u32 tree_b3(u32 a, u32 b, u32 c, unsigned F) {
+    u32 r = 0;
+    for (int i = 0; i < 8; i++)
+        if ((F >> i) & 1) r |= ((i & 4) ? a : ~a) & ((i & 2) ? b : ~b) & ((i & 1) ? c : ~c);
+    return r;
+}
+#define TREE_B3(a, b, c, F) (cse::tree::tree_b3((a), (b), (c), (F) & 0xffu))
+template <u32 K> inline u32 andk(u32 v) { return v & K; }
+inline u32 nz1(u32 t) { return t ? ~0u : 0u; }
+inline void nz2(u32 &t, u32 &u) {
+    t = nz1(t);
+    u = nz1(u);
+}
+template <u32 K> inline u32 bitk(u32 v) { return nz1(v & K); }
+template <u32 K> inline void bitk2(u32 v, u32 w, u32 &r, u32 &q) {
+    r = nz1(v & K);
+    q = nz1(w & K);
+}
+inline u32 pop_mask(u32 &t) {
+    const u32 m = nz1(t >> 31);
+    t += t;
+    return m;
+}
+inline u32 push_nz(u32 w, u32 t) { return (w >> 1) | (t ? 0x80000000u : 0u); }
+template <int N> inline void rows(u32 *r, u32 &tv, u32 &tw, u32 a, u32 b) {
+    for (int x = 0; x < N; x++) {
+        r[x] ^= pop_mask(tv) & a;
+        r[x] ^= pop_mask(tw) & b;
+    }
+}
+inline void row2(u32 &r, u32 &q, u32 &tv, u32 &tw, u32 a, u32 b, u32 c, u32 d) {
+    const u32 m = pop_mask(tv), l = pop_mask(tw);
+    r ^= (m & a) ^ (l & b);
+    q ^= (m & c) ^ (l & d);
+}
+template <int K> inline void picked(u32 o, u32 *w) {
+    static const u32 with[5] = {0x55555555u, 0x33333333u, 0x0f0f0f0fu, 0x00ff00ffu, 0x0000ffffu};
+    for (int k = 0; k < K; k++) w[k] = nz1(o & with[k]);
+}
+#endif
+// x ^ (a & b)
+#define TREE_XA(x, a, b) TREE_B3(x, a, b, TA ^ (TB & TC))
 
 // rows below slot 32 are kept as one word (the part of a row at slots >= 32
 // is read from the rows of those slots), the NH rows from slot 32 on as two
@@ -58,117 +206,137 @@ template <int NH> struct Form {
     u32 d1h, d2h, Ah, Th;   // slots 32..
     u32 x2;                 // parity word: 4 per set bit
     u32 z;                  // top bit set: the sum is 0
-    int nb, q1;             // steps of the third kind; phase in units of 2
+    u32 nb, q1;             // steps of the third kind; phase in units of 2
 };
 
-// bits of slots below c, c <= 32
-TREE_DEV u32 low32(int c) { return c >= 32 ? ~0u : (1u << c) - 1u; }
+constexpr u32 slot_bit(int x) { return 0x80000000u >> x; }
+// bits of the slots below c, c < 32
+constexpr u32 below(int c) { return c == 0 ? 0u : ~0u << (32 - c); }
+// bits of a slot number below N
+constexpr int index_bits(int N) { return N > 16 ? 5 : N > 8 ? 4 : N > 4 ? 3 : N > 2 ? 2 : N > 1 ? 1 : 0; }
+
+// r[the slot of masks b], a tree of selects over r[LO .. LO + 2^K - 1] below N
+template <int N, int K, int LO> struct Pick {
+    static TREE_DEV u32 run(const u32 *r, const u32 *b) {
+        const u32 lo = Pick<N, K - 1, LO>::run(r, b);
+        constexpr int UP = LO + (1 << (K - 1));
+        if (UP >= N) return lo;
+        const u32 up = Pick<N, K - 1, (UP < N ? UP : LO)>::run(r, b);
+        return TREE_B3(b[K - 1], up, lo, (TA & TB) | (~TA & TC));
+    }
+};
+template <int N, int LO> struct Pick<N, 0, LO> {
+    static TREE_DEV u32 run(const u32 *r, const u32 *) { return r[LO]; }
+};
+template <int N> TREE_DEV u32 pick(const u32 *r, const u32 *b) { return Pick<N, index_bits(N), 0>::run(r, b); }
 
 // Step of slot C < 32 (all slots above it done).
 template <int NH, bool HT, int C> TREE_DEV void step(Form<NH> &f) {
-    const u32 below = low32(C);
-    const u32 act = TREE_BFE(f.A, C);
-    const u32 odd = TREE_BFE(f.d1, C);
-    if (HT) {
-        // a dropped slot is taken at T: D_x += 4 T J_cx
-        const u32 at1 = TREE_BFE(f.T, C) & ~act;
-        f.d2 ^= f.lo[C] & at1 & below;
-    }
-    const u32 hi = TREE_BFE(HT ? f.d2 ^ f.T : f.d2, C);
-    const u32 v = f.lo[C] & act & below;
-    const u32 o = v & (0u - v) & ~odd;      // the slot solved for, if any
-    const u32 i = TREE_FFS(v);              // all ones when v is empty
-    // second kind, in the top bit (i < 32 otherwise)
-    const u32 iso = act & ~odd & i;
-    f.z |= iso & hi;
+    u32 act, odd;
+    bitk2<slot_bit(C)>(f.A, f.d1, act, odd);
+    const u32 row = andk<below(C)>(f.lo[C]);
+    // a dropped slot is taken at T: D_x += 4 T J_cx
+    if (HT) f.d2 = TREE_XA(f.d2, row, TREE_B3(bitk<slot_bit(C)>(f.T), act, act, TA & ~TB));
+    const u32 hi = bitk<slot_bit(C)>(HT ? f.d2 ^ f.T : f.d2);
+    const u32 v = row & act, neg = 0u - v;
+    // second kind (v empty), in the top bit
+    const u32 iso = TREE_B3(act, odd, v | neg, TA & ~TB & ~TC);
+    f.z = TREE_B3(f.z, iso, hi, TA | (TB & TC));
     if (C == 0) return;
-    const u32 oddi = TREE_BFE(f.d1, i), d2i = TREE_BFE(f.d2, i);
+    const u32 o = TREE_B3(v, neg, odd, TA & TB & ~TC);  // the slot solved for, if any
+    const u32 bm = nz1(o);
+    f.nb -= bm;
+    u32 oddi = f.d1 & o, d2i = f.d2 & o;
+    nz2(oddi, d2i);
     const u32 e = odd | oddi;
-    const u32 u = d2i ^ (hi & oddi);
-    const u32 h = (odd & ~hi) | (~odd & u);
-    u32 w = 0;
-#pragma unroll
-    for (int x = 0; x < C; x++) w = TREE_XA(w, TREE_BFE(o, x), f.lo[x]);
-    w &= below & ~o;
-    const u32 vp = v & ~o;
+    const u32 u = TREE_XA(d2i, hi, oddi);
+    const u32 h = TREE_B3(odd, hi, u, (TA & ~TB) | (~TA & TC));
+    u32 p[5];
+    picked<index_bits(C)>(o, p);
+    const u32 w = TREE_B3(pick<C>(f.lo, p), andk<below(C)>(bm), o, TA & TB & ~TC);
+    const u32 vp = TREE_B3(v, o, o, TA & ~TB);
     const u32 ev = e & vp;
-    const u32 al = w ^ o ^ ev;
-    const u32 wm = w | (o & ~oddi);
+    const u32 al = TREE_B3(w, o, ev, TA ^ TB ^ TC);
+    u32 wm = TREE_B3(w, o, oddi, TA | (TB & ~TC));
     const u32 oh = o & hi;
-    f.q1 += TREE_POP(oh & f.d1);
-    f.x2 ^= oh & f.d2;
-    f.nb += TREE_POP(o);
-    const u32 g = h ^ (e & f.d1);
-    f.d2 ^= (vp & g) ^ (w & (hi ^ vp));
-    f.d1 = (f.d1 ^ ev) & ~o;
-    f.d2 = (f.d2 & ~o) | oh;
-#pragma unroll
-    for (int x = 0; x < C; x++)
-        f.lo[x] = TREE_XA(TREE_XA(f.lo[x], TREE_BFE(v, x), al), TREE_BFE(wm, x), v);
+    f.q1 -= TREE_B3(hi, oddi, bm, TA & TB & TC);
+    f.x2 = TREE_XA(f.x2, oh, f.d2);
+    const u32 g = TREE_XA(h, e, f.d1);
+    f.d2 = TREE_XA(f.d2, vp, g);
+    f.d2 ^= TREE_B3(w, hi, vp, TA & (TB ^ TC));
+    f.d2 = TREE_B3(f.d2, o, oh, (TA & ~TB) | TC);
+    f.d1 = TREE_B3(f.d1, ev, o, (TA ^ TB) & ~TC);
+    u32 tv = v;
+    rows<C>(f.lo, tv, wm, al, v);
     f.A ^= o;
 }
 
 // Step of slot 32 + C.
 template <int NH, bool HT, int C> TREE_DEV void step_hi(Form<NH> &f) {
-    const u32 below = low32(C);
-    const u32 act = TREE_BFE(f.Ah, C);
-    const u32 odd = TREE_BFE(f.d1h, C);
+    u32 act, odd;
+    bitk2<slot_bit(C)>(f.Ah, f.d1h, act, odd);
+    const u32 rowl = f.lo[32 + C], rowh = andk<below(C)>(f.hi[C]);
     if (HT) {
-        const u32 at1 = TREE_BFE(f.Th, C) & ~act;
-        f.d2 ^= f.lo[32 + C] & at1;
-        f.d2h ^= f.hi[C] & at1 & below;
+        const u32 at1 = TREE_B3(bitk<slot_bit(C)>(f.Th), act, act, TA & ~TB);
+        f.d2 = TREE_XA(f.d2, rowl, at1);
+        f.d2h = TREE_XA(f.d2h, rowh, at1);
     }
-    const u32 hi = TREE_BFE(HT ? f.d2h ^ f.Th : f.d2h, C);
-    const u32 vl = f.lo[32 + C] & act, vh = f.hi[C] & act & below;
-    const u32 inl = vh ? 0u : ~0u;          // the solved slot is below 32
-    const u32 ol = vl & (0u - vl) & ~odd & inl, oh = vh & (0u - vh) & ~odd;
-    const u32 iso = (vl | vh) ? 0u : act & ~odd;
-    f.z |= iso & hi & 0x80000000u;
-    const u32 oddi = ((f.d1 & ol) | (f.d1h & oh)) ? ~0u : 0u;
-    const u32 d2i = ((f.d2 & ol) | (f.d2h & oh)) ? ~0u : 0u;
+    const u32 hi = bitk<slot_bit(C)>(HT ? f.d2h ^ f.Th : f.d2h);
+    const u32 vl = rowl & act, vh = rowh & act, negl = 0u - vl, negh = 0u - vh;
+    const u32 nh = vh | negh;               // top bit: vh is not empty
+    const u32 iso = TREE_B3(act, odd, TREE_B3(nh, vl, negl, TA | TB | TC), TA & ~TB & ~TC);
+    f.z = TREE_B3(f.z, iso, hi, TA | (TB & TC));
+    // the slot solved for, among those from 32 on if there is one
+    u32 nhm = nh;
+    const u32 ol = TREE_B3(TREE_B3(vl, negl, odd, TA & TB & ~TC), pop_mask(nhm), odd, TA & ~TB);
+    const u32 oh = TREE_B3(vh, negh, odd, TA & TB & ~TC);
+    u32 bl = ol, bh = oh;
+    nz2(bl, bh);
+    f.nb -= bl;
+    f.nb -= bh;
+    u32 oddi = TREE_B3(f.d1 & ol, f.d1h, oh, TA | (TB & TC));
+    u32 d2i = TREE_B3(f.d2 & ol, f.d2h, oh, TA | (TB & TC));
+    nz2(oddi, d2i);
     const u32 e = odd | oddi;
-    const u32 u = d2i ^ (hi & oddi);
-    const u32 h = (odd & ~hi) | (~odd & u);
-    u32 wl = 0, wh = 0;
+    const u32 u = TREE_XA(d2i, hi, oddi);
+    const u32 h = TREE_B3(odd, hi, u, (TA & ~TB) | (~TA & TC));
+    // the row of that slot
+    u32 pl[5];
+    picked<5>(ol, pl);
+    u32 wl = pick<32>(f.lo, pl) & bl, wh = 0;
+    if (C > 0) {
+        u32 ph[5];
+        picked<index_bits(C)>(oh, ph);
+        wl = TREE_B3(wl, pick<(C > 0 ? C : 1)>(f.lo + 32, ph), bh, TA | (TB & TC));
+        // its slots from 32 on: of a row below 32, one bit of each of theirs
 #pragma unroll
-    for (int x = 0; x < 32; x++) wl = TREE_XA(wl, TREE_BFE(ol, x), f.lo[x]);
-    const u32 il = TREE_FFS(ol);
-#pragma unroll
-    for (int x = 0; x < C; x++) {
-        const u32 m = TREE_BFE(oh, x);
-        wl = TREE_XA(wl, m, f.lo[32 + x]);
-        wh = TREE_XA(wh, m, f.hi[x]);
+        for (int x = C - 1; x >= 0; x--) wh = push_nz(wh, f.lo[32 + x] & ol);
+        wh = TREE_B3(wh, pick<(C > 0 ? C : 1)>(f.hi, ph), bh, TA | (TB & TC));
     }
-    u32 col = 0;  // column il of the rows above, when il is a slot
-#pragma unroll
-    for (int x = 0; x < C; x++) col |= (TREE_BFE(f.lo[32 + x], il) & 1u) << x;
-    wh ^= col & (ol ? ~0u : 0u);
-    wl &= ~ol;
-    wh &= below & ~oh;
-    const u32 vpl = vl & ~ol, vph = vh & ~oh;
+    wl = TREE_B3(wl, ol, ol, TA & ~TB);
+    wh = TREE_B3(andk<below(C)>(wh), oh, oh, TA & ~TB);
+    const u32 vpl = TREE_B3(vl, ol, ol, TA & ~TB), vph = TREE_B3(vh, oh, oh, TA & ~TB);
     const u32 evl = e & vpl, evh = e & vph;
-    const u32 all = wl ^ ol ^ evl, alh = wh ^ oh ^ evh;
-    const u32 wml = wl | (ol & ~oddi), wmh = wh | (oh & ~oddi);
+    const u32 all = TREE_B3(wl, ol, evl, TA ^ TB ^ TC), alh = TREE_B3(wh, oh, evh, TA ^ TB ^ TC);
+    u32 wml = TREE_B3(wl, ol, oddi, TA | (TB & ~TC)), wmh = TREE_B3(wh, oh, oddi, TA | (TB & ~TC));
     const u32 ohl = ol & hi, ohh = oh & hi;
-    f.q1 += TREE_POP(ohl & f.d1) + TREE_POP(ohh & f.d1h);
-    f.x2 ^= (ohl & f.d2) ^ (ohh & f.d2h);
-    f.nb += TREE_POP(ol) + TREE_POP(oh);
-    const u32 gl = h ^ (e & f.d1), gh = h ^ (e & f.d1h);
-    f.d2 ^= (vpl & gl) ^ (wl & (hi ^ vpl));
-    f.d2h ^= (vph & gh) ^ (wh & (hi ^ vph));
-    f.d1 = (f.d1 ^ evl) & ~ol;
-    f.d1h = (f.d1h ^ evh) & ~oh;
-    f.d2 = (f.d2 & ~ol) | ohl;
-    f.d2h = (f.d2h & ~oh) | ohh;
+    f.q1 -= TREE_B3(hi, oddi, bl | bh, TA & TB & TC);
+    f.x2 = TREE_XA(f.x2, ohl, f.d2);
+    f.x2 = TREE_XA(f.x2, ohh, f.d2h);
+    const u32 gl = TREE_XA(h, e, f.d1), gh = TREE_XA(h, e, f.d1h);
+    f.d2 = TREE_XA(f.d2, vpl, gl);
+    f.d2 ^= TREE_B3(wl, hi, vpl, TA & (TB ^ TC));
+    f.d2 = TREE_B3(f.d2, ol, ohl, (TA & ~TB) | TC);
+    f.d2h = TREE_XA(f.d2h, vph, gh);
+    f.d2h ^= TREE_B3(wh, hi, vph, TA & (TB ^ TC));
+    f.d2h = TREE_B3(f.d2h, oh, ohh, (TA & ~TB) | TC);
+    f.d1 = TREE_B3(f.d1, evl, ol, (TA ^ TB) & ~TC);
+    f.d1h = TREE_B3(f.d1h, evh, oh, (TA ^ TB) & ~TC);
+    u32 tv = vl;
+    rows<32>(f.lo, tv, wml, all, vl);
+    tv = vh;
 #pragma unroll
-    for (int x = 0; x < 32; x++)
-        f.lo[x] = TREE_XA(TREE_XA(f.lo[x], TREE_BFE(vl, x), all), TREE_BFE(wml, x), vl);
-#pragma unroll
-    for (int x = 0; x < C; x++) {
-        const u32 m1 = TREE_BFE(vh, x), m2 = TREE_BFE(wmh, x);
-        f.lo[32 + x] = TREE_XA(TREE_XA(f.lo[32 + x], m1, all), m2, vl);
-        f.hi[x] = TREE_XA(TREE_XA(f.hi[x], m1, alh), m2, vh);
-    }
+    for (int x = 0; x < C; x++) row2(f.lo[32 + x], f.hi[x], tv, wmh, all, vl, alh, vh);
     f.A ^= ol;
     f.Ah ^= oh;
 }

@@ -41,8 +41,8 @@ template <int NH, bool HT> static void go(int n, const uint64_t *row, const uint
     Steps<NH, HT, 31>::run(f, 0, (u32)(low / 2));
     fold<HT>(f.d1, f.d2, f.A, f.T, ph, cnt);
     out[0] = (f.z >> 31) ? 0 : 1;
-    out[1] = cnt - f.nb - n;
-    out[2] = (ph + 2 * f.q1 + 4 * TREE_POP(f.x2)) & 7;
+    out[1] = cnt - (int)f.nb - n;
+    out[2] = (ph + 2 * (int)f.q1 + 4 * TREE_POP(f.x2)) & 7;
 }
 extern "C" void tree_eval(int nh, int ht, int n, const uint64_t *row, const uint64_t *w, int *out) {
     if (nh == 0) ht ? go<0, true>(n, row, w, out) : go<0, false>(n, row, w, out);
@@ -59,6 +59,11 @@ def tree(tmp_path_factory):
     subprocess.run(["g++", "-O1", "-shared", "-fPIC", "-I", CSRC, "-o", str(d / "shim.so"), str(d / "shim.cpp")],
                    check=True)
     return ctypes.CDLL(str(d / "shim.so"))
+
+
+def words(v):
+    """slot x of a mask at bit 31 - x of its half, as the header keeps it"""
+    return sum(1 << (31 - x if x < 32 else 95 - x) for x in range(64) if v >> x & 1)
 
 
 def brute(J, d1, d2, A, F, T):
@@ -108,9 +113,9 @@ def test_form_sums_match_brute_force(tree, nh, n, signs):
 
         rows = (ctypes.c_uint64 * 64)()
         for i, p in enumerate(pos):
-            rows[p] = up(J[i])
+            rows[p] = words(up(J[i]))
         out = (ctypes.c_int * 3)()
-        tree.tree_eval(nh, signs, n, rows, (ctypes.c_uint64 * 4)(up(d1), up(d2), up(A), up(T)), out)
+        tree.tree_eval(nh, signs, n, rows, (ctypes.c_uint64 * 4)(*[words(up(v)) for v in (d1, d2, A, T)]), out)
         # the n - nv empty slots are pivots without a sum: 2^{-1/2} each
         got = out[0] * 2.0 ** ((out[1] + n - nv) / 2) * cmath.exp(1j * math.pi * out[2] / 4)
         assert abs(got - brute(J, d1, d2, A, F, T)) <= 1e-9
