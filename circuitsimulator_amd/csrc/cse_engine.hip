@@ -54,7 +54,7 @@ struct cse_ctx {
     int cus = 0;
     char name[128] = {0};
     char err[512] = {0};
-    DevBuf s1, s2, out, recs, terms, queue, thr, sexp, L, idx, errflag, lsh, stack;
+    DevBuf s1, s2, out, recs, terms, queue, thr, sexp, L, idx, errflag, lsh, stack, leaf;
     // a batch's plan: instance descriptors, item and record offsets and
     // projectors in one allocation, laid out as the pinned staging buffer
     DevBuf plan;
@@ -280,7 +280,7 @@ struct Plan {
         ninst++;
         nmax = std::max(nmax, d.n);
         anyH = anyH || d.exact;
-        stack_words = std::max(stack_words, (long long)d.spare);
+        stack_words = std::max(stack_words, (long long)d.beyond);
         rec_off[ninst] = nrec;
         item_off[ninst] = nitems;
     }
@@ -495,6 +495,7 @@ int run_sweep(cse_ctx *ctx, const Plan &pl, int mode, bool want_terms) {
     A.queue = ctx->b_queue;
     A.stack = ctx->b_stack;
     A.stack_words = pl.stack_words;
+    A.leaf = dp<uint8_t>(ctx->leaf) + (pl.anyH ? 1 << tree::LeafBits<false>::value : 0);
     A.terms = want_terms ? ctx->b_terms : nullptr;
     A.zsum = ctx->d_zsum;
     A.kahan = ctx->d_kahan;
@@ -591,43 +592,40 @@ int run_batch(cse_ctx *ctx, const Plan &pl, int mode, bool want_terms, size_t pl
 }
 
 // Cost model of a lane's tree, in VALU instructions: a step of slot c takes
-// about 31 for its own state (a signed one, |H^t>, 4 more) and 6 for every
-// slot below it, a slot beyond 32 twice that; a term's sums take about 70.
+// about 58 for its own state (a signed one, |H^t>, 8 more) and 7 for every
+// slot below it, a slot beyond 32 14 for those beyond; a term's sums take
+// about 60.
 double step_cost(int c, bool h) {
-    return c < 32 ? 31.0 + (h ? 4 : 0) + 6.0 * c : 60.0 + (h ? 6 : 0) + 6.0 * 32 + 11.0 * (c - 32);
+    return c < 32 ? 58.0 + (h ? 8 : 0) + 7.0 * c : 90.0 + (h ? 10 : 0) + 7.0 * 32 + 14.0 * (c - 32);
 }
 
-// G, the slot order and the stack of an instance.  G takes the largest share
-// of the work off the terms as long as the launch keeps the chip busy: with W
-// the instructions of one lane's tree, the launch takes about 4 W cycles for
-// its last wave plus 4 W per wave that each SIMD runs, and the G of the least
-// sum is taken (an instance of a batch bears its share of the last wave).
-// max_words: LDS words when the stack has to stay there.
-void plan_tree(InstDesc &d, int mode, int simds, int ninst, bool lds_only, int max_terms) {
+// G and the stack of an instance.  G takes the largest share of the work off
+// the terms as long as the launch keeps the chip busy: with W the instructions
+// of one lane's tree, the launch takes about 4 W cycles for its last wave plus
+// 4 W per wave that each SIMD runs, and the G of the least sum is taken (an
+// instance of a batch bears its share of the last wave).  lds_only: the stack
+// has to stay in LDS.
+void plan_tree(InstDesc &d, int mode, long long nrec, int simds, int ninst, bool lds_only, int max_terms) {
     const int lds = mode == 0 ? TREE_LDS_WORDS0 : TREE_LDS_WORDS1;
-    double best = 0.0, path[TREE_MAXG + 1];
-    // path[g]: steps of the slots from ub[g] up to ub[g + 1]
     auto steps = [&](int lo, int hi) {
         double w = 0;
         for (int c = lo; c < hi; c++) w += step_cost(c, d.exact);
         return w;
     };
     const int top = std::min(d.k, TREE_MAXG);
+    for (int g = 0; g <= top; g++) d.ub[g] = (uint8_t)std::max((int)d.ub[g], TREE_LEAF);
     int words = 0;
+    double best = 0.0, below = 0.0;  // below: steps of the slots below ub[g], per term
     d.G = 0;
-    double below = 0.0;  // steps of the slots below ub[g], per term
     for (int g = 0; g <= top; g++) {
         if (g > 0) {
             if (d.ub[g] > 32 || (1ll << g) > max_terms) break;
-            words += TREE_STATE_WORDS + d.ub[g];
+            if (d.ub[g] > TREE_LEAF) words += TREE_STATE_WORDS + d.ub[g];
             if (lds_only && words > lds) break;
-            path[g - 1] = steps(d.ub[g - 1], d.ub[g]);
-            below += path[g - 1] / (double)(1ll << (g - 1));
+            below += steps(d.ub[g - 1], d.ub[g]) / (double)(1ll << (g - 1));
         }
-        const double terms = (double)(1ll << g);
-        const double W = (below + 70.0) * terms + steps(d.ub[g], d.n) + 500.0;
-        const double nrec = mode == 0 ? (double)d.lanes : (double)d.chi;
-        const double lanes = nrec * (double)(d.chi >> g) * (mode == 0 ? 1.0 : 0.5);
+        const double W = (below + 60.0) * (double)(1ll << g) + steps(d.ub[g], d.n) + 500.0;
+        const double lanes = (double)nrec * (double)(d.chi >> g) * (mode == 0 ? 1.0 : 0.5);
         const double f = W / ninst + W * std::max(lanes / 64.0, 1.0) / simds;
         if (g == 0 || f < best) {
             best = f;
@@ -635,20 +633,20 @@ void plan_tree(InstDesc &d, int mode, int simds, int ninst, bool lds_only, int m
         }
     }
     words = 0;
-    d.nlds = 0;
-    int beyond = 0;
+    d.nlds = d.leaf = d.beyond = 0;
     for (int g = 1; g <= d.G; g++) {
         const int w = TREE_STATE_WORDS + d.ub[g];
-        if (d.nlds == g - 1 && words + w <= lds) {
+        if (d.ub[g] <= TREE_LEAF) {
+            d.leaf = d.nlds = g;
+        } else if (d.nlds == g - 1 && words + w <= lds) {
             d.soff[g] = (uint16_t)words;
             words += w;
             d.nlds = g;
         } else {
-            d.soff[g] = (uint16_t)beyond;
-            beyond += w;
+            d.soff[g] = (uint16_t)d.beyond;
+            d.beyond += w;
         }
     }
-    d.spare = beyond;
 }
 
 // the bit of a slot in a record's words
@@ -686,8 +684,7 @@ InstDesc make_inst(const cse_ctx *ctx, int mode, int t, int k, int exact, const 
             for (uint64_t r = d.L[b]; r; r &= r - 1) d.LP[b] |= slot_word(pos[__builtin_ctzll(r)]);
     }
     for (int p = 0; p < 64; p++) d.inv[p] = p < t ? col[p] : (uint8_t)p;
-    d.lanes = nsamp;
-    plan_tree(d, mode, 4 * ctx->cus, ninst, lds_only, max_terms > 0 ? max_terms : 1 << 30);
+    plan_tree(d, mode, mode == 0 ? nsamp : d.chi, 4 * ctx->cus, ninst, lds_only, max_terms > 0 ? max_terms : 1 << 30);
     const long long per = d.chi >> d.G;
     d.lanes = mode == 0 ? nsamp * per : tri_before(1ll << d.G, per, per);
     return d;
@@ -735,6 +732,12 @@ int init_ctx(cse_ctx *ctx, int device) {
     snprintf(ctx->name, sizeof(ctx->name), "%s (%s)", prop.name, prop.gcnArchName);
     if (strncmp(prop.gcnArchName, "gfx950", 6) != 0)
         return fail(ctx, CSE_ERR_HIP, "device %d is %s; this engine is built for gfx950", device, prop.gcnArchName);
+    // the sweep's leaf tables, kept for the context's life
+    const int plain = 1 << tree::LeafBits<false>::value, sign = 1 << tree::LeafBits<true>::value;
+    ENSURE(leaf, (size_t)(plain + sign));
+    hipLaunchKernelGGL(k_leaf_table, dim3((sign + 63) / 64), dim3(64), 0, ctx->stream, dp<uint8_t>(ctx->leaf),
+                       dp<uint8_t>(ctx->leaf) + plain);
+    HIPCHK(hipGetLastError());
     if (const char *ft = getenv("CSE_FLUSH_TERMS")) {
         const long long v = atoll(ft);
         if (v < 1 || v > CSE_FLUSH_TERMS_MAX)
@@ -809,7 +812,7 @@ void cse_destroy(cse_ctx *ctx) {
         if (g.exec) (void)hipGraphExecDestroy(g.exec);
     ctx->graphs.clear();
     DevBuf *bufs[] = {&ctx->s1, &ctx->s2, &ctx->out, &ctx->recs, &ctx->terms, &ctx->queue, &ctx->thr,
-                      &ctx->sexp, &ctx->L, &ctx->idx, &ctx->errflag, &ctx->lsh, &ctx->plan, &ctx->outb, &ctx->stack};
+                      &ctx->sexp, &ctx->L, &ctx->idx, &ctx->errflag, &ctx->lsh, &ctx->plan, &ctx->outb, &ctx->stack, &ctx->leaf};
     for (DevBuf *b : bufs)
         if (b->p) (void)hipFree(b->p);
     if (ctx->hstage.p) (void)hipHostFree(ctx->hstage.p);

@@ -38,8 +38,8 @@ inline __host__ __device__ long long tri_before(long long ch, long long nch, lon
 #define TREE_MAXG 12        // largest log2 of the terms of one lane
 // Words per lane of a wave's LDS stack: the most that leaves room for four
 // blocks of four waves on a CU (160 KB), next to the exact sweep's histogram
-#define TREE_LDS_WORDS0 39
-#define TREE_LDS_WORDS1 35
+#define TREE_LDS_WORDS0 38
+#define TREE_LDS_WORDS1 34
 // words of a saved form besides its rows
 #define TREE_STATE_WORDS 5
 
@@ -62,6 +62,8 @@ struct InstDesc {
     uint64_t seed;      // mode 0: Philox key of the random states
     long long first;    // mode 0: sample index of the first record
     int nlds;           // levels 1 .. nlds of the stack are in LDS
+    int leaf;           // levels up to this one only move the looked-up slots
+    int beyond;         // stack words (per lane) outside LDS
     int spare;
     uint8_t inv[64];    // column of each slot
     uint8_t ub[TREE_MAXG + 4];    // ub[g]: slots that index bits below g move
@@ -86,6 +88,7 @@ struct SweepArgs {
     unsigned long long *queue;
     uint32_t *stack;          // levels beyond LDS: stack_words x 64 per wave
     long long stack_words;
+    const uint8_t *leaf;      // table of the last slots (k_leaf_table)
     int32_t *terms;           // optional per-term output
     long long *zsum;          // mode 0: 4 per record
     double *kahan;            // mode 0: 2 per record; mode 1: 2 per instance

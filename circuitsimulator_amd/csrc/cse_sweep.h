@@ -37,54 +37,13 @@ DEV void tri_item(long long l, long long ch, long long nch, long long &r, long l
     c = g + off % per;
 }
 
-// FP32 value of 2^{P/2} e^{i pi m/4}
-DEV void term_f32(int P, int m, float &re, float &im) {
-    const float r = 0.70710678118654752f;
-    const int mm = m & 7;
-    const float c = (mm == 0) ? 1.f : (mm == 4) ? -1.f : (mm == 2 || mm == 6) ? 0.f : (mm == 1 || mm == 7) ? r : -r;
-    const float s = (mm == 2) ? 1.f : (mm == 6) ? -1.f : (mm == 0 || mm == 4) ? 0.f : (mm == 1 || mm == 3) ? r : -r;
-    const float mag = ldexpf((P & 1) ? 1.41421356237309505f : 1.f, P >> 1);
-    re = mag * c;
-    im = mag * s;
+// Kahan step: sum s with compensation c, plus v
+DEV void kahan1(float &s, float &c, float v) {
+    const float y = v - c;
+    const float t = s + y;
+    c = (t - s) - y;
+    s = t;
 }
-
-// Per-lane sums of the terms.
-struct LaneAcc {
-    long long c0, c1, c2, c3;   // exact Z[w] partial sums, scale 2^32 (mode 0)
-    float sr, cr, si, ci;       // Kahan FP32 partial sums
-    DEV void clear() {
-        c0 = c1 = c2 = c3 = 0;
-        sr = cr = si = ci = 0.f;
-    }
-    DEV static void kahan1(float &s, float &c, float v) {
-        const float y = v - c;
-        const float t = s + y;
-        c = (t - s) - y;
-        s = t;
-    }
-    // + 2^{p/2} w^m in Z[w] coordinates (scale 2^32, -64 <= p <= 0)
-    DEV void zomega(int p, int m) {
-        const long long v = 1ll << (32 + (p >> 1));
-        const int mm = m & 7;
-        int qa, qb;
-        long long sa, sb;
-        if (!(p & 1)) {
-            qa = mm; sa = v; qb = 0; sb = 0;
-        } else {
-            // sqrt2 w^m = w^{m+1} - w^{m+3}
-            qa = (mm + 1) & 7; sa = v;
-            qb = (mm + 3) & 7; sb = -v;
-        }
-        if (qa & 4) sa = -sa;
-        if (qb & 4) sb = -sb;
-        qa &= 3;
-        qb &= 3;
-        c0 += (qa == 0 ? sa : 0) + (qb == 0 ? sb : 0);
-        c1 += (qa == 1 ? sa : 0) + (qb == 1 ? sb : 0);
-        c2 += (qa == 2 ? sa : 0) + (qb == 2 ? sb : 0);
-        c3 += (qa == 3 ? sa : 0) + (qb == 3 ? sb : 0);
-    }
-};
 
 DEV double wave_sumf64(double v) {
 #pragma unroll
@@ -100,18 +59,29 @@ DEV long long wave_sum64(long long v) {
 // Saves the slots below c of a form (and its state words) to words 0 .. of p,
 // 64 lanes apart, and reads them back.  A holds toggles of the current term
 // that are not part of the node: `a` is A without them.
+template <int NH, int X> DEV void rows_save(const tree::Form<NH> &f, int c, uint32_t *p) {
+    if constexpr (X < 32) {
+        if (c <= X) return;
+        p[64 * (TREE_STATE_WORDS + X)] = f.lo[X];
+        if (c > X + 1) p[64 * (TREE_STATE_WORDS + X + 1)] = f.lo[X + 1];
+        rows_save<NH, X + 2>(f, c, p);
+    }
+}
+template <int NH, int X> DEV void rows_load(tree::Form<NH> &f, int c, const uint32_t *p) {
+    if constexpr (X < 32) {
+        if (c <= X) return;
+        f.lo[X] = p[64 * (TREE_STATE_WORDS + X)];
+        if (c > X + 1) f.lo[X + 1] = p[64 * (TREE_STATE_WORDS + X + 1)];
+        rows_load<NH, X + 2>(f, c, p);
+    }
+}
 template <int NH> DEV void form_save(const tree::Form<NH> &f, unsigned a, int c, uint32_t *p) {
     p[0] = f.d1;
     p[64] = f.d2;
     p[128] = a;
     p[192] = f.x2;
     p[256] = (f.z & 0x80000000u) | (f.q1 << 8) | f.nb;
-#pragma unroll
-    for (int x = 0; x < 32; x += 2)
-        if (c > x) {
-            p[64 * (TREE_STATE_WORDS + x)] = f.lo[x];
-            if (c > x + 1) p[64 * (TREE_STATE_WORDS + x + 1)] = f.lo[x + 1];
-        }
+    rows_save<NH, 0>(f, c, p);
 }
 template <int NH> DEV void form_load(tree::Form<NH> &f, int c, const uint32_t *p) {
     f.d1 = p[0];
@@ -122,13 +92,38 @@ template <int NH> DEV void form_load(tree::Form<NH> &f, int c, const uint32_t *p
     f.z = w & 0x80000000u;
     f.q1 = (w >> 8) & 0xffu;
     f.nb = w & 0xffu;
-#pragma unroll
-    for (int x = 0; x < 32; x += 2)
-        if (c > x) {
-            f.lo[x] = p[64 * (TREE_STATE_WORDS + x)];
-            if (c > x + 1) f.lo[x + 1] = p[64 * (TREE_STATE_WORDS + x + 1)];
-        }
+    rows_load<NH, 0>(f, c, p);
 }
+
+// What a term adds, by (p odd) 8 + m: 2^{(p odd)/2} w^m in the basis 1, w,
+// w^2, w^3 and as an FP32 pair, to be scaled by 2^{p >> 1}.
+struct TermTables {
+    double z[16][4];
+    float f[16][2];
+    DEV void fill(int t) {
+        if (t >= 16) return;
+        const int m = t & 7;
+        const float r = 0.70710678118654752f;
+        for (int k = 0; k < 4; k++) {
+            double v = 0.0;
+            if (t < 8) {
+                v = (m & 3) == k ? 1.0 : 0.0;
+                if (m & 4) v = -v;
+            } else {
+                // sqrt2 w^m = w^{m+1} - w^{m+3}
+                const int a = (m + 1) & 7, b = (m + 3) & 7;
+                if ((a & 3) == k) v += a & 4 ? -1.0 : 1.0;
+                if ((b & 3) == k) v -= b & 4 ? -1.0 : 1.0;
+            }
+            z[t][k] = v;
+        }
+        const float mag = t < 8 ? 1.f : 1.41421356237309505f;
+        const float c = m == 0 ? 1.f : m == 4 ? -1.f : m == 2 || m == 6 ? 0.f : m == 1 || m == 7 ? r : -r;
+        const float s = m == 2 ? 1.f : m == 6 ? -1.f : m == 0 || m == 4 ? 0.f : m == 1 || m == 3 ? r : -r;
+        f[t][0] = mag * c;
+        f[t][1] = mag * s;
+    }
+};
 
 }  // namespace
 
@@ -147,6 +142,8 @@ template <int NH, bool HT, int MODE> DEV void sweep_body(const SweepArgs &A) {
     __shared__ long long s_item;
     __shared__ double s_k[4];
     __shared__ unsigned long long s_ips[4];
+    __shared__ __align__(16) TermTables s_tab;
+    __shared__ uint8_t s_leaf[1 << tree::LeafBits<HT>::value];
     const int tid = (int)threadIdx.x, x = lane_id(), wv = uni(tid >> 6);
     uint32_t *const lst = &lstack[wv][x];
     uint32_t *const gst =
@@ -154,8 +151,12 @@ template <int NH, bool HT, int MODE> DEV void sweep_body(const SweepArgs &A) {
     int cur = -1;
     long long pend = 0;         // MODE 1: terms counted since the last flush
     unsigned long long ips = 0; // per lane, of instance cur
-    LaneAcc acc;
-    acc.clear();
+    // the lane's sums: Z[w] coefficients at scale 2^32 as integers in FP64
+    // (at most 2^G 2^32 <= 2^44, exact), Kahan FP32 pair
+    double c0 = 0.0, c1 = 0.0, c2 = 0.0, c3 = 0.0;
+    float sr = 0.f, cr = 0.f, si = 0.f, ci = 0.f;
+    s_tab.fill(tid);
+    for (int b = tid; b < 1 << tree::LeafBits<HT>::value; b += 256) s_leaf[b] = A.leaf[b];
     if (MODE == 1)
         for (int b = tid; b < HIST_STRIDE; b += 256) hist[b] = 0;
 
@@ -163,7 +164,7 @@ template <int NH, bool HT, int MODE> DEV void sweep_body(const SweepArgs &A) {
     auto flush = [&]() {
         const unsigned long long wi = (unsigned long long)wave_sum64((long long)ips);
         double wk = 0.0;
-        if (MODE == 1) wk = wave_sumf64((double)acc.sr - (double)acc.cr);
+        if (MODE == 1) wk = wave_sumf64((double)sr - (double)cr);
         if (x == 0) {
             s_ips[wv] = wi;
             s_k[wv] = wk;
@@ -185,7 +186,7 @@ template <int NH, bool HT, int MODE> DEV void sweep_body(const SweepArgs &A) {
                 atomicAdd(&h[b], (unsigned long long)v << (m == 4 ? 1 : 0));
                 if (m & 3) atomicAdd(&h[(b & ~7) | (8 - m)], (unsigned long long)v);
             }
-            acc.clear();
+            sr = cr = 0.f;
         }
         ips = 0;
         pend = 0;
@@ -259,9 +260,16 @@ template <int NH, bool HT, int MODE> DEV void sweep_body(const SweepArgs &A) {
         int ph0 = (int)((w0 >> 16) & 7), cnt0 = -n;
         if (NH > 0) {
             tree::StepsHi<NH, HT, NH - 1>::run(f, n);
-            tree::fold<HT>(f.d1h, f.d2h, f.Ah, f.Th, ph0, cnt0);
+            tree::fold<HT>(f.d1h, f.d2h, f.Ah, f.Th, ~0u, ph0, cnt0);
         }
-        // the term within the lane (Gray code of t), and what its bits toggle
+        // by index bit g (in lane g): the slots it toggles, their signs, the
+        // index j; by level: slots and place of the saved form
+        const int gl = x < TREE_MAXG ? x : TREE_MAXG;
+        const int v_lp = x < TREE_MAXG ? (int)(unsigned)D->LP[x] : 0;
+        const int v_lt = HT && x < TREE_MAXG && D->exact ? (int)(unsigned)D->L[x] : 0;
+        const int v_lev = (int)D->ub[gl] | (int)D->soff[gl] << 8;
+        const int nlds = D->nlds, leaf = D->leaf;
+        // the term within the lane (Gray code of t - 1), and what it toggles
         const unsigned T0 = f.T;
         unsigned gray = 0, ta = 0, tt = 0, tj = 0;
         // MODE 1: the lane's block holds the diagonal at term rl
@@ -277,37 +285,53 @@ template <int NH, bool HT, int MODE> DEV void sweep_body(const SweepArgs &A) {
             // the one lane that holds its diagonal
             if (valid && rl >= 0) ips += (unsigned long long)(D->chi - (long long)ri);
         }
-        if (MODE == 0) acc.clear();
-        int lev = G, c0 = n < 32 ? n : 32;
+        if (MODE == 0) {
+            c0 = c1 = c2 = c3 = 0.0;
+            sr = cr = si = ci = 0.f;
+        }
+        int lev = G, top = n < 32 ? n : 32;
+        int p0 = 0, m0 = 0;   // the term's exponent and phase without its leaf slots
         for (int t = 1;; t++) {
-            // down from c0 to the term, saving the form at every level
-            while (true) {
-                const int c1 = lev ? (int)D->ub[lev] : 0;
-                tree::Steps<NH, HT, 31>::run(f, c1, (unsigned)(c0 - c1));
-                if (lev == 0) break;
-                if (lev <= D->nlds) form_save(f, f.A ^ ta, c1, lst + 64 * (int)D->soff[lev]);
-                else form_save(f, f.A ^ ta, c1, gst + 64 * (int)D->soff[lev]);
-                c0 = c1;
-                lev--;
-            }
-            int ph = ph0, cnt = cnt0;
-            tree::fold<HT>(f.d1, f.d2, f.A, f.T, ph, cnt);
-            const int p = cnt - (int)f.nb;
-            const int m = (ph + 2 * (int)f.q1 + 4 * __popc(f.x2)) & 7;
-            const bool nz = valid && (int)f.z >= 0;
-            float vr, vi;
-            if (MODE == 0) {
-                if (nz) {
-                    acc.zomega(p, m);
-                    term_f32(p, m, vr, vi);
-                    LaneAcc::kahan1(acc.sr, acc.cr, vr);
-                    LaneAcc::kahan1(acc.si, acc.ci, vi);
+            if (lev >= leaf) {
+                // down from `top` to the leaf slots, saving the form at every
+                // level on the way
+                while (true) {
+                    const int w = __builtin_amdgcn_readlane(v_lev, lev);
+                    const int c = lev > leaf ? w & 0xff : TREE_LEAF;
+                    if (top > c) tree::steps<NH, HT>(f, top, c);
+                    if (lev == leaf) break;
+                    uint32_t *const st = lev <= nlds ? lst : gst;
+                    form_save(f, f.A ^ ta, c, st + 64 * (w >> 8));
+                    top = c;
+                    lev--;
                 }
+                int cnt = cnt0;
+                m0 = ph0;
+                tree::fold<HT>(f.d1, f.d2, f.A, f.T, ~(~0u << (32 - TREE_LEAF)), m0, cnt);
+                p0 = cnt - (int)f.nb;
+                m0 += 2 * (int)f.q1 + 4 * __popc(f.x2);
+            }
+            // the leaf slots from the table: phase, steps of the second kind,
+            // whether the sum is 0
+            const unsigned lf = s_leaf[tree::leaf_index<HT>(f.A, f.T, f.d1, f.d2, f.lo[1])];
+            const int p = p0 + (int)((lf >> 3) & 7u);
+            const int m = (m0 + (int)lf) & 7;
+            const bool nz = valid && (int)f.z >= 0 && lf < 128u;
+            if (MODE == 0) {
+                const int row = ((p & 1) << 3) | m;
+                const double s = ldexp(1.0, nz ? 32 + (p >> 1) : -2000);
+                c0 = fma(s_tab.z[row][0], s, c0);
+                c1 = fma(s_tab.z[row][1], s, c1);
+                c2 = fma(s_tab.z[row][2], s, c2);
+                c3 = fma(s_tab.z[row][3], s, c3);
+                const float e = ldexpf(1.f, nz ? p >> 1 : -2000);
+                kahan1(sr, cr, s_tab.f[row][0] * e);
+                kahan1(si, ci, s_tab.f[row][1] * e);
             } else if (nz && (int)gray >= rl) {
                 const bool off = (int)gray != rl;
-                term_f32(p - sexp, m, vr, vi);
-                LaneAcc::kahan1(acc.sr, acc.cr, off ? 2.f * vr : vr);
-                atomicAdd(&hist[(sexp - p) * 8 + m], off && m == 0 ? 2u : 1u);
+                const int P = p - sexp;
+                kahan1(sr, cr, ldexpf(s_tab.f[((P & 1) << 3) | m][0], (P >> 1) + (off ? 1 : 0)));
+                atomicAdd(&hist[m - 8 * P], off && m == 0 ? 2u : 1u);
             }
             if (A.terms && live) {
                 long long j = jhi ^ tj;
@@ -333,45 +357,55 @@ template <int NH, bool HT, int MODE> DEV void sweep_body(const SweepArgs &A) {
             if (t == lg) break;
             const int g = __builtin_ctz(t);
             gray ^= 1u << g;
-            ta ^= (unsigned)D->LP[g];
-            if (HT && D->exact) tt ^= (unsigned)D->L[g];
             if (A.terms) tj ^= D->jmap[g];
-            c0 = (int)D->ub[g + 1];
-            if (g + 1 <= D->nlds) form_load(f, c0, lst + 64 * (int)D->soff[g + 1]);
-            else form_load(f, c0, gst + 64 * (int)D->soff[g + 1]);
-            f.A ^= ta;
-            if (HT) f.T = T0 ^ tt;
+            const unsigned la = (unsigned)__builtin_amdgcn_readlane(v_lp, g);
+            const unsigned lt = HT ? (unsigned)__builtin_amdgcn_readlane(v_lt, g) : 0u;
+            ta ^= la;
+            tt ^= lt;
             lev = g;
+            if (g < leaf) {
+                // only leaf slots change
+                f.A ^= la;
+                if (HT) f.T ^= lt;
+            } else {
+                const int w = __builtin_amdgcn_readlane(v_lev, g + 1);
+                top = w & 0xff;
+                form_load(f, top, (g + 1 <= nlds ? lst : gst) + 64 * (w >> 8));
+                f.A ^= ta;
+                if (HT) f.T = T0 ^ tt;
+            }
         }
         if (MODE == 0) {
             if (valid) ips += (unsigned long long)lg;
-            // the record's sums over the lanes that share it: aligned groups
-            // of up to a wave, then atomics when several waves do
+            // the record's sums over the lanes that share it (integers below
+            // 2^50, exact in FP64): aligned groups of up to a wave, then atomics when several waves do
             const int seg = k - G < 6 ? 1 << (k - G) : 64;
-            double kr = (double)acc.sr - (double)acc.cr, ki = (double)acc.si - (double)acc.ci;
+            double kr = (double)sr - (double)cr, ki = (double)si - (double)ci;
             for (int o = 1; o < seg; o <<= 1) {
-                acc.c0 += (long long)shfl_xor64((u64)acc.c0, o);
-                acc.c1 += (long long)shfl_xor64((u64)acc.c1, o);
-                acc.c2 += (long long)shfl_xor64((u64)acc.c2, o);
-                acc.c3 += (long long)shfl_xor64((u64)acc.c3, o);
+                c0 += __shfl_xor(c0, o, 64);
+                c1 += __shfl_xor(c1, o, 64);
+                c2 += __shfl_xor(c2, o, 64);
+                c3 += __shfl_xor(c3, o, 64);
                 kr += __shfl_xor(kr, o, 64);
                 ki += __shfl_xor(ki, o, 64);
             }
             if (valid && (x & (seg - 1)) == 0) {
                 unsigned long long *z = (unsigned long long *)A.zsum + 4 * (size_t)(D->rec_off + r);
                 double *kz = A.kahan + 2 * (size_t)(D->rec_off + r);
+                const unsigned long long z0 = (unsigned long long)(long long)c0, z1 = (unsigned long long)(long long)c1;
+                const unsigned long long z2 = (unsigned long long)(long long)c2, z3 = (unsigned long long)(long long)c3;
                 if (k - G <= 6) {
-                    z[0] = (unsigned long long)acc.c0;
-                    z[1] = (unsigned long long)acc.c1;
-                    z[2] = (unsigned long long)acc.c2;
-                    z[3] = (unsigned long long)acc.c3;
+                    z[0] = z0;
+                    z[1] = z1;
+                    z[2] = z2;
+                    z[3] = z3;
                     kz[0] = kr;
                     kz[1] = ki;
                 } else {
-                    atomicAdd(&z[0], (unsigned long long)acc.c0);
-                    atomicAdd(&z[1], (unsigned long long)acc.c1);
-                    atomicAdd(&z[2], (unsigned long long)acc.c2);
-                    atomicAdd(&z[3], (unsigned long long)acc.c3);
+                    atomicAdd(&z[0], z0);
+                    atomicAdd(&z[1], z1);
+                    atomicAdd(&z[2], z2);
+                    atomicAdd(&z[3], z3);
                     atomicAdd(&kz[0], kr);
                     atomicAdd(&kz[1], ki);
                 }
@@ -379,6 +413,24 @@ template <int NH, bool HT, int MODE> DEV void sweep_body(const SweepArgs &A) {
         }
     }
     if (cur >= 0) flush();
+}
+
+// The table of the leaf slots: every form on TREE_LEAF slots taken through its
+// steps.  Bits 0..2 the phase, 3..5 the steps of the second kind, 7 set when
+// the sum is 0.
+template <bool HT> DEV void leaf_entry(unsigned i, uint8_t *out) {
+    tree::Form<0> f = {};
+    tree::leaf_form<HT>(i, f);
+    tree::steps<0, HT>(f, TREE_LEAF, 0);
+    int ph = 0, cnt = 0;
+    tree::fold<HT>(f.d1, f.d2, f.A, f.T, ~0u, ph, cnt);
+    ph += 2 * (int)f.q1 + 4 * __popc(f.x2);
+    out[i] = (uint8_t)((ph & 7) | ((cnt - (int)f.nb) << 3) | ((int)f.z < 0 ? 128 : 0));
+}
+extern "C" __global__ void k_leaf_table(uint8_t *plain, uint8_t *sign) {
+    const unsigned i = blockIdx.x * blockDim.x + threadIdx.x;
+    if (i < 1u << tree::LeafBits<false>::value) leaf_entry<false>(i, plain);
+    if (i < 1u << tree::LeafBits<true>::value) leaf_entry<true>(i, sign);
 }
 
 #define SWEEP_KERNEL(NAME, NH, HT, MODE, WAVES)                                            \

@@ -55,6 +55,8 @@ constexpr unsigned TA = 0xF0, TB = 0xCC, TC = 0xAA;
 // the three-operand boolean function of truth table F in one instruction
 #define TREE_B3(a, b, c, F) ((cse::tree::u32)__builtin_amdgcn_bitop3_b32((a), (b), (c), (F) & 0xffu))
 #define TREE_POP(v) __popc(v)
+// the top n bits of v shifted in below i
+#define TREE_SHIN(i, v, n) ((cse::tree::u32)__builtin_amdgcn_alignbit((i), (v), 32 - (n)))
 template <u32 K> TREE_DEV u32 andk(u32 v) {
     u32 r;
     asm("v_and_b32 %0, %2, %1" : "=v"(r) : "v"(v), "n"(K));
@@ -161,6 +163,7 @@ inline u32 tree_b3(u32 a, u32 b, u32 c, unsigned F) {
     return r;
 }
 #define TREE_B3(a, b, c, F) (cse::tree::tree_b3((a), (b), (c), (F) & 0xffu))
+#define TREE_SHIN(i, v, n) (((i) << (n)) | ((v) >> (32 - (n))))
 template <u32 K> inline u32 andk(u32 v) { return v & K; }
 inline u32 nz1(u32 t) { return t ? ~0u : 0u; }
 inline void nz2(u32 &t, u32 &u) {
@@ -341,16 +344,30 @@ template <int NH, bool HT, int C> TREE_DEV void step_hi(Form<NH> &f) {
     f.Ah ^= oh;
 }
 
-// Steps of the slots c1 + cn - 1 .. c1 (uniform bounds, c1 + cn <= 32).
-template <int NH, bool HT, int C> struct Steps {
-    static TREE_DEV void run(Form<NH> &f, int c1, u32 cn) {
-        if ((u32)(C - c1) < cn) step<NH, HT, C>(f);
-        Steps<NH, HT, C - 1>::run(f, c1, cn);
+// Steps of the slots whose bits are set in `todo` (uniform; bit C for slot C),
+// the highest first.  A stretch tests a bit a slot, in groups of 16, 8 and 4
+// behind one test each: the |H^t> sweep takes two steps a stretch, and with
+// two comparisons for each of the 32 slots its scalar instructions, one a
+// cycle and CU, outlasted the vector ones.
+template <int NH, bool HT, int C, int N> struct Steps {
+    static TREE_DEV void run(Form<NH> &f, u32 todo) {
+        if (N <= 2 || (todo & (((1u << N) - 1u) << C))) {
+            Steps<NH, HT, C + N / 2, N / 2>::run(f, todo);
+            Steps<NH, HT, C, N / 2>::run(f, todo);
+        }
     }
 };
-template <int NH, bool HT> struct Steps<NH, HT, -1> {
-    static TREE_DEV void run(Form<NH> &, int, u32) {}
+template <int NH, bool HT, int C> struct Steps<NH, HT, C, 1> {
+    static TREE_DEV void run(Form<NH> &f, u32 todo) {
+        if (todo & (1u << C)) step<NH, HT, C>(f);
+    }
 };
+// Steps of the slots c0 - 1 .. c1, 32 >= c0 > c1.
+template <int NH, bool HT> TREE_DEV void steps(Form<NH> &f, int c0, int c1) {
+    const u32 todo = (~0u >> (32 - c0)) & (~0u << c1);
+    Steps<NH, HT, 16, 16>::run(f, todo);
+    Steps<NH, HT, 0, 16>::run(f, todo);
+}
 template <int NH, bool HT, int C> struct StepsHi {
     static TREE_DEV void run(Form<NH> &f, int c0) {
         if (c0 > 32 + C) step_hi<NH, HT, C>(f);
@@ -361,15 +378,43 @@ template <int NH, bool HT> struct StepsHi<NH, HT, -1> {
     static TREE_DEV void run(Form<NH> &, int) {}
 };
 
-// What the finished slots below 32 (word arguments) or above (the h words)
-// give: phase in units of 1 and the count of active slots less the steps of
-// the first kind; the third kind's share (nb, q1, x2) is added at the end.
-template <bool HT> TREE_DEV void fold(u32 d1, u32 d2, u32 A, u32 T, int &ph, int &cnt) {
-    const u32 a1 = A & d1;
+// What finished slots give, those of `in` of a word's 32: phase in units of 1
+// and the count of active slots less the steps of the first kind; the third
+// kind's share (nb, q1, x2) is added at the end.
+template <bool HT> TREE_DEV void fold(u32 d1, u32 d2, u32 A, u32 T, u32 in, int &ph, int &cnt) {
+    const u32 a1 = A & d1 & in;
     const int na = TREE_POP(a1);
-    cnt += TREE_POP(A) - na;
+    cnt += TREE_POP(A & in) - na;
     ph += na - 2 * TREE_POP(a1 & (HT ? d2 ^ T : d2));
-    if (HT) ph += 2 * TREE_POP(T & ~A & d1) + 4 * TREE_POP(T & ~A & d2);
+    if (HT) {
+        const u32 t = T & ~A & in;
+        ph += 2 * TREE_POP(t & d1) + 4 * TREE_POP(t & d2);
+    }
+}
+
+// The last TREE_LEAF slots are looked up: the index of their form is the top
+// bits of A, d1, d2 and J_10 (and T).
+#define TREE_LEAF 2
+template <bool HT> struct LeafBits {
+    static constexpr int value = HT ? 9 : 7;
+};
+template <bool HT> TREE_DEV u32 leaf_index(u32 A, u32 T, u32 d1, u32 d2, u32 row1) {
+    u32 i = A >> 30;
+    i = TREE_SHIN(i, d1, 2);
+    i = TREE_SHIN(i, d2, 2);
+    i = TREE_SHIN(i, row1, 1);
+    return HT ? TREE_SHIN(i, T, 2) : i;
+}
+template <bool HT> TREE_DEV void leaf_form(u32 i, Form<0> &f) {
+    if (HT) {
+        f.T = i << 30;
+        i >>= 2;
+    }
+    f.lo[1] = i << 31;
+    f.lo[0] = (i & 1u) << 30;
+    f.d2 = (i >> 1) << 30;
+    f.d1 = (i >> 3) << 30;
+    f.A = (i >> 5) << 30;
 }
 
 }  // namespace tree

@@ -34,12 +34,12 @@ template <int NH, bool HT> static void go(int n, const uint64_t *row, const uint
     int ph = 0, cnt = 0;
     if (NH) {
         StepsHi<NH, HT, NH - 1>::run(f, n);
-        fold<HT>(f.d1h, f.d2h, f.Ah, f.Th, ph, cnt);
+        fold<HT>(f.d1h, f.d2h, f.Ah, f.Th, ~0u, ph, cnt);
     }
     const int low = n < 32 ? n : 32;
-    Steps<NH, HT, 31>::run(f, low / 2, (u32)(low - low / 2));   // two stretches, as a tree's levels
-    Steps<NH, HT, 31>::run(f, 0, (u32)(low / 2));
-    fold<HT>(f.d1, f.d2, f.A, f.T, ph, cnt);
+    steps<NH, HT>(f, low, low / 2);   // two stretches, as a tree's levels
+    if (low / 2 > 0) steps<NH, HT>(f, low / 2, 0);
+    fold<HT>(f.d1, f.d2, f.A, f.T, ~0u, ph, cnt);
     out[0] = (f.z >> 31) ? 0 : 1;
     out[1] = cnt - (int)f.nb - n;
     out[2] = (ph + 2 * (int)f.q1 + 4 * TREE_POP(f.x2)) & 7;
