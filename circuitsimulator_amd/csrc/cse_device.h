@@ -91,28 +91,76 @@ DEV P4 philox(uint32_t c0, uint32_t c1, uint32_t c2, uint32_t c3, uint32_t k0, u
     return o;
 }
 
-// Sequential 64-bit draws from the stream (key, stream id, domain): word w
-// is output (w & 3) of block w >> 2; a 64-bit draw is words (w, w+1).
+// 64-bit draws from the stream (key, stream id, domain): draw i is words 2 (i &
+// 1) and 2 (i & 1) + 1 of block i >> 1.  Lane l computes block l of a window
+// of 64 blocks, so the wave draws 128 values for one evaluation of Philox;
+// next64() hands them out in order, the same in every lane.
 struct Stream {
     uint32_t k0, k1, s0, s1, dom;
-    uint64_t w;
-    P4 blk;
-    uint64_t blk_id;
+    uint64_t i;     // next draw (uniform)
+    u64 even, odd;  // draws 2 l and 2 l + 1 of the window, in lane l
     DEV void init(uint64_t key, uint64_t stream, uint32_t domain) {
         k0 = (uint32_t)key; k1 = (uint32_t)(key >> 32);
         s0 = (uint32_t)stream; s1 = (uint32_t)(stream >> 32);
-        dom = domain; w = 0; blk_id = ~0ull;
+        dom = domain; i = 0;
     }
-    DEV uint32_t word() {
-        uint64_t b = w >> 2;
-        if (b != blk_id) { blk = philox((uint32_t)b, s0, s1, dom, k0, k1); blk_id = b; }
-        const int q = (int)(w & 3);
-        uint32_t v = q == 0 ? blk.x[0] : q == 1 ? blk.x[1] : q == 2 ? blk.x[2] : blk.x[3];
-        w++;
+    DEV void block(uint32_t b, u64 &e, u64 &o) const {
+        const P4 p = philox(b, s0, s1, dom, k0, k1);
+        e = (u64)p.x[0] | ((u64)p.x[1] << 32);
+        o = (u64)p.x[2] | ((u64)p.x[3] << 32);
+    }
+    DEV u64 next64() {
+        if ((i & 127) == 0) block((uint32_t)(i >> 1) + (uint32_t)lane_id(), even, odd);
+        const u64 v = rl64(i & 1 ? odd : even, (int)((i >> 1) & 63));
+        i++;
         return v;
     }
-    DEV u64 next64() { u64 lo = word(); u64 hi = word(); return lo | (hi << 32); }
+    // draw i + lane, a different one in every lane (i does not move)
+    DEV u64 lane64() const {
+        const uint64_t d = i + (uint64_t)lane_id();
+        u64 e, o;
+        block((uint32_t)(d >> 1), e, o);
+        return d & 1 ? o : e;
+    }
 };
+
+// The value of lane x ^ S, in registers: DPP within rows of 16 lanes (a
+// rotation by 8 is the exchange, by 4 or 12 depending on the lane), the
+// half-wave and row swaps across them.  All lanes active.
+template <int S> DEV unsigned xor_lane32(unsigned v) {
+    const int x = lane_id();
+    if constexpr (S == 1) return dpp_mov<0xB1>(v);
+    else if constexpr (S == 2) return dpp_mov<0x4E>(v);
+    else if constexpr (S == 4) {
+        const unsigned down = dpp_mov<0x124>(v), up = dpp_mov<0x12C>(v);
+        return x & 4 ? down : up;
+    } else if constexpr (S == 8) return dpp_mov<0x128>(v);
+    else if constexpr (S == 16) {
+        const auto r = __builtin_amdgcn_permlane16_swap(v, v, false, false);
+        return x & 16 ? r[0] : r[1];
+    } else {
+        const auto r = __builtin_amdgcn_permlane32_swap(v, v, false, false);
+        return x & 32 ? r[0] : r[1];
+    }
+}
+template <int S> DEV u64 xor_lane(u64 v) {
+    return (u64)xor_lane32<S>((unsigned)v) | ((u64)xor_lane32<S>((unsigned)(v >> 32)) << 32);
+}
+
+// Transpose of a 64x64 bit matrix held one row per lane: log2 steps, each
+// exchanging the off-diagonal blocks of the lanes that differ in one bit.
+template <int S> DEV u64 transpose_step(u64 v, u64 m) {
+    const u64 o = xor_lane<S>(v);
+    return lane_id() & S ? (v & ~m) | ((o & ~m) >> S) : (v & m) | ((o & m) << S);
+}
+DEV u64 transpose64(u64 v) {
+    v = transpose_step<32>(v, 0x00000000ffffffffull);
+    v = transpose_step<16>(v, 0x0000ffff0000ffffull);
+    v = transpose_step<8>(v, 0x00ff00ff00ff00ffull);
+    v = transpose_step<4>(v, 0x0f0f0f0f0f0f0f0full);
+    v = transpose_step<2>(v, 0x3333333333333333ull);
+    return transpose_step<1>(v, 0x5555555555555555ull);
+}
 
 // ------------------------------------------------------- reference layout
 struct RState {
@@ -259,9 +307,10 @@ DEV bool rs_random_state(RState &s, int n, const uint64_t *thr, uint64_t key, ui
     Stream rng;
     rng.init(key, stream, 1u);
     const u64 nm = lowmask(n);
-    u64 r = rng.next64() >> 11;
-    int d = 0;
-    while (d < n && !(r + 1 <= thr[d])) d++;
+    const u64 r = rng.next64() >> 11;
+    // the first d with r < thr[d] (the thresholds do not decrease), else n
+    const u64 ok = ballot(x < n && r + 1 <= thr[x < n ? x : 0]);
+    const int d = ok ? __builtin_ctzll(ok) : n;
     const int k = n - d;
     rs_init(s, n);
     int iters = 0;
@@ -274,11 +323,9 @@ DEV bool rs_random_state(RState &s, int n, const uint64_t *thr, uint64_t key, ui
     u64 D1 = rng.next64() & nm;
     u64 D2 = rng.next64() & nm;
     s.d = 2 * (int)((D1 >> x) & 1ull) + 4 * (int)((D2 >> x) & 1ull);
-    for (int i = 0; i < k; i++) {
-        u64 lo = rng.next64() & lowmask(i);
-        if (x == i) s.J |= lo;
-        if ((lo >> x) & 1ull) s.J |= bit(i);
-    }
+    // draw x of the next k is row x below the diagonal
+    const u64 lo = x < k ? rng.lane64() & lowmask(x) : 0ull;
+    s.J = lo | transpose64(lo);
     if (x < k && ((D1 >> x) & 1ull)) s.J |= bit(x);
     s.Q = 0;
     return true;

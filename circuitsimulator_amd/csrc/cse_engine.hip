@@ -104,7 +104,7 @@ struct cse_ctx {
 // that device is created, and host code only ever uses that address.
 constexpr int kStaticMaxLogChi = 13;
 constexpr long long kStaticMaxChi = 1ll << kStaticMaxLogChi;
-constexpr size_t kStaticPlanBytes = 4096;  // one instance: 3,072 B
+constexpr size_t kStaticPlanBytes = 4096;  // one instance: 3,328 B
 constexpr size_t kStaticOutBytes = 8448;   // one instance's results block: 8,288 B
 constexpr size_t kScratchQueue = 0;
 constexpr size_t kScratchPlan = 256;
@@ -222,15 +222,30 @@ int ensure_thresholds(cse_ctx *ctx) {
     return CSE_OK;
 }
 
-DevProjector to_dev(const cse_projector *P) {
+// products: for an |H^t> instance's sweep, the generators in the coordinates
+// of its records (to_products: u = x_2q in column 2q and s = x_2q + x_2q+1 in
+// column 2q+1, after a controlled sign on each pair).  i^m Z(z) X(x) picks up
+// the sign of x_u x_v, z_u ^= x_v and z_v ^= x_u from the controlled sign;
+// then z_u ^= z_v and x_s = x_u + x_v.
+DevProjector to_dev(const cse_projector *P, bool products = false) {
     DevProjector d;
     memset(&d, 0, sizeof(d));
     if (!P) return d;
     d.nstabs = P->nstabs;
     for (int g = 0; g < P->nstabs && g < 64; g++) {
         d.phase[g] = P->phase[g] & 3;
-        d.xs[g] = P->xs[g];
-        d.zs[g] = P->zs[g];
+        uint64_t x = P->xs[g], z = P->zs[g];
+        if (products) {
+            const int pairs = P->nqubits & ~1;
+            const uint64_t even = 0x5555555555555555ull & (pairs >= 64 ? ~0ull : (1ull << pairs) - 1);
+            const uint64_t xu = x & even, xv = (x >> 1) & even;
+            d.phase[g] = (d.phase[g] + 2 * (__builtin_popcountll(xu & xv) & 1)) & 3;
+            z ^= xv | (xu << 1);
+            z ^= (z >> 1) & even;
+            x ^= xu << 1;
+        }
+        d.xs[g] = x;
+        d.zs[g] = z;
     }
     return d;
 }
@@ -672,16 +687,18 @@ InstDesc make_inst(const cse_ctx *ctx, int mode, int t, int k, int exact, const 
             col[s] = (uint8_t)(odd && b == 0 ? t - 1 : 2 * q + 1);
             if (u >= 0) col[u] = (uint8_t)(2 * q);
             d.LP[b] = slot_word(s);
-            d.L[b] = u >= 0 ? slot_word(u) : 0ull;
+            d.LT[b] = u >= 0 ? slot_word(u) : 0ull;
+            d.col[b] = 1ull << col[s];
+            d.sgn[b] = u >= 0 ? 1ull << col[u] : 0ull;
             d.jmap[b] = 1u << b;
             if (b < TREE_MAXG) d.ub[b + 1] = (uint8_t)(s + 1);
         }
     } else {
-        cse_chain_basis(t, k, L, TREE_MAXG, d.L, d.jmap, d.ub, col);
+        cse_chain_basis(t, k, L, TREE_MAXG, d.col, d.jmap, d.ub, col);
         uint8_t pos[64];
         for (int p = 0; p < t; p++) pos[col[p]] = (uint8_t)p;
         for (int b = 0; b < k; b++)
-            for (uint64_t r = d.L[b]; r; r &= r - 1) d.LP[b] |= slot_word(pos[__builtin_ctzll(r)]);
+            for (uint64_t r = d.col[b]; r; r &= r - 1) d.LP[b] |= slot_word(pos[__builtin_ctzll(r)]);
     }
     for (int p = 0; p < 64; p++) d.inv[p] = p < t ? col[p] : (uint8_t)p;
     plan_tree(d, mode, mode == 0 ? nsamp : d.chi, 4 * ctx->cus, ninst, lds_only, max_terms > 0 ? max_terms : 1 << 30);
@@ -1001,7 +1018,7 @@ static int sampled_batch(cse_ctx *ctx, const cse_sampled_instance *in, int ninst
         InstDesc d = make_inst(ctx, 0, in[i].P.nqubits, in[i].k, in[i].exact, in[i].L, in[i].count, ninst, false, chunk);
         d.seed = in[i].seed;
         d.first = in[i].first;
-        pl.add(d, to_dev(&in[i].P), in[i].count, (d.lanes + 255) / 256, in[i].count * d.chi);
+        pl.add(d, to_dev(&in[i].P, in[i].exact != 0), in[i].count, (d.lanes + 255) / 256, in[i].count * d.chi);
         want_terms = want_terms || res[i].terms != nullptr;
     }
     if (pl.nrec > kMaxSamples) return fail(ctx, CSE_ERR_ARG, "%lld samples above 2^24 per call", pl.nrec);
@@ -1128,7 +1145,7 @@ static int exact_batch(cse_ctx *ctx, const cse_instance *in, int ninst, int chun
     for (int i = 0; i < ninst; i++) {
         const InstDesc d =
             make_inst(ctx, 1, in[i].P.nqubits, in[i].k, in[i].exact, in[i].L, 0, ninst, use_static, chunk);
-        pl.add(d, to_dev(&in[i].P), d.chi, (d.lanes + 255) / 256, d.chi * (d.chi + 1) / 2);
+        pl.add(d, to_dev(&in[i].P, in[i].exact != 0), d.chi, (d.lanes + 255) / 256, d.chi * (d.chi + 1) / 2);
     }
     if (terms_out && pl.nterms > (1ll << 31)) return fail(ctx, CSE_ERR_ARG, "per-term output too large");
     int rc = use_static ? bind_static_mem(ctx, pl, hup, hstage) : bind_ctx_mem(ctx, pl, 1, terms_out != nullptr);

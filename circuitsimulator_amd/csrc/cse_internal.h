@@ -68,10 +68,12 @@ struct InstDesc {
     uint8_t inv[64];    // column of each slot
     uint8_t ub[TREE_MAXG + 4];    // ub[g]: slots that index bits below g move
     uint16_t soff[TREE_MAXG + 4]; // first word of level g's part of its stack
-    // per index bit: the slots it toggles (LP, bits as in a record), and by
-    // columns (|L>) or the slots whose sign it toggles (|H^t>, as LP)
+    // per index bit: the slots it toggles and the slots whose sign it toggles
+    // (|H^t>), bits as in a record, and both as columns of the state
     uint64_t LP[TREE_MAXLOG];
-    uint64_t L[TREE_MAXLOG];
+    uint64_t LT[TREE_MAXLOG];
+    uint64_t col[TREE_MAXLOG];
+    uint64_t sgn[TREE_MAXLOG];
     uint32_t jmap[TREE_MAXLOG];   // the reference's index j of each bit
 };
 

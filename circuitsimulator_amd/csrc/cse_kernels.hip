@@ -320,20 +320,6 @@ DEV u64 shfl64(u64 v, int lane) {
     return ((u64)hi << 32) | lo;
 }
 
-// Transpose of a 64x64 bit matrix held one row per lane: log2 steps, each
-// exchanging the off-diagonal blocks of the lanes that differ in one bit.
-DEV u64 transpose64(u64 v) {
-    const int x = lane_id();
-    u64 m = 0x00000000ffffffffull;
-#pragma unroll
-    for (int s = 32; s >= 1; s >>= 1) {
-        const u64 o = shfl_xor64(v, s);
-        v = (x & s) ? (v & ~m) | ((o & ~m) >> s) : (v & m) | ((o & m) << s);
-        m ^= m << (s >> 1);
-    }
-    return v;
-}
-
 // slot x at bit 31 - x of each half, as the sweep keeps its words
 DEV u64 brev32x2(u64 v) { return (u64)__brev((unsigned)v) | (u64)__brev((unsigned)(v >> 32)) << 32; }
 
@@ -344,30 +330,26 @@ DEV u64 brev32x2(u64 v) { return (u64)__brev((unsigned)v) | (u64)__brev((unsigne
 //    #edges(J in H), D_a -> -D_a on H, D_x += 4 |J_x & H|;
 //  * the slot of another column q is the multiplier of x_q = h_q + G_.q . z:
 //    J_q = the column of G, D_q = 4 (h_q + |column & H|);
-//  * slots are the columns in the order D.inv: rows, then (by a transpose)
-//    columns of the symmetric matrix move to it.
+//  * slots are the columns in the order D.inv.  The matrix is U + U^T with U
+//    the pivot rows' part of it (J below the diagonal, G at the other
+//    columns), and U's rows, then by a transpose its columns move to their
+//    slots.
 DEV void store_form(const AState &s, const InstDesc &D, int sexp, uint64_t *rec) {
     const int x = lane_id();
     const int n = D.n;
+    const int src = x < n ? (int)D.inv[x] : x;
     const bool a = lane_in(s.act);
     const u64 H = s.act & s.h, nonact = lowmask(n) & ~s.act;
-    u64 M = a ? (s.J & s.act & ~bit(x)) : 0ull;
+    const u64 J = a ? s.J & s.act & ~bit(x) : 0ull, Jl = J & lowmask(x);
     int d = a ? (s.d & 6) : 0;
     const int Q = s.Q + 2 * __popcll(ballot(lane_in(H) && (d & 2))) + 4 * __popcll(ballot(lane_in(H) && (d & 4))) +
-                  4 * __popcll(ballot(lane_in(H) && par64(M & H & lowmask(x))));
+                  4 * __popcll(ballot(lane_in(H) && par64(Jl & H)));
+    const u64 hq = s.h ^ wave_xor(lane_in(H) ? s.G : 0ull);
     if (lane_in(H)) d = (8 - d) & 7;
-    d = (d + 4 * par64(M & H)) & 7;
-    if (a) M |= s.G & nonact;
-    for (u64 rest = nonact; rest; rest &= rest - 1) {
-        const int q = __builtin_ctzll(rest);
-        const u64 c = ballot(a && ((s.G >> q) & 1ull));
-        if (x == q) {
-            M = c;
-            d = 4 * ((int)((s.h >> q) & 1ull) ^ par64(c & H));
-        }
-    }
-    const int src = x < n ? (int)D.inv[x] : x;
-    M = shfl64(transpose64(shfl64(M, src)), src);
+    d = (d + 4 * par64(J & H)) & 7;
+    if (!a) d = 4 * (int)((hq & nonact) >> x & 1ull);
+    const u64 Ut = shfl64(transpose64(shfl64(a ? Jl | (s.G & nonact) : 0ull, src)), src);
+    const u64 M = Ut ^ transpose64(Ut);
     d = __shfl(d, src, 64);
     const bool f = __shfl((int)((nonact >> x) & 1ull), src, 64) != 0;
     const u64 d1 = ballot(d & 2), d2 = ballot(d & 4), F = ballot(f);
@@ -380,61 +362,54 @@ DEV void store_form(const AState &s, const InstDesc &D, int sexp, uint64_t *rec)
     rec[REC_ROWS + x] = brev32x2(M);
 }
 
-// Reduced row echelon basis of the active rows (basis changes of the form,
-// so the state is unchanged), rows moved to their pivot lanes, then the
-// record.  For an |H^t> instance the state is first taken through the
-// Clifford that makes every pair's two terms products: with u = x_2q and s =
-// x_2q + x_2q+1, the term with coupling is the sum over u and s after a
-// controlled sign on (x_2q, x_2q+1), and |00> + |11> is s = 0 with the sum
-// over u signed (-1)^u (the same controlled sign undone).
-DEV void to_record(const RState &r, const InstDesc &D, int sexp, uint64_t *rec) {
-    const int x = lane_id();
-    AState s;
-    to_astate(r, s);
-    if (D.exact) {
-        for (int u = 0; u + 1 < D.n; u += 2) {
-            const u64 cu = ballot(x < r.k && ((s.G >> u) & 1ull)), cv = ballot(x < r.k && ((s.G >> (u + 1)) & 1ull));
-            const int hu = (int)((s.h >> u) & 1ull), hv = (int)((s.h >> (u + 1)) & 1ull);
-            s.Q += 4 * (hu & hv);
-            if (lane_in((cv & allmask(hu)) ^ (cu & allmask(hv)) ^ (cu & cv))) s.d = (s.d + 4) & 7;
-            if (lane_in(cu)) s.J ^= cv;
-            if (lane_in(cv)) s.J ^= cu;
-        }
-        const u64 even = 0x5555555555555555ull & lowmask(D.n & ~1);
-        s.G ^= (s.G & even) << 1;
-        s.h ^= (s.h & even) << 1;
+// The coordinates in which an |H^t> instance's terms are products
+// (to_dev on the host is the same change for the projector): with
+// u = x_2q and s = x_2q + x_2q+1 in columns 2q and 2q+1, the term with
+// coupling is the sum over u and s after a controlled sign on (x_2q, x_2q+1),
+// and |00> + |11> is s = 0 with the sum over u signed (-1)^u (the same
+// controlled sign undone).
+DEV void to_products(AState &s, int n) {
+    for (int u = 0; u + 1 < n; u += 2) {
+        const u64 cu = ballot(lane_in(s.act) && ((s.G >> u) & 1ull));
+        const u64 cv = ballot(lane_in(s.act) && ((s.G >> (u + 1)) & 1ull));
+        const int hu = (int)((s.h >> u) & 1ull), hv = (int)((s.h >> (u + 1)) & 1ull);
+        s.Q = (s.Q + 4 * (hu & hv)) & 7;
+        if (lane_in((cv & allmask(hu)) ^ (cu & allmask(hv)) ^ (cu & cv))) s.d = (s.d + 4) & 7;
+        if (lane_in(cu)) s.J ^= cv;
+        if (lane_in(cv)) s.J ^= cu;
     }
+    const u64 even = 0x5555555555555555ull & lowmask(n & ~1);
+    s.G ^= (s.G & even) << 1;
+    s.h ^= (s.h & even) << 1;
+}
+
+// Reduced row echelon basis of the active rows 0 .. k - 1 (basis changes of
+// the form, so the state is unchanged), the rows at their pivot lanes.
+DEV void to_rref(AState &s, int k) {
+    const int x = lane_id();
     int src = x;
     u64 Pm = 0;
-    for (int a = 0; a < r.k; a++) {
+    for (int a = 0; a < k; a++) {
         const u64 Ga = rl64(s.G, a);
         const int pc = __ffsll((long long)Ga) - 1;
         if (x == pc) src = a;
         Pm |= bit(pc);
-        const u64 Sp = ballot(x < r.k && x != a && ((s.G >> pc) & 1ull));
+        const u64 Sp = ballot(x < k && x != a && ((s.G >> pc) & 1ull));
         int dummy;
-        as_basis_change<false>(s, a, Sp, true, &dummy);
+        if (Sp) as_basis_change<false>(s, a, Sp, true, &dummy);
     }
-    // rows to their pivot lanes, then J's columns: lane p's row is row src of
-    // the state, and bit p of a row is its bit src (a transpose away from
-    // the same move)
+    // lane p's row is row src of the state, and bit p of a row is its bit src
+    // (a transpose away from the same move)
     const bool piv = lane_in(Pm);
-    AState o;
-    o.G = shfl64(s.G, src);
-    u64 J = shfl64(s.J & lowmask(r.k), src);
-    if (!piv) {
-        o.G = 0;
-        J = 0;
-    }
-    o.d = __shfl(s.d, src, 64);
-    if (!piv) o.d = 0;
-    J = transpose64(J);
-    J = shfl64(J, src);
-    o.J = piv ? J : 0ull;
-    o.act = Pm;
-    o.h = s.h;
-    o.Q = s.Q;
-    store_form(o, D, sexp, rec);
+    const u64 G = shfl64(s.G, src);
+    const int d = __shfl(s.d, src, 64);
+    u64 J = shfl64(s.J & lowmask(k), src);
+    if (!piv) J = 0;
+    J = shfl64(transpose64(J), src);
+    s.G = piv ? G : 0ull;
+    s.J = piv ? J : 0ull;
+    s.d = piv ? d & 6 : 0;
+    s.act = Pm;
 }
 
 }  // namespace
@@ -485,10 +460,14 @@ k_random_states(int n, const uint64_t *__restrict__ thr, uint64_t seed, long lon
 // Returns the number of 2^-1/2 factors, -1 if the projection vanishes.
 DEV int rs_project_rref(AState &s, const DevProjector &P) {
     const int x = lane_id();
+    // generator x in lane x: one load for all instead of one per step
+    const u64 pz = P.zs[x], px = P.xs[x];
+    const int pm = P.phase[x];
+    const int ng = P.nstabs;
     int sexp = 0;
-    for (int g = 0; g < P.nstabs; g++) {
-        const int m = P.phase[g] & 3;
-        const u64 zeta = P.zs[g], xi = P.xs[g];
+    for (int g = 0; g < ng; g++) {
+        const int m = rl32(pm, g) & 3;
+        const u64 zeta = rl64(pz, g), xi = rl64(px, g);
         const u64 c = xi & s.act;
         const bool inA = lane_in(s.act), inC = lane_in(c);
         const u64 rho = xi ^ wave_xor(inC ? s.G : 0ull);
@@ -538,7 +517,9 @@ DEV int rs_project_rref(AState &s, const DevProjector &P) {
 // mode 0: theta_s = random stabilizer state s = first + local index of the
 //         instance's Philox stream (seed)
 // mode 1: phi_i = prepH(i) (exact) or prepL(i) (|L>), i = local index
-// then Pi (innerprod.c:95-116 / :218-241) and the elimination-ready record.
+// then Pi (innerprod.c:95-116 / :218-241), in reduced row echelon form, and
+// the record.  |H^t> instances are taken to the coordinates of to_products
+// first, their projector with them.
 // The instance that holds global index key: the largest i < n with
 // off[i] <= key, for nondecreasing off with off[0] <= key.  The whole wave
 // searches: each round lane x reads off[lo + x*step] and the ballot's highest
@@ -570,8 +551,9 @@ k_records(int mode, int ninst, const long long *__restrict__ rec_off, const Inst
     const long long local = g - rec_off[in];
     const int n = D.n;
     uint64_t *rec = recs + (size_t)REC_WORDS * (size_t)g;
-    RState s;
+    AState a;
     if (mode == 0) {
+        RState s;
         if (!rs_random_state(s, n, thr_table + 65 * n, D.seed, (uint64_t)(D.first + local))) {
             if (lane_id() == 0) {
                 atomicOr(err, 1);
@@ -580,33 +562,27 @@ k_records(int mode, int ninst, const long long *__restrict__ rec_off, const Inst
             Rec::store_vanished(rec, n);
             return;
         }
-    } else if (D.exact) {
-        rs_prepH(s, (u64)local, n);
+        to_astate(s, a);
+        if (D.exact) to_products(a, n);
+        to_rref(a, s.k);
     } else {
-        // |L> records directly in reduced row echelon form
-        u64 xv = 0;
-        for (int j = 0; j < D.k; j++)
-            if (((u64)local >> j) & 1ull) xv ^= D.L[j];
-        AState a;
+        // the decomposition state, a product of |0>, |+> and (|H^t>) |->
+        const int x = lane_id();
+        const u64 row = x < D.k ? D.col[x] : 0ull, sgn = x < D.k && D.exact ? D.sgn[x] : 0ull;
+        const bool on = x < D.k && ((local >> x) & 1);
+        const u64 xv = (D.exact ? lowmask(n) : 0ull) ^ wave_xor(on ? row : 0ull);
+        const u64 neg = D.exact ? wave_xor(on ? sgn : 0ull) : 0ull;
         a.act = xv & lowmask(n);
-        a.G = lane_in(a.act) ? bit(lane_id()) : 0ull;
+        a.G = lane_in(a.act) ? bit(x) : 0ull;
         a.J = 0;
-        a.d = 0;
+        a.d = lane_in(a.act & neg) ? 4 : 0;
         a.h = 0;
         a.Q = 0;
-        const int se = rs_project_rref(a, projs[in]);
-        if (lane_id() == 0) sexp_out[g] = se;
-        if (se < 0) Rec::store_vanished(rec, n);
-        else store_form(a, D, se, rec);
-        return;
     }
-    const int se = rs_project(s, projs[in]);
+    const int se = rs_project_rref(a, projs[in]);
     if (lane_id() == 0) sexp_out[g] = se;
-    if (se < 0) {
-        Rec::store_vanished(rec, n);
-        return;
-    }
-    to_record(s, D, se, rec);
+    if (se < 0) Rec::store_vanished(rec, n);
+    else store_form(a, D, se, rec);
 }
 
 #include "cse_sweep.h"

@@ -193,12 +193,7 @@ template <int NH, bool HT, int MODE> DEV void sweep_body(const SweepArgs &A) {
         __syncthreads();
     };
 
-    while (true) {
-        __syncthreads();
-        if (tid == 0) s_item = (long long)atomicAdd(A.queue, 1ull);
-        __syncthreads();
-        const long long item = (long long)uniform64((u64)s_item);
-        if (item >= A.nitems) break;
+    auto run_item = [&](long long item) {
         const int inst = A.ninst > 1 ? uni(find_instance(A.item_off, A.ninst, item)) : 0;
         if (inst != cur || (MODE == 1 && pend >= A.flush_terms)) {
             if (cur >= 0) flush();
@@ -223,7 +218,13 @@ template <int NH, bool HT, int MODE> DEV void sweep_body(const SweepArgs &A) {
         const u64 w0 = rec[0];
         const bool valid = live && !((w0 >> 40) & 1);
         const int sexp = (int)((w0 >> 24) & 0xffff);
-        if (!ballot(valid) && !A.terms) continue;
+        if (!ballot(valid) && !A.terms) return;
+
+        // index bit b's toggles and index in lane b (read by readlane, so
+        // only where all lanes are active)
+        const u64 w_lp = x < TREE_MAXLOG ? A.inst[inst].LP[x] : 0ull;
+        const u64 w_lt = HT && x < TREE_MAXLOG ? A.inst[inst].LT[x] : 0ull;
+        const int w_jm = x < TREE_MAXLOG ? (int)A.inst[inst].jmap[x] : 0;
 
         tree::Form<NH> f;
         {
@@ -232,8 +233,8 @@ template <int NH, bool HT, int MODE> DEV void sweep_body(const SweepArgs &A) {
             u64 T = 0;
             for (int b = G; b < k; b++) {
                 const u64 on = 0ull - (u64)((jh >> (b - G)) & 1);
-                xj ^= D->LP[b] & on;
-                if (HT && D->exact) T ^= D->L[b] & on;
+                xj ^= rl64(w_lp, b) & on;
+                if (HT) T ^= rl64(w_lt, b) & on;
             }
             const u64 a = xj ^ F;
             f.A = (unsigned)a;
@@ -265,9 +266,8 @@ template <int NH, bool HT, int MODE> DEV void sweep_body(const SweepArgs &A) {
         // by index bit g (in lane g): the slots it toggles, their signs, the
         // index j; by level: slots and place of the saved form
         const int gl = x < TREE_MAXG ? x : TREE_MAXG;
-        const int v_lp = x < TREE_MAXG ? (int)(unsigned)D->LP[x] : 0;
-        const int v_lt = HT && x < TREE_MAXG && D->exact ? (int)(unsigned)D->L[x] : 0;
-        const int v_lev = (int)D->ub[gl] | (int)D->soff[gl] << 8;
+        const int v_lp = (int)(unsigned)w_lp, v_lt = (int)(unsigned)w_lt;
+        const int v_lev = (int)A.inst[inst].ub[gl] | (int)A.inst[inst].soff[gl] << 8;
         const int nlds = D->nlds, leaf = D->leaf;
         // the term within the lane (Gray code of t - 1), and what it toggles
         const unsigned T0 = f.T;
@@ -277,10 +277,10 @@ template <int NH, bool HT, int MODE> DEV void sweep_body(const SweepArgs &A) {
         unsigned jhi = 0, ri = 0;
         if (A.terms)
             for (int b = G; b < k; b++)
-                if ((jh >> (b - G)) & 1) jhi ^= D->jmap[b];
+                jhi ^= (unsigned)__builtin_amdgcn_readlane(w_jm, b) & (0u - (unsigned)((jh >> (b - G)) & 1));
         if (MODE == 1) {
             for (int b = 0; b < k; b++)
-                if ((r >> b) & 1) ri ^= D->jmap[b];
+                ri ^= (unsigned)__builtin_amdgcn_readlane(w_jm, b) & (0u - (unsigned)((r >> b) & 1));
             // the record's pairs i <= j in the reference's order, counted by
             // the one lane that holds its diagonal
             if (valid && rl >= 0) ips += (unsigned long long)(D->chi - (long long)ri);
@@ -411,6 +411,19 @@ template <int NH, bool HT, int MODE> DEV void sweep_body(const SweepArgs &A) {
                 }
             }
         }
+    };
+
+    // The first item is the block's own; the others come from the queue, each
+    // claimed when the one before is done (claimed ahead, a launch of a few
+    // items a block loses 10% to its slower blocks).
+    const bool more = A.nitems > (long long)gridDim.x;
+    for (long long item = (long long)blockIdx.x; item < A.nitems;) {
+        run_item(item);
+        if (!more) break;
+        __syncthreads();  // the item's sums are complete, s_item has been read
+        if (tid == 0) s_item = (long long)(gridDim.x + atomicAdd(A.queue, 1ull));
+        __syncthreads();
+        item = (long long)uniform64((u64)s_item);
     }
     if (cur >= 0) flush();
 }
