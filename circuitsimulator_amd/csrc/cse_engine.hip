@@ -31,26 +31,10 @@ struct HostBuf {
     size_t cap = 0;
 };
 
-// What a captured batch depends on besides the plan's and the results'
-// contents: its sizes, kernels and grids (all functions of these) and every
-// buffer address its nodes hold.  A call whose key matches replays the graph.
-struct GraphKey {
-    int mode, ninst, kernel;
-    long long nrec, nitems, stack_words;
-    size_t plan_bytes, out_bytes;
-    const void *ptr[9];
-};
-
-struct GraphEntry {
-    GraphKey key;
-    hipGraphExec_t exec = nullptr;
-    unsigned long long used = 0;
-};
-
 struct cse_ctx {
     int device = 0;
     hipStream_t stream = nullptr;
-    hipEvent_t e0 = nullptr, e1 = nullptr, e2 = nullptr;
+    hipEvent_t e0 = nullptr, e1 = nullptr;  // cse_inner_products' times
     int cus = 0;
     char name[128] = {0};
     char err[512] = {0};
@@ -70,8 +54,17 @@ struct cse_ctx {
     unsigned long long *d_hist = nullptr, *d_ips = nullptr;
     int32_t *d_sexp = nullptr;
     int *d_err = nullptr;
+    unsigned long long *d_clock = nullptr;
     HostBuf hstage;  // results coming back (per-sample sums, histograms)
     HostBuf hup;     // the plan going up
+    // the number of the last finished call whose results came back in one
+    // block, written by the device after them (pinned), and that of the last
+    // one started
+    HostBuf hdone;
+    uint32_t calls = 0;
+    double ms_per_tick = 1e-5;  // of the device's constant-rate clock
+    // the bound host stages are pinned: kernels read and write them
+    bool b_pinned = false;
     // the memory the current batched call works in: the buffers above, or
     // the static scratch array (cse_exact_projector_noalloc)
     char *b_plan = nullptr, *b_out = nullptr, *b_hup = nullptr, *b_hstage = nullptr;
@@ -79,10 +72,6 @@ struct cse_ctx {
     uint32_t *b_stack = nullptr;
     unsigned long long *b_queue = nullptr;
     int32_t *b_sexp1 = nullptr, *b_terms = nullptr;
-    // batched calls replayed from captured HIP graphs (cse_set_graphs)
-    bool use_graphs = false;
-    std::vector<GraphEntry> graphs;
-    unsigned long long graph_clock = 0;
     // this device's copy of the static scratch array (nullptr if its address
     // could not be obtained; scratch_err says why)
     char *scratch = nullptr;
@@ -105,7 +94,7 @@ struct cse_ctx {
 constexpr int kStaticMaxLogChi = 13;
 constexpr long long kStaticMaxChi = 1ll << kStaticMaxLogChi;
 constexpr size_t kStaticPlanBytes = 4096;  // one instance: 3,328 B
-constexpr size_t kStaticOutBytes = 8448;   // one instance's results block: 8,288 B
+constexpr size_t kStaticOutBytes = 8448;   // one instance's results block: 8,320 B
 constexpr size_t kScratchQueue = 0;
 constexpr size_t kScratchPlan = 256;
 constexpr size_t kScratchOut = kScratchPlan + kStaticPlanBytes;
@@ -189,24 +178,6 @@ int zero64(cse_ctx *ctx, void *p, long long words) {
     int blocks = (int)((words + 255) / 256);
     if (blocks > 4096) blocks = 4096;
     hipLaunchKernelGGL(k_zero64, dim3(blocks), dim3(256), 0, ctx->stream, (unsigned long long *)p, words);
-    HIPCHK(hipGetLastError());
-    return CSE_OK;
-}
-
-// buffers a batch clears before its launches, in one k_zero_list launch
-void zl_add(ZeroList &zl, void *p, long long words) {
-    if (words <= 0) return;
-    zl.p[zl.count] = (unsigned long long *)p;
-    zl.n[zl.count] = words;
-    zl.count++;
-}
-
-int zero_list(cse_ctx *ctx, const ZeroList &zl) {
-    long long most = 0;
-    for (int b = 0; b < zl.count; b++) most = std::max(most, zl.n[b]);
-    if (most == 0) return CSE_OK;
-    const int blocks = (int)std::min<long long>(4096, (most + 255) / 256);
-    hipLaunchKernelGGL(k_zero_list, dim3(blocks), dim3(256), 0, ctx->stream, zl);
     HIPCHK(hipGetLastError());
     return CSE_OK;
 }
@@ -335,9 +306,9 @@ size_t plan_layout(const Plan &pl, size_t off[4], size_t sz[4]) {
 }
 
 // The plan is written into the bound host stage in its device layout, and
-// the device pointers into the bound plan are set; copy_plan then moves it
-// in one transfer.  Every call synchronizes its stream before returning, so
-// the stage is free again at the next call.
+// the device pointers into the bound plan are set; prep_batch then moves it
+// in one launch.  Every call has its results before it returns, so the stage
+// is free again at the next call.
 size_t stage_plan(cse_ctx *ctx, const Plan &pl) {
     size_t off[4], sz[4];
     const size_t total = plan_layout(pl, off, sz);
@@ -352,11 +323,6 @@ size_t stage_plan(cse_ctx *ctx, const Plan &pl) {
     return total;
 }
 
-int copy_plan(cse_ctx *ctx, size_t bytes) {
-    HIPCHK(hipMemcpyAsync(ctx->b_plan, ctx->b_hup, bytes, hipMemcpyHostToDevice, ctx->stream));
-    return CSE_OK;
-}
-
 int run_records(cse_ctx *ctx, const Plan &pl, int mode) {
     const int ninst = pl.ninst;
     const long long waves = pl.nrec;
@@ -365,7 +331,7 @@ int run_records(cse_ctx *ctx, const Plan &pl, int mode) {
         hipLaunchKernelGGL(k_records, dim3((unsigned)blocks), dim3(256), 0, ctx->stream, mode, ninst,
                            ctx->d_recoff, ctx->d_inst, ctx->d_projs,
                            mode == 0 ? dp<uint64_t>(ctx->thr) : nullptr, pl.nrec, ctx->b_recs, ctx->d_sexp,
-                           ctx->d_err);
+                           ctx->d_err, ctx->d_clock);
         HIPCHK(hipGetLastError());
     }
     return CSE_OK;
@@ -375,9 +341,9 @@ int run_records(cse_ctx *ctx, const Plan &pl, int mode) {
 // pinned stage.  Sampled mode (0): per-sample Z[omega] sums (32 B), Kahan
 // pairs (16 B) and projection exponents (4 B), then per-instance counts and
 // the error flag.  Exact mode (1): per-instance histograms, Kahan pairs and
-// counts, then the error flag.
+// counts, then the error flag; both end with the clock readings.
 struct OutLayout {
-    size_t zsum, kahan, sexp, hist, ips, err, total;
+    size_t zsum, kahan, sexp, hist, ips, err, clock, total;
 };
 
 OutLayout out_layout(const Plan &pl, int mode) {
@@ -397,7 +363,8 @@ OutLayout out_layout(const Plan &pl, int mode) {
         o.ips = o.kahan + 16 * ni;
         o.err = o.ips + 8 * ni;
     }
-    o.total = o.err + 8;
+    o.clock = o.err + 8;  // three readings, see BatchTimes
+    o.total = (o.clock + 3 * 8 + 15) & ~(size_t)15;
     return o;
 }
 
@@ -443,6 +410,7 @@ int bind_ctx_mem(cse_ctx *ctx, const Plan &pl, int mode, bool want_terms) {
     int rc = ensure_host(ctx, ctx->hup, pbytes);
     if (!rc) rc = ensure_host(ctx, ctx->hstage, o.total);
     if (rc) return rc;
+    ctx->b_pinned = true;
     ctx->b_plan = (char *)ctx->plan.p;
     ctx->b_out = (char *)ctx->outb.p;
     ctx->b_recs = dp<uint64_t>(ctx->recs);
@@ -476,12 +444,17 @@ int bind_static_mem(cse_ctx *ctx, const Plan &pl, char *hup, char *hstage) {
     ctx->b_terms = nullptr;
     ctx->b_hup = hup;
     ctx->b_hstage = hstage;
+    ctx->b_pinned = false;
     return CSE_OK;
 }
 
-// One launch that clears the bound results block (every sum, count and flag;
-// the exponents are rewritten by the record launch) and the work queue.
-int prep_batch(cse_ctx *ctx, const Plan &pl, int mode) {
+// One launch that brings the staged plan to the device and clears the bound
+// results block (every sum, count and flag; the exponents are rewritten by
+// the record launch) and the work queue.  From pinned memory the kernel reads
+// the plan itself: a copy call of its own costs 6 us of host time and, before
+// kernels, a wait of the command processor (copy, three launches, copy and
+// three events took 46 us, the same four launches without them 19).
+int prep_batch(cse_ctx *ctx, const Plan &pl, int mode, size_t plan_bytes) {
     const OutLayout o = out_layout(pl, mode);
     char *b = ctx->b_out;
     ctx->out_bytes = o.total;
@@ -491,11 +464,21 @@ int prep_batch(cse_ctx *ctx, const Plan &pl, int mode) {
     ctx->d_hist = mode == 1 ? (unsigned long long *)(b + o.hist) : nullptr;
     ctx->d_ips = (unsigned long long *)(b + o.ips);
     ctx->d_err = (int *)(b + o.err);
-    ZeroList zl;
-    memset(&zl, 0, sizeof(zl));
-    zl_add(zl, b, (long long)(o.total / 8));
-    zl_add(zl, ctx->b_queue, 1);
-    return zero_list(ctx, zl);
+    ctx->d_clock = (unsigned long long *)(b + o.clock);
+    PrepArgs a;
+    a.src = (const uint4 *)ctx->b_hup;
+    a.dst = (uint4 *)ctx->b_plan;
+    a.ncopy = ctx->b_pinned ? (long long)(plan_bytes / 16) : 0;
+    a.zero = (uint4 *)b;
+    a.nzero = (long long)(o.total / 16);
+    a.queue = ctx->b_queue;
+    if (!ctx->b_pinned)
+        HIPCHK(hipMemcpyAsync(ctx->b_plan, ctx->b_hup, plan_bytes, hipMemcpyHostToDevice, ctx->stream));
+    const long long most = std::max(a.ncopy, a.nzero);
+    hipLaunchKernelGGL(k_prep, dim3((unsigned)std::min<long long>(4096, (most + 255) / 256)), dim3(256), 0,
+                       ctx->stream, a);
+    HIPCHK(hipGetLastError());
+    return CSE_OK;
 }
 
 int run_sweep(cse_ctx *ctx, const Plan &pl, int mode, bool want_terms) {
@@ -516,94 +499,71 @@ int run_sweep(cse_ctx *ctx, const Plan &pl, int mode, bool want_terms) {
     A.kahan = ctx->d_kahan;
     A.hist = ctx->d_hist;
     A.ips = ctx->d_ips;
+    A.clock = ctx->d_clock;
     const SweepKernel k = sweep_choice(pl, mode);
     hipLaunchKernelGGL(k.fn, dim3(sweep_grid(ctx, pl, k)), dim3(256), 0, ctx->stream, A);
     HIPCHK(hipGetLastError());
     return CSE_OK;
 }
 
-// The device work of a bound, staged batch in stream order: plan copy,
-// clear, records, sweep, results copy; with events between the launches
-// when timed.
-int enqueue_batch(cse_ctx *ctx, const Plan &pl, int mode, bool want_terms, size_t plan_bytes, bool timed) {
-    int rc = copy_plan(ctx, plan_bytes);
-    if (!rc) rc = prep_batch(ctx, pl, mode);
+// Results of at most this size come back in one block's stores, followed by
+// the call's number, which the host polls: 4 us less than a wait for the
+// stream.  Larger ones take a grid of blocks (faster than a copy call at 64 KB
+// to 1 MB: 14 to 32 us against 21 to 39).
+constexpr size_t kPollBytes = 16384;
+constexpr size_t kGridBytes = 64 << 20;
+
+// Runs a bound, staged batch, in stream order: plan and clear, records,
+// sweep, results (and, with terms, their copies to the caller, which `copy`
+// enqueues), and waits for it.
+template <class F> int run_batch(cse_ctx *ctx, const Plan &pl, int mode, bool want_terms, size_t plan_bytes, F &&copy) {
+    int rc = prep_batch(ctx, pl, mode, plan_bytes);
+    if (!rc) rc = run_records(ctx, pl, mode);
+    if (!rc) rc = run_sweep(ctx, pl, mode, want_terms);
     if (rc) return rc;
-    if (timed) HIPCHK(hipEventRecord(ctx->e0, ctx->stream));
-    rc = run_records(ctx, pl, mode);
-    if (rc) return rc;
-    if (timed) HIPCHK(hipEventRecord(ctx->e1, ctx->stream));
-    rc = run_sweep(ctx, pl, mode, want_terms);
-    if (rc) return rc;
-    if (timed) HIPCHK(hipEventRecord(ctx->e2, ctx->stream));
-    HIPCHK(hipMemcpyAsync(ctx->b_hstage, ctx->b_out, ctx->out_bytes, hipMemcpyDeviceToHost, ctx->stream));
+    const bool poll = ctx->b_pinned && ctx->out_bytes <= kPollBytes && !want_terms;
+    ResultArgs a;
+    a.src = (const uint4 *)ctx->b_out;
+    a.dst = (uint4 *)ctx->b_hstage;
+    a.n = (long long)(ctx->out_bytes / 16);
+    a.clock = ctx->d_clock + 2;
+    a.done = poll ? (uint32_t *)ctx->hdone.p : nullptr;
+    a.call = ++ctx->calls;
+    const bool dma = !ctx->b_pinned || ctx->out_bytes > kGridBytes;
+    if (dma) a.n = 0;
+    const long long blocks = poll ? 1 : std::min<long long>(1024, (a.n + 255) / 256);
+    hipLaunchKernelGGL(k_results, dim3((unsigned)std::max(1ll, blocks)), dim3(256), 0, ctx->stream, a);
+    HIPCHK(hipGetLastError());
+    if (dma)
+        HIPCHK(hipMemcpyAsync(ctx->b_hstage, ctx->b_out, ctx->out_bytes, hipMemcpyDeviceToHost, ctx->stream));
+    if (want_terms) {
+        rc = copy();
+        if (rc) return rc;
+    }
+    if (poll) {
+        // about a millisecond of polling, then the stream's own wait (long calls,
+        // and whatever goes wrong on the device)
+        const uint32_t *done = (const uint32_t *)ctx->hdone.p;
+        for (int i = 0; i < 20000; i++) {
+            if (__atomic_load_n(done, __ATOMIC_ACQUIRE) == a.call) return CSE_OK;
+            __builtin_ia32_pause();
+        }
+    }
+    HIPCHK(hipStreamSynchronize(ctx->stream));
     return CSE_OK;
 }
 
-constexpr size_t kMaxGraphs = 16;
-
-// Runs a bound, staged batch: eagerly, or -- when the context replays graphs
-// and the call writes no per-term output -- from the context's graph of the
-// same key, captured at the first call of that key.  *graphed tells which;
-// the caller synchronizes the stream.
-int run_batch(cse_ctx *ctx, const Plan &pl, int mode, bool want_terms, size_t plan_bytes, bool *graphed) {
-    *graphed = false;
-    if (!ctx->use_graphs || want_terms) return enqueue_batch(ctx, pl, mode, want_terms, plan_bytes, true);
-    GraphKey key;
-    memset(&key, 0, sizeof(key));
-    key.mode = mode;
-    key.ninst = pl.ninst;
-    key.kernel = sweep_choice(pl, mode).id;
-    key.nrec = pl.nrec;
-    key.nitems = pl.nitems;
-    key.stack_words = pl.stack_words;
-    key.plan_bytes = plan_bytes;
-    key.out_bytes = out_layout(pl, mode).total;
-    const void *ptr[9] = {ctx->b_plan, ctx->b_out, ctx->b_recs, ctx->b_queue, ctx->b_stack,
-                          ctx->b_sexp1, ctx->b_hup, ctx->b_hstage, mode == 0 ? ctx->thr.p : nullptr};
-    memcpy(key.ptr, ptr, sizeof(ptr));
-    GraphEntry *hit = nullptr;
-    for (GraphEntry &g : ctx->graphs)
-        if (memcmp(&g.key, &key, sizeof(key)) == 0) {
-            hit = &g;
-            break;
-        }
-    if (!hit) {
-        hipGraph_t graph = nullptr;
-        HIPCHK(hipStreamBeginCapture(ctx->stream, hipStreamCaptureModeThreadLocal));
-        const int rc = enqueue_batch(ctx, pl, mode, false, plan_bytes, false);
-        const hipError_t e = hipStreamEndCapture(ctx->stream, &graph);
-        if (rc || e != hipSuccess) {
-            if (graph) (void)hipGraphDestroy(graph);
-            (void)hipGetLastError();
-            return rc ? rc : fail(ctx, CSE_ERR_HIP, "hipStreamEndCapture: %s", hipGetErrorString(e));
-        }
-        hipGraphExec_t exec = nullptr;
-        const hipError_t ei = hipGraphInstantiate(&exec, graph, nullptr, nullptr, 0);
-        (void)hipGraphDestroy(graph);
-        if (ei != hipSuccess) {
-            (void)hipGetLastError();
-            return fail(ctx, CSE_ERR_HIP, "hipGraphInstantiate: %s", hipGetErrorString(ei));
-        }
-        if (ctx->graphs.size() >= kMaxGraphs) {
-            size_t old = 0;
-            for (size_t g = 1; g < ctx->graphs.size(); g++)
-                if (ctx->graphs[g].used < ctx->graphs[old].used) old = g;
-            (void)hipGraphExecDestroy(ctx->graphs[old].exec);
-            ctx->graphs.erase(ctx->graphs.begin() + (long)old);
-        }
-        GraphEntry ent;
-        ent.key = key;
-        ent.exec = exec;
-        ctx->graphs.push_back(ent);
-        hit = &ctx->graphs.back();
-    }
-    hit->used = ++ctx->graph_clock;
-    HIPCHK(hipEventRecord(ctx->e0, ctx->stream));
-    HIPCHK(hipGraphLaunch(hit->exec, ctx->stream));
-    HIPCHK(hipEventRecord(ctx->e2, ctx->stream));
-    *graphed = true;
-    return CSE_OK;
+// Device times of a finished batch from its clock readings: at the start of
+// the records, of the sweep, and of the results copy.
+struct BatchTimes {
+    double records, sweep;
+};
+BatchTimes batch_times(const cse_ctx *ctx, const OutLayout &o) {
+    const unsigned long long *c = (const unsigned long long *)(ctx->b_hstage + o.clock);
+    BatchTimes t;
+    t.records = (double)(long long)(c[1] - c[0]) * ctx->ms_per_tick;
+    t.sweep = (double)(long long)(c[2] - c[1]) * ctx->ms_per_tick;
+    return t;
 }
 
 // Cost model of a lane's tree, in VALU instructions: a step of slot c takes
@@ -742,13 +702,18 @@ int init_ctx(cse_ctx *ctx, int device) {
     HIPCHK(hipStreamCreateWithFlags(&ctx->stream, hipStreamNonBlocking));
     HIPCHK(hipEventCreate(&ctx->e0));
     HIPCHK(hipEventCreate(&ctx->e1));
-    HIPCHK(hipEventCreate(&ctx->e2));
     hipDeviceProp_t prop;
     HIPCHK(hipGetDeviceProperties(&prop, device));
     ctx->cus = prop.multiProcessorCount;
     snprintf(ctx->name, sizeof(ctx->name), "%s (%s)", prop.name, prop.gcnArchName);
     if (strncmp(prop.gcnArchName, "gfx950", 6) != 0)
         return fail(ctx, CSE_ERR_HIP, "device %d is %s; this engine is built for gfx950", device, prop.gcnArchName);
+    int khz = 0;
+    if (hipDeviceGetAttribute(&khz, hipDeviceAttributeWallClockRate, device) == hipSuccess && khz > 0)
+        ctx->ms_per_tick = 1.0 / khz;
+    const int rc_done = ensure_host(ctx, ctx->hdone, 64);
+    if (rc_done) return rc_done;
+    memset(ctx->hdone.p, 0, 64);
     // the sweep's leaf tables, kept for the context's life
     const int plain = 1 << tree::LeafBits<false>::value, sign = 1 << tree::LeafBits<true>::value;
     ENSURE(leaf, (size_t)(plain + sign));
@@ -825,18 +790,15 @@ void cse_destroy(cse_ctx *ctx) {
     if (!ctx) return;
     (void)hipSetDevice(ctx->device);
     if (ctx->stream) (void)hipStreamSynchronize(ctx->stream);
-    for (GraphEntry &g : ctx->graphs)
-        if (g.exec) (void)hipGraphExecDestroy(g.exec);
-    ctx->graphs.clear();
     DevBuf *bufs[] = {&ctx->s1, &ctx->s2, &ctx->out, &ctx->recs, &ctx->terms, &ctx->queue, &ctx->thr,
                       &ctx->sexp, &ctx->L, &ctx->idx, &ctx->errflag, &ctx->lsh, &ctx->plan, &ctx->outb, &ctx->stack, &ctx->leaf};
     for (DevBuf *b : bufs)
         if (b->p) (void)hipFree(b->p);
     if (ctx->hstage.p) (void)hipHostFree(ctx->hstage.p);
     if (ctx->hup.p) (void)hipHostFree(ctx->hup.p);
+    if (ctx->hdone.p) (void)hipHostFree(ctx->hdone.p);
     if (ctx->e0) (void)hipEventDestroy(ctx->e0);
     if (ctx->e1) (void)hipEventDestroy(ctx->e1);
-    if (ctx->e2) (void)hipEventDestroy(ctx->e2);
     if (ctx->stream) (void)hipStreamDestroy(ctx->stream);
     delete ctx;
 }
@@ -855,9 +817,8 @@ int cse_set_sweep_kernel(cse_ctx *ctx, int mode, int kernel) {
 }
 
 int cse_set_graphs(cse_ctx *ctx, int enable) {
-    if (!ctx) return CSE_ERR_ARG;
-    ctx->use_graphs = enable != 0;
-    return CSE_OK;
+    (void)enable;
+    return ctx ? CSE_OK : CSE_ERR_ARG;
 }
 
 int cse_device_info(cse_ctx *ctx, int *cus, char *name, int name_len) {
@@ -1026,8 +987,14 @@ static int sampled_batch(cse_ctx *ctx, const cse_sampled_instance *in, int ninst
     int rc = ensure_thresholds(ctx);
     if (!rc) rc = bind_ctx_mem(ctx, pl, 0, want_terms);
     if (rc) return rc;
-    bool graphed = false;
-    rc = run_batch(ctx, pl, 0, want_terms, stage_plan(ctx, pl), &graphed);
+    rc = run_batch(ctx, pl, 0, want_terms, stage_plan(ctx, pl), [&]() -> int {
+        for (int i = 0; i < ninst; i++)
+            if (res[i].terms)
+                HIPCHK(hipMemcpyAsync(res[i].terms, ctx->b_terms + pl.inst[i].term_off,
+                                      4 * (size_t)(in[i].count * pl.inst[i].chi), hipMemcpyDeviceToHost,
+                                      ctx->stream));
+        return CSE_OK;
+    });
     if (rc) return rc;
 
     // the results block came back in one copy, into a pinned stage of the
@@ -1039,16 +1006,10 @@ static int sampled_batch(cse_ctx *ctx, const cse_sampled_instance *in, int ninst
     const int32_t *se = (const int32_t *)(hs + o.sexp);
     const unsigned long long *nips = (const unsigned long long *)(hs + o.ips);
     int *errp = (int *)(hs + o.err);
-    for (int i = 0; i < ninst; i++)
-        if (res[i].terms)
-            HIPCHK(hipMemcpyAsync(res[i].terms, ctx->b_terms + pl.inst[i].term_off,
-                                  4 * (size_t)(in[i].count * pl.inst[i].chi), hipMemcpyDeviceToHost, ctx->stream));
-    HIPCHK(hipStreamSynchronize(ctx->stream));
     const int errv = *errp;
     if (errv & 1) return fail(ctx, CSE_ERR_RNG, "random state draw exceeded its shrink cap");
-    // a replayed graph is timed as a whole (records and sweep together)
-    const double pms = graphed ? 0.0 : elapsed(ctx->e0, ctx->e1);
-    const double kms = graphed ? elapsed(ctx->e0, ctx->e2) : elapsed(ctx->e1, ctx->e2);
+    const BatchTimes bt = batch_times(ctx, o);
+    const double pms = bt.records, kms = bt.sweep;
     if (kernel_ms) *kernel_ms = kms;
     const unsigned hw = std::thread::hardware_concurrency();
     const int nthr = (ninst >= 8 && pl.nrec >= (1 << 16)) ? (int)std::min(8u, hw ? hw : 1u) : 1;
@@ -1150,12 +1111,10 @@ static int exact_batch(cse_ctx *ctx, const cse_instance *in, int ninst, int chun
     if (terms_out && pl.nterms > (1ll << 31)) return fail(ctx, CSE_ERR_ARG, "per-term output too large");
     int rc = use_static ? bind_static_mem(ctx, pl, hup, hstage) : bind_ctx_mem(ctx, pl, 1, terms_out != nullptr);
     if (rc) return rc;
-    // the static path never captures (graph memory nodes would be
-    // allocations of their own)
-    bool graphed = false;
-    const size_t plan_bytes = stage_plan(ctx, pl);
-    rc = use_static ? enqueue_batch(ctx, pl, 1, false, plan_bytes, true)
-                    : run_batch(ctx, pl, 1, terms_out != nullptr, plan_bytes, &graphed);
+    rc = run_batch(ctx, pl, 1, terms_out != nullptr, stage_plan(ctx, pl), [&]() -> int {
+        HIPCHK(hipMemcpyAsync(terms_out, ctx->b_terms, 4 * (size_t)pl.nterms, hipMemcpyDeviceToHost, ctx->stream));
+        return CSE_OK;
+    });
     if (rc) return rc;
     // the results block came back in one copy, into a pinned stage of the
     // same layout: histograms (HIST_STRIDE words per instance), the Kahan
@@ -1165,11 +1124,8 @@ static int exact_batch(cse_ctx *ctx, const cse_instance *in, int ninst, int chun
     const unsigned long long *hist = (const unsigned long long *)(hs + o.hist);
     const double *kz = (const double *)(hs + o.kahan);
     const unsigned long long *nips = (const unsigned long long *)(hs + o.ips);
-    if (terms_out)
-        HIPCHK(hipMemcpyAsync(terms_out, ctx->b_terms, 4 * (size_t)pl.nterms, hipMemcpyDeviceToHost, ctx->stream));
-    HIPCHK(hipStreamSynchronize(ctx->stream));
-    const double tms = elapsed(ctx->e0, ctx->e2);
-    const double kms = graphed ? tms : elapsed(ctx->e1, ctx->e2);
+    const BatchTimes bt = batch_times(ctx, o);
+    const double kms = bt.sweep, tms = bt.records + bt.sweep;
     if (kernel_ms) *kernel_ms = kms;
     // each instance's exact value from its histogram (a few microseconds
     // each): split over host threads for large batches

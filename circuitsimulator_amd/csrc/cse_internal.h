@@ -96,6 +96,7 @@ struct SweepArgs {
     double *kahan;            // mode 0: 2 per record; mode 1: 2 per instance
     unsigned long long *hist; // HIST_STRIDE per instance
     unsigned long long *ips;  // per instance
+    unsigned long long *clock; // readings: records, sweep, results start
 };
 
 #ifdef __HIPCC__

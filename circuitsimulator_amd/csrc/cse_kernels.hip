@@ -12,7 +12,8 @@
 //                    exactly (int64) plus a Kahan-FP32 shadow (cse_sweep.h);
 //                    s / e: sampled, exact mode; h: with |H^t> instances;
 //                    32, 48, 64: widest state
-//   k_zero_list      clears a call's result and queue blocks in one launch
+//   k_prep, k_results  a call's plan to the device and its results cleared;
+//                    the results to pinned host memory
 //   k_lspace_hist    histogram of |x| over the row space of L (decompose's
 //                    fidelity)
 #include "cse_device.h"
@@ -543,7 +544,9 @@ DEV int find_instance(const long long *__restrict__ off, int n, long long key) {
 extern "C" __global__ void __launch_bounds__(256)
 k_records(int mode, int ninst, const long long *__restrict__ rec_off, const InstDesc *__restrict__ inst,
           const DevProjector *__restrict__ projs, const uint64_t *__restrict__ thr_table, long long nrec,
-          uint64_t *__restrict__ recs, int32_t *__restrict__ sexp_out, int *__restrict__ err) {
+          uint64_t *__restrict__ recs, int32_t *__restrict__ sexp_out, int *__restrict__ err,
+          unsigned long long *__restrict__ clock) {
+    if (blockIdx.x == 0 && threadIdx.x == 0) *clock = wall_clock64();
     const long long g = (long long)blockIdx.x * (blockDim.x >> 6) + (threadIdx.x >> 6);
     if (g >= nrec) return;
     const int in = ninst > 1 ? find_instance(rec_off, ninst, g) : 0;
@@ -624,17 +627,57 @@ extern "C" __global__ void k_zero64(unsigned long long *p, long long n) {
     for (; i < n; i += (long long)gridDim.x * blockDim.x) p[i] = 0ull;
 }
 
-// The per-call sums, counters and flags of a batch (up to 8 buffers of
-// 64-bit words) cleared in one launch, grid-stride over each buffer.
-struct ZeroList {
-    unsigned long long *p[8];
-    long long n[8];
-    int count;
+// A batch's plan copied from pinned host memory, its results block and work
+// queue cleared, grid-stride.
+struct PrepArgs {
+    const uint4 *src;
+    uint4 *dst, *zero;
+    long long ncopy, nzero;  // 16-byte words
+    unsigned long long *queue;
 };
-
-extern "C" __global__ void k_zero_list(ZeroList L) {
+extern "C" __global__ void k_prep(PrepArgs a) {
     const long long stride = (long long)gridDim.x * blockDim.x;
     const long long i0 = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-    for (int b = 0; b < L.count; b++)
-        for (long long i = i0; i < L.n[b]; i += stride) L.p[b][i] = 0ull;
+    for (long long i = i0; i < a.ncopy; i += stride) a.dst[i] = a.src[i];
+    for (long long i = i0; i < a.nzero; i += stride) a.zero[i] = make_uint4(0, 0, 0, 0);
+    if (i0 == 0) *a.queue = 0;
+}
+
+// A batch's results block to pinned host memory, grid-stride; with `done`
+// (one block), the call's number after them.
+struct ResultArgs {
+    const uint4 *src;
+    uint4 *dst;
+    long long n;             // 16-byte words
+    unsigned long long *clock;
+    uint32_t *done;
+    uint32_t call;
+};
+extern "C" __global__ void k_results(ResultArgs a) {
+    const long long stride = (long long)gridDim.x * blockDim.x;
+    const long long i0 = (long long)blockIdx.x * blockDim.x + threadIdx.x;
+    // the clock is part of the block's last words: its 16 bytes are put
+    // together by the thread that copies them
+    const unsigned long long now = wall_clock64();
+    const long long off = (const char *)a.clock - (const char *)a.src, at = off >> 4;
+    const int half = (int)(off >> 3) & 1;
+    if (i0 == 0 && a.n == 0) *a.clock = now;
+    for (long long i = i0; i < a.n; i += stride) {
+        uint4 v = a.src[i];
+        if (i == at) {
+            if (half) {
+                v.z = (unsigned)now;
+                v.w = (unsigned)(now >> 32);
+            } else {
+                v.x = (unsigned)now;
+                v.y = (unsigned)(now >> 32);
+            }
+        }
+        a.dst[i] = v;
+    }
+    if (a.done) {
+        __threadfence_system();
+        __syncthreads();
+        if (threadIdx.x == 0) __hip_atomic_store(a.done, a.call, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+    }
 }

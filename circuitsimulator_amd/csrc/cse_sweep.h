@@ -155,6 +155,7 @@ template <int NH, bool HT, int MODE> DEV void sweep_body(const SweepArgs &A) {
     // (at most 2^G 2^32 <= 2^44, exact), Kahan FP32 pair
     double c0 = 0.0, c1 = 0.0, c2 = 0.0, c3 = 0.0;
     float sr = 0.f, cr = 0.f, si = 0.f, ci = 0.f;
+    if (blockIdx.x == 0 && tid == 0) A.clock[1] = wall_clock64();
     s_tab.fill(tid);
     for (int b = tid; b < 1 << tree::LeafBits<HT>::value; b += 256) s_leaf[b] = A.leaf[b];
     if (MODE == 1)

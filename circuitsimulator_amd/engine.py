@@ -178,8 +178,8 @@ class Engine:
             raise EngineError(f"engine error {rc}: {self._L.cse_error(self.h).decode()}")
 
     def set_graphs(self, enable=True):
-        """replay batched calls of a repeated shape from captured HIP graphs
-        (cse_set_graphs)"""
+        """accepted and without effect (cse_set_graphs): a call's four launches
+        are faster than a captured graph of them"""
         self._check(self._L.cse_set_graphs(self.h, 1 if enable else 0))
 
     def set_sweep_kernel(self, kernel, mode=0):
@@ -375,9 +375,6 @@ def shared_engine(device=0):
     e = _shared.get(key)
     if e is None or not e.h:
         e = _shared[key] = Engine(device)
-        # its batches repeat their shape round after round: replay them from
-        # captured graphs unless CSE_GRAPHS=0
-        e.set_graphs(os.environ.get("CSE_GRAPHS", "1") != "0")
     return e
 
 

@@ -64,16 +64,11 @@ const char *cse_error(const cse_ctx *ctx);
 int cse_device_info(cse_ctx *ctx, int *cus, char *name, int name_len);
 
 /*
- * enable != 0: the context's batched calls (cse_exact_projector,
- * cse_sampled_projector, cse_batch_exact, cse_batch_sampled and the
- * projector norms) replay HIP graphs: the first call of a given shape
- * (instance count, records, work items, buffers) captures its plan copy,
- * clearing launch, record launch, sweep and results copy, and later calls
- * of that shape launch the captured graph after writing their plan into
- * the same pinned stage.  Results are identical; calls that return
- * per-term output always run eagerly.  No reference counterpart: the
- * reference starts one backend process per probability() call
- * (probability.py:237-244).  Default off.
+ * Accepted and without effect: batched calls used to be replayed from captured
+ * HIP graphs when enabled.  A call is now four kernel launches (plan, records,
+ * sweep, results), which take 19 us of host and queue time where a graph of
+ * them takes 34.  No reference counterpart: the reference starts one backend
+ * process per probability() call (probability.py:237-244).
  */
 int cse_set_graphs(cse_ctx *ctx, int enable);
 
