@@ -198,10 +198,7 @@ int ensure_thresholds(cse_ctx *ctx) {
 // column 2q+1, after a controlled sign on each pair).  i^m Z(z) X(x) picks up
 // the sign of x_u x_v, z_u ^= x_v and z_v ^= x_u from the controlled sign;
 // then z_u ^= z_v and x_s = x_u + x_v.
-DevProjector to_dev(const cse_projector *P, bool products = false) {
-    DevProjector d;
-    memset(&d, 0, sizeof(d));
-    if (!P) return d;
+void to_dev(DevProjector &d, const cse_projector *P, bool products = false) {
     d.nstabs = P->nstabs;
     for (int g = 0; g < P->nstabs && g < 64; g++) {
         d.phase[g] = P->phase[g] & 3;
@@ -218,7 +215,6 @@ DevProjector to_dev(const cse_projector *P, bool products = false) {
         d.xs[g] = x;
         d.zs[g] = z;
     }
-    return d;
 }
 
 int check_projector(cse_ctx *ctx, const cse_projector *P) {
@@ -252,51 +248,32 @@ struct Plan {
     long long stack_words = 0;  // per lane and wave, beyond LDS
     int nmax = 0;
     bool anyH = false;
-    // appends an instance of nr records, ni work items and nt terms (its
-    // record and term offsets are set here)
-    void add(InstDesc d, const DevProjector &p, long long nr, long long ni, long long nt) {
-        if (ninst == 0) rec_off[0] = item_off[0] = 0;
-        d.rec_off = nrec;
-        d.term_off = nterms;
-        inst[ninst] = d;
-        projs[ninst] = p;
-        nrec += nr;
-        nitems += ni;
-        nterms += nt;
-        ninst++;
-        nmax = std::max(nmax, d.n);
-        anyH = anyH || d.exact;
-        stack_words = std::max(stack_words, (long long)d.beyond);
-        rec_off[ninst] = nrec;
-        item_off[ninst] = nitems;
-    }
-};
-
-// Heap storage of a plan of up to n instances.
-struct PlanStore {
-    std::vector<InstDesc> inst;
-    std::vector<long long> ro, io;
-    std::vector<DevProjector> pj;
-    // n = 0 allocates nothing (the static path brings its own storage)
-    explicit PlanStore(int n) : inst(n), ro(n ? n + 1 : 0), io(n ? n + 1 : 0), pj(n) {}
-    Plan plan() {
-        Plan p;
-        p.inst = inst.data();
-        p.rec_off = ro.data();
-        p.item_off = io.data();
-        p.projs = pj.data();
-        return p;
+    // counts the instances, whose descriptors are complete but for their
+    // offsets: instance i has nr(i) records and nt(i) terms
+    template <class R, class T> void finish(int n, R &&nr, T &&nt) {
+        rec_off[0] = item_off[0] = 0;
+        for (ninst = 0; ninst < n; ninst++) {
+            InstDesc &d = inst[ninst];
+            d.rec_off = nrec;
+            d.term_off = nterms;
+            nrec += nr(ninst);
+            nitems += (d.lanes + 255) / 256;
+            nterms += nt(ninst);
+            nmax = std::max(nmax, d.n);
+            anyH = anyH || d.exact;
+            stack_words = std::max(stack_words, (long long)d.beyond);
+            rec_off[ninst + 1] = nrec;
+            item_off[ninst + 1] = nitems;
+        }
     }
 };
 
 // Plan layout: instance descriptors, item and record offsets, projectors,
 // each part 256-byte aligned.  Returns the total size.
-size_t plan_layout(const Plan &pl, size_t off[4], size_t sz[4]) {
-    const size_t ninst = (size_t)pl.ninst;
-    sz[0] = sizeof(InstDesc) * ninst;
-    sz[1] = sizeof(long long) * (ninst + 1);
-    sz[2] = sizeof(long long) * (ninst + 1);
-    sz[3] = sizeof(DevProjector) * ninst;
+size_t plan_layout(int n, size_t off[4]) {
+    const size_t ninst = (size_t)n;
+    const size_t sz[4] = {sizeof(InstDesc) * ninst, sizeof(long long) * (ninst + 1), sizeof(long long) * (ninst + 1),
+                          sizeof(DevProjector) * ninst};
     size_t total = 0;
     for (int b = 0; b < 4; b++) {
         off[b] = total;
@@ -305,16 +282,24 @@ size_t plan_layout(const Plan &pl, size_t off[4], size_t sz[4]) {
     return total;
 }
 
-// The plan is written into the bound host stage in its device layout, and
-// the device pointers into the bound plan are set; prep_batch then moves it
-// in one launch.  Every call has its results before it returns, so the stage
-// is free again at the next call.
+// A plan of n instances in a host stage, in its device layout.
+Plan plan_in(char *h, int n) {
+    size_t off[4];
+    plan_layout(n, off);
+    Plan p;
+    p.inst = (InstDesc *)(h + off[0]);
+    p.item_off = (long long *)(h + off[1]);
+    p.rec_off = (long long *)(h + off[2]);
+    p.projs = (DevProjector *)(h + off[3]);
+    return p;
+}
+
+// The device pointers into the bound plan; its size.  The plan was built in
+// the bound host stage, and prep_batch moves it in one launch.  Every call has
+// its results before it returns, so the stage is free again at the next call.
 size_t stage_plan(cse_ctx *ctx, const Plan &pl) {
-    size_t off[4], sz[4];
-    const size_t total = plan_layout(pl, off, sz);
-    const void *src[4] = {pl.inst, pl.item_off, pl.rec_off, pl.projs};
-    char *h = ctx->b_hup;
-    for (int b = 0; b < 4; b++) memcpy(h + off[b], src[b], sz[b]);
+    size_t off[4];
+    const size_t total = plan_layout(pl.ninst, off);
     char *d = ctx->b_plan;
     ctx->d_inst = (InstDesc *)(d + off[0]);
     ctx->d_itemoff = (long long *)(d + off[1]);
@@ -395,10 +380,10 @@ int sweep_grid(const cse_ctx *ctx, const Plan &pl, const SweepKernel &k) {
 }
 
 // Binds a batch to the context's own buffers, grown on demand (device memory
-// and pinned host stages).
+// and the pinned host stage of the results; the plan is in ctx->hup).
 int bind_ctx_mem(cse_ctx *ctx, const Plan &pl, int mode, bool want_terms) {
-    size_t off[4], sz[4];
-    const size_t pbytes = plan_layout(pl, off, sz);
+    size_t off[4];
+    const size_t pbytes = plan_layout(pl.ninst, off);
     const OutLayout o = out_layout(pl, mode);
     ENSURE(plan, pbytes);
     ENSURE(outb, o.total);
@@ -407,8 +392,7 @@ int bind_ctx_mem(cse_ctx *ctx, const Plan &pl, int mode, bool want_terms) {
     ENSURE(stack, (size_t)pl.stack_words * 64 * 4 * 4 * (size_t)sweep_grid(ctx, pl, sweep_choice(pl, mode)));
     if (mode == 1) ENSURE(sexp, 4 * (size_t)pl.nrec);
     if (want_terms) ENSURE(terms, 4 * (size_t)(pl.nterms > 0 ? pl.nterms : 1));
-    int rc = ensure_host(ctx, ctx->hup, pbytes);
-    if (!rc) rc = ensure_host(ctx, ctx->hstage, o.total);
+    int rc = ensure_host(ctx, ctx->hstage, o.total);
     if (rc) return rc;
     ctx->b_pinned = true;
     ctx->b_plan = (char *)ctx->plan.p;
@@ -427,8 +411,8 @@ int bind_ctx_mem(cse_ctx *ctx, const Plan &pl, int mode, bool want_terms) {
 // array and the caller's host stages; allocates nothing.
 int bind_static_mem(cse_ctx *ctx, const Plan &pl, char *hup, char *hstage) {
     if (!ctx->scratch) return fail(ctx, CSE_ERR_HIP, "static scratch array unavailable: %s", ctx->scratch_err);
-    size_t off[4], sz[4];
-    const size_t pbytes = plan_layout(pl, off, sz);
+    size_t off[4];
+    const size_t pbytes = plan_layout(pl.ninst, off);
     const OutLayout o = out_layout(pl, 1);
     if (pl.nrec > kStaticMaxChi)
         return fail(ctx, CSE_ERR_ARG, "chi=%lld above the no-allocation limit 2^%d", pl.nrec, kStaticMaxLogChi);
@@ -573,25 +557,34 @@ BatchTimes batch_times(const cse_ctx *ctx, const OutLayout &o) {
 double step_cost(int c, bool h) {
     return c < 32 ? 58.0 + (h ? 8 : 0) + 7.0 * c : 90.0 + (h ? 10 : 0) + 7.0 * 32 + 14.0 * (c - 32);
 }
+// of the slots below c
+struct StepCosts {
+    double sum[2][65];
+    StepCosts() {
+        for (int h = 0; h < 2; h++) {
+            sum[h][0] = 0.0;
+            for (int c = 0; c < 64; c++) sum[h][c + 1] = sum[h][c] + step_cost(c, h != 0);
+        }
+    }
+};
 
-// G and the stack of an instance.  G takes the largest share of the work off
-// the terms as long as the launch keeps the chip busy: with W the instructions
-// of one lane's tree, the launch takes about 4 W cycles for its last wave plus
-// 4 W per wave that each SIMD runs, and the G of the least sum is taken (an
-// instance of a batch bears its share of the last wave).  lds_only: the stack
-// has to stay in LDS.
-void plan_tree(InstDesc &d, int mode, long long nrec, int simds, int ninst, bool lds_only, int max_terms) {
+// What an instance's lane (W) and all its lanes on one SIMD's share of them
+// (work) take for each G up to top, in VALU instructions.
+struct TreeCosts {
+    int top;
+    float W[TREE_MAXG + 1], work[TREE_MAXG + 1];
+};
+
+// lds_only: the stack has to stay in LDS.
+void tree_costs(InstDesc &d, TreeCosts &c, int mode, long long nrec, int simds, bool lds_only, int max_terms) {
     const int lds = mode == 0 ? TREE_LDS_WORDS0 : TREE_LDS_WORDS1;
-    auto steps = [&](int lo, int hi) {
-        double w = 0;
-        for (int c = lo; c < hi; c++) w += step_cost(c, d.exact);
-        return w;
-    };
+    static const StepCosts costs;
+    const double *sum = costs.sum[d.exact];
+    auto steps = [&](int lo, int hi) { return hi > lo ? sum[hi] - sum[lo] : 0.0; };
     const int top = std::min(d.k, TREE_MAXG);
     for (int g = 0; g <= top; g++) d.ub[g] = (uint8_t)std::max((int)d.ub[g], TREE_LEAF);
     int words = 0;
-    double best = 0.0, below = 0.0;  // below: steps of the slots below ub[g], per term
-    d.G = 0;
+    double below = 0.0;  // steps of the slots below ub[g], per term
     for (int g = 0; g <= top; g++) {
         if (g > 0) {
             if (d.ub[g] > 32 || (1ll << g) > max_terms) break;
@@ -601,13 +594,17 @@ void plan_tree(InstDesc &d, int mode, long long nrec, int simds, int ninst, bool
         }
         const double W = (below + 60.0) * (double)(1ll << g) + steps(d.ub[g], d.n) + 500.0;
         const double lanes = (double)nrec * (double)(d.chi >> g) * (mode == 0 ? 1.0 : 0.5);
-        const double f = W / ninst + W * std::max(lanes / 64.0, 1.0) / simds;
-        if (g == 0 || f < best) {
-            best = f;
-            d.G = g;
-        }
+        c.top = g;
+        c.W[g] = (float)W;
+        c.work[g] = (float)(W * std::max(lanes / 64.0, 1.0) / simds);
     }
-    words = 0;
+}
+
+// An instance's G and stack.
+void set_tree(InstDesc &d, int mode, long long nrec, int G) {
+    const int lds = mode == 0 ? TREE_LDS_WORDS0 : TREE_LDS_WORDS1;
+    d.G = G;
+    int words = 0;
     d.nlds = d.leaf = d.beyond = 0;
     for (int g = 1; g <= d.G; g++) {
         const int w = TREE_STATE_WORDS + d.ub[g];
@@ -622,17 +619,62 @@ void plan_tree(InstDesc &d, int mode, long long nrec, int simds, int ninst, bool
             d.beyond += w;
         }
     }
+    const long long per = d.chi >> d.G;
+    d.lanes = mode == 0 ? nrec * per : tri_before(1ll << d.G, per, per);
+}
+
+// The G of each instance.  A launch takes about the work of all its lanes
+// spread over the SIMDs plus one lane's tree, the last to finish; a larger G
+// shares more of the work and makes the trees longer.  So the longest tree is
+// bounded, by the bound that gives the least sum (steps of 2^(1/4)), and each
+// instance takes its cheapest G within it.  (192 uneven instances 3.9 -> 3.4
+// ms, 20 small ones 42 -> 28 us against each instance on its own.)
+constexpr int kBounds = 96;
+inline double tree_bound(int b) { return 512.0 * exp2(0.25 * b); }
+// the first bound of at least W
+inline int bound_of(float W) {
+    int e;
+    const float m = frexpf(W / 512.0f, &e);  // in [1/2, 1)
+    return 4 * (e - 1) + (m > 0.5f) + (m > 0.59460356f) + (m > 0.70710678f) + (m > 0.84089642f);
+}
+inline int cheapest(const TreeCosts &c, double bound) {
+    int best = 0;
+    for (int g = 1; g <= c.top; g++)
+        if (c.W[g] <= bound * 1.0001 && c.work[g] < c.work[best]) best = g;
+    return best;
+}
+double best_bound(const TreeCosts *c, int n) {
+    double sum[kBounds] = {0};
+    int first = kBounds, last = 0;
+    for (int i = 0; i < n; i++) {
+        // the work under each bound: the cheapest G so far, bound by bound
+        double least = c[i].work[0];
+        int b = 0;
+        for (int g = 1; g <= c[i].top; g++) {
+            const int at = std::min(kBounds - 1, std::max(0, bound_of(c[i].W[g])));
+            if (g == 1) first = std::min(first, at);
+            last = std::max(last, at);
+            for (; b < at; b++) sum[b] += least;
+            least = std::min(least, (double)c[i].work[g]);
+        }
+        for (; b < kBounds; b++) sum[b] += least;
+    }
+    int best = std::max(0, std::min(first, last) - 1);
+    for (int b = best; b <= last; b++)
+        if (sum[b] + tree_bound(b) < sum[best] + tree_bound(best)) best = b;
+    return tree_bound(best);
 }
 
 // the bit of a slot in a record's words
 uint64_t slot_word(int x) { return x < 32 ? 1ull << (31 - x) : 1ull << (95 - x); }
 
-// mode 0: nsamp records; mode 1: chi records.  max_terms > 0 bounds the terms
-// of a lane (the calls' chunk).
-InstDesc make_inst(const cse_ctx *ctx, int mode, int t, int k, int exact, const uint64_t *L, long long nsamp,
-                   int ninst, bool lds_only, int max_terms) {
-    InstDesc d;
-    memset(&d, 0, sizeof(d));
+// An instance's descriptor but for its tree, and what its trees cost.  mode 0:
+// nsamp records; mode 1: chi records.  max_terms > 0 bounds the terms of a
+// lane (the calls' chunk).
+void make_inst(InstDesc &d, TreeCosts &c, const cse_ctx *ctx, int mode, int t, int k, int exact, const uint64_t *L,
+               long long nsamp, bool lds_only, int max_terms) {
+    memset(d.ub, 0, sizeof(d.ub));
+    memset(d.soff, 0, sizeof(d.soff));
     d.n = t;
     d.k = exact ? (t + 1) / 2 : k;
     d.exact = exact ? 1 : 0;
@@ -657,14 +699,15 @@ InstDesc make_inst(const cse_ctx *ctx, int mode, int t, int k, int exact, const 
         cse_chain_basis(t, k, L, TREE_MAXG, d.col, d.jmap, d.ub, col);
         uint8_t pos[64];
         for (int p = 0; p < t; p++) pos[col[p]] = (uint8_t)p;
-        for (int b = 0; b < k; b++)
-            for (uint64_t r = d.col[b]; r; r &= r - 1) d.LP[b] |= slot_word(pos[__builtin_ctzll(r)]);
+        for (int b = 0; b < k; b++) {
+            uint64_t w = 0;
+            for (uint64_t r = d.col[b]; r; r &= r - 1) w |= slot_word(pos[__builtin_ctzll(r)]);
+            d.LP[b] = w;
+            d.LT[b] = d.sgn[b] = 0;
+        }
     }
     for (int p = 0; p < 64; p++) d.inv[p] = p < t ? col[p] : (uint8_t)p;
-    plan_tree(d, mode, mode == 0 ? nsamp : d.chi, 4 * ctx->cus, ninst, lds_only, max_terms > 0 ? max_terms : 1 << 30);
-    const long long per = d.chi >> d.G;
-    d.lanes = mode == 0 ? nsamp * per : tri_before(1ll << d.G, per, per);
-    return d;
+    tree_costs(d, c, mode, mode == 0 ? nsamp : d.chi, 4 * ctx->cus, lds_only, max_terms > 0 ? max_terms : 1 << 30);
 }
 
 // chi <= 2^30 keeps every per-theta Z[omega] sum exact in int64: a term is at
@@ -918,7 +961,9 @@ int cse_random_states(cse_ctx *ctx, int n, uint64_t seed, int64_t first, size_t 
     ENSURE(errflag, 8);
     rc = zero64(ctx, ctx->errflag.p, 1);
     if (rc) return rc;
-    DevProjector dpj = to_dev(P);
+    DevProjector dpj;
+    memset(&dpj, 0, sizeof(dpj));
+    if (P) to_dev(dpj, P);
     hipLaunchKernelGGL(k_random_states, dim3((unsigned)((count + 3) / 4)), dim3(256), 0, ctx->stream, n,
                        dp<uint64_t>(ctx->thr) + 65 * n, seed, (long long)first, (int)count, dpj, P ? 1 : 0,
                        out ? dp<uint64_t>(ctx->s1) : nullptr, dp<int32_t>(ctx->sexp), dp<int>(ctx->errflag));
@@ -949,6 +994,17 @@ static void run_jobs(int nw, F &&job) {
     for (std::thread &th : pool) th.join();
 }
 
+// job(lo, hi) over [0, n): on several threads from 128 on (a thread takes
+// about 15 us to start, an instance of a plan about 1 us)
+extern "C++" template <class F>
+static void run_ranges(int n, F &&job) {
+    const unsigned hw = std::thread::hardware_concurrency();
+    const int nw = n >= 128 ? (int)std::min(4u, hw ? hw : 1u) : 1;
+    if (nw == 1) return job(0, n);
+    const int per = (n + nw - 1) / nw;
+    run_jobs(nw, [&](int w) { job(std::min(n, w * per), std::min(n, (w + 1) * per)); });
+}
+
 // One instance's estimators over count samples: fixed parts of kEstPart
 // samples (so the Kahan mean depends on count alone), spread over nthr host
 // threads.  At 2^16 samples one thread takes about 0.5 ms.
@@ -972,19 +1028,29 @@ static void split_estimators(int t, int64_t count, const long long *z, const int
 
 static int sampled_batch(cse_ctx *ctx, const cse_sampled_instance *in, int ninst, int chunk,
                          cse_sampled_result *res, double *kernel_ms) {
-    PlanStore store(ninst);
-    Plan pl = store.plan();
+    size_t poff[4];
+    int rc = ensure_host(ctx, ctx->hup, plan_layout(ninst, poff));
+    if (rc) return rc;
+    Plan pl = plan_in((char *)ctx->hup.p, ninst);
     bool want_terms = false;
-    for (int i = 0; i < ninst; i++) {
-        InstDesc d = make_inst(ctx, 0, in[i].P.nqubits, in[i].k, in[i].exact, in[i].L, in[i].count, ninst, false, chunk);
-        d.seed = in[i].seed;
-        d.first = in[i].first;
-        pl.add(d, to_dev(&in[i].P, in[i].exact != 0), in[i].count, (d.lanes + 255) / 256, in[i].count * d.chi);
-        want_terms = want_terms || res[i].terms != nullptr;
-    }
+    for (int i = 0; i < ninst; i++) want_terms = want_terms || res[i].terms != nullptr;
+    std::vector<TreeCosts> costs((size_t)ninst);
+    run_ranges(ninst, [&](int lo, int hi) {
+        for (int i = lo; i < hi; i++) {
+            make_inst(pl.inst[i], costs[(size_t)i], ctx, 0, in[i].P.nqubits, in[i].k, in[i].exact, in[i].L,
+                      in[i].count, false, chunk);
+            pl.inst[i].seed = in[i].seed;
+            pl.inst[i].first = in[i].first;
+            to_dev(pl.projs[i], &in[i].P, in[i].exact != 0);
+        }
+    });
+    const double bound = best_bound(costs.data(), ninst);
+    for (int i = 0; i < ninst; i++) set_tree(pl.inst[i], 0, in[i].count, cheapest(costs[(size_t)i], bound));
+    pl.finish(ninst, [&](int i) { return (long long)in[i].count; },
+              [&](int i) { return (long long)in[i].count * pl.inst[i].chi; });
     if (pl.nrec > kMaxSamples) return fail(ctx, CSE_ERR_ARG, "%lld samples above 2^24 per call", pl.nrec);
     if (want_terms && pl.nterms > (1ll << 31)) return fail(ctx, CSE_ERR_ARG, "per-term output too large");
-    int rc = ensure_thresholds(ctx);
+    rc = ensure_thresholds(ctx);
     if (!rc) rc = bind_ctx_mem(ctx, pl, 0, want_terms);
     if (rc) return rc;
     rc = run_batch(ctx, pl, 0, want_terms, stage_plan(ctx, pl), [&]() -> int {
@@ -1090,26 +1156,30 @@ int cse_batch_sampled(cse_ctx *ctx, const cse_sampled_instance *inst, int ninst,
 static int exact_batch(cse_ctx *ctx, const cse_instance *in, int ninst, int chunk, cse_exact_result *res,
                        int32_t *terms_out, double *kernel_ms, bool use_static = false, char *hup = nullptr,
                        char *hstage = nullptr) {
-    // the static path keeps its one-instance plan on the stack
-    InstDesc s_inst[1];
-    long long s_ro[2], s_io[2];
-    DevProjector s_pj[1];
-    PlanStore store(use_static ? 0 : ninst);
-    Plan pl = store.plan();
-    if (use_static) {
-        if (ninst != 1) return fail(ctx, CSE_ERR_ARG, "internal: static call with %d instances", ninst);
-        pl.inst = s_inst;
-        pl.rec_off = s_ro;
-        pl.item_off = s_io;
-        pl.projs = s_pj;
-    }
-    for (int i = 0; i < ninst; i++) {
-        const InstDesc d =
-            make_inst(ctx, 1, in[i].P.nqubits, in[i].k, in[i].exact, in[i].L, 0, ninst, use_static, chunk);
-        pl.add(d, to_dev(&in[i].P, in[i].exact != 0), d.chi, (d.lanes + 255) / 256, d.chi * (d.chi + 1) / 2);
-    }
+    if (use_static && ninst != 1) return fail(ctx, CSE_ERR_ARG, "internal: static call with %d instances", ninst);
+    size_t poff[4];
+    const size_t pbytes = plan_layout(ninst, poff);
+    if (use_static && pbytes > kStaticPlanBytes)
+        return fail(ctx, CSE_ERR_ARG, "internal: plan of %zu B above the static stage", pbytes);
+    int rc = use_static ? CSE_OK : ensure_host(ctx, ctx->hup, pbytes);
+    if (rc) return rc;
+    Plan pl = plan_in(use_static ? hup : (char *)ctx->hup.p, ninst);
+    TreeCosts one;
+    std::vector<TreeCosts> many((size_t)(ninst > 1 ? ninst : 0));
+    TreeCosts *const costs = ninst > 1 ? many.data() : &one;
+    run_ranges(ninst, [&](int lo, int hi) {
+        for (int i = lo; i < hi; i++) {
+            make_inst(pl.inst[i], costs[i], ctx, 1, in[i].P.nqubits, in[i].k, in[i].exact, in[i].L, 0, use_static,
+                      chunk);
+            to_dev(pl.projs[i], &in[i].P, in[i].exact != 0);
+        }
+    });
+    const double bound = best_bound(costs, ninst);
+    for (int i = 0; i < ninst; i++) set_tree(pl.inst[i], 1, pl.inst[i].chi, cheapest(costs[i], bound));
+    pl.finish(ninst, [&](int i) { return pl.inst[i].chi; },
+              [&](int i) { return pl.inst[i].chi * (pl.inst[i].chi + 1) / 2; });
     if (terms_out && pl.nterms > (1ll << 31)) return fail(ctx, CSE_ERR_ARG, "per-term output too large");
-    int rc = use_static ? bind_static_mem(ctx, pl, hup, hstage) : bind_ctx_mem(ctx, pl, 1, terms_out != nullptr);
+    rc = use_static ? bind_static_mem(ctx, pl, hup, hstage) : bind_ctx_mem(ctx, pl, 1, terms_out != nullptr);
     if (rc) return rc;
     rc = run_batch(ctx, pl, 1, terms_out != nullptr, stage_plan(ctx, pl), [&]() -> int {
         HIPCHK(hipMemcpyAsync(terms_out, ctx->b_terms, 4 * (size_t)pl.nterms, hipMemcpyDeviceToHost, ctx->stream));

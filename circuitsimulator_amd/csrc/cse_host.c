@@ -289,6 +289,9 @@ static uint64_t lightest(const uint64_t *w, int m, uint64_t U, uint32_t *best) {
 
 /* Combinations are searched among at most this many rows at a time. */
 #define CHAIN_SEARCH 12
+/* ... and no more once this many columns have moved: a tree has no levels of
+ * its own beyond 32 slots. */
+#define CHAIN_MOVED 32
 
 void cse_chain_basis(int t, int k, const uint64_t *L, int levels, uint64_t *rows, uint32_t *jmap, uint8_t *ub,
                      uint8_t *col) {
@@ -303,7 +306,7 @@ void cse_chain_basis(int t, int k, const uint64_t *L, int levels, uint64_t *rows
     for (int g = 0; g < k; g++) {
         uint32_t pick = 1;
         uint64_t x = w[0];
-        if (g < levels) {
+        if (g < levels && nc <= CHAIN_MOVED) {
             if (left > CHAIN_SEARCH) {
                 /* reduced row echelon form outside U: the lightest rows of a
                  * systematic basis first */
@@ -346,8 +349,7 @@ void cse_chain_basis(int t, int k, const uint64_t *L, int levels, uint64_t *rows
             if (b < 32 && ((pick >> b) & 1)) jm ^= m[b];
         rows[g] = x;
         jmap[g] = jm;
-        for (int q = 0; q < t; q++)
-            if (((x & ~U) >> q) & 1) col[nc++] = (uint8_t)q;
+        for (uint64_t r = x & ~U; r; r &= r - 1) col[nc++] = (uint8_t)__builtin_ctzll(r);
         U |= x;
         if (g < levels) ub[g + 1] = (uint8_t)nc;
         /* one row of the combination makes room (the rest still spans) */
@@ -358,8 +360,7 @@ void cse_chain_basis(int t, int k, const uint64_t *L, int levels, uint64_t *rows
         }
         left--;
     }
-    for (int q = 0; q < t; q++)
-        if (!((U >> q) & 1)) col[nc++] = (uint8_t)q;
+    for (uint64_t r = (t >= 64 ? ~0ull : (1ull << t) - 1) & ~U; r; r &= r - 1) col[nc++] = (uint8_t)__builtin_ctzll(r);
 }
 
 /* ------------------------------------------------------------- rank */
