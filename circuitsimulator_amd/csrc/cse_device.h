@@ -336,15 +336,14 @@ DEV bool rs_random_state(RState &s, int n, const uint64_t *thr, uint64_t key, ui
 // stays symmetric, so bit x of row i is J_xi) and D_x in Z8 (always even).
 // Uniform: the active rows, h and Q.
 //
-// Packed form (PK = true, n <= 60): D_x lives in bits 61..63 of the J row,
-// so one broadcast of row a gives both the J-row and D_a, and adding to D is
+// D_x is in a register of its own.  The packed form that pk_restrict_general
+// and as_expsum_packed work on (n <= 60) has it in bits 61..63 of the J row,
+// so one broadcast of row a gives both the J row and D_a, and adding to D is
 // a 64-bit add on the row (mod 8 in the top three bits, no carry into the
-// row).  Unpacked form (PK = false): D_x in its own register.
-#define CSE_ROWMASK 0x1FFFFFFFFFFFFFFFull
-
+// row).
 struct AState {
     u64 G, J;
-    int d;      // PK = false only
+    int d;
     u64 act;
     u64 h;
     int Q;
@@ -356,54 +355,27 @@ DEV bool lane_in(u64 mask) { return __builtin_amdgcn_inverse_ballot_w64(mask); }
 // all-ones if b else 0 (uniform integer select)
 DEV u64 allmask(int b) { return 0ull - (u64)(b & 1); }
 
-template <bool PK> DEV int d_of_row(u64 row, const AState &s, int a) {
-    if (PK) return (int)(row >> 61);
-    return rl32(s.d, a);
-}
-template <bool PK> DEV u64 row_bits(u64 row) { return PK ? (row & CSE_ROWMASK) : row; }
-// D_x += v on lanes in U (v uniform, 0..7)
-template <bool PK> DEV void d_add(AState &s, u64 U, int v) {
-    if (PK) {
-        if (lane_in(U)) s.J += (u64)v << 61;
-    } else {
-        if (lane_in(U)) s.d = (s.d + v) & 7;
-    }
-}
-// D_x += 4 on lanes in U
-template <bool PK> DEV void d_add4(AState &s, u64 U) {
-    if (PK) {
-        if (lane_in(U)) s.J ^= bit(63);
-    } else {
-        if (lane_in(U)) s.d ^= 4;
-    }
-}
-
 // Basis change R = I + sum_{b in Sp} e_b e_i^T of the quadratic form
 // (updateDJ of the reference, stabilizer.c:129-160, for a rank-1 R):
 //   D_b += D_i + 4 J_bi, J <- R J R^T  (and G_b ^= G_i when withG).
 // J_ii is taken as [D_i in {2,6}].  Returns M = column i of R J (bit x =
 // (RJ)_xi), which fixing z_i needs; *di_out = D_i.
-template <bool PK> DEV u64 as_basis_change(AState &s, int i, u64 Sp, bool withG, int *di_out) {
+DEV u64 as_basis_change(AState &s, int i, u64 Sp, bool withG, int *di_out) {
     const u64 bi = bit(i);
     const u64 Jr = rl64(s.J, i);
-    const int di = d_of_row<PK>(Jr, s, i);
+    const int di = rl32(s.d, i);
     const int jii = (di >> 1) & 1;
-    const u64 Jc = (row_bits<PK>(Jr) & ~bi) | ((u64)jii << i);
+    const u64 Jc = (Jr & ~bi) | ((u64)jii << i);
     const u64 M = Jc ^ (Sp & allmask(jii));
     if (withG) {
         const u64 Gi = rl64(s.G, i);
         if (lane_in(Sp)) s.G ^= Gi;
     }
     // rows b in Sp: J_b ^= Jc, D_b += D_i + 4 J_bi (J_bi = bit b of Jc)
-    if (PK) {
-        if (lane_in(Sp)) s.J = (s.J ^ Jc) + ((u64)di << 61);
-        if (lane_in(Sp & Jc)) s.J ^= bit(63);
-    } else {
-        const int four = lane_in(Jc) ? 4 : 0;
-        if (lane_in(Sp)) {
-            s.d = (s.d + di + four) & 7;
-            s.J ^= Jc;
-        }
+    const int four = lane_in(Jc) ? 4 : 0;
+    if (lane_in(Sp)) {
+        s.d = (s.d + di + four) & 7;
+        s.J ^= Jc;
     }
     // columns: rows x with (RJ)_xi = 1 get J_x ^= Sp
     if (lane_in(M)) s.J ^= Sp;
@@ -412,24 +384,24 @@ template <bool PK> DEV u64 as_basis_change(AState &s, int i, u64 Sp, bool withG,
 }
 
 // Basis change as above, then fix z_i = c and retire row i.
-template <bool PK> DEV void as_eliminate(AState &s, int i, u64 Sp, int c, bool withG) {
+DEV void as_eliminate(AState &s, int i, u64 Sp, int c, bool withG) {
     int di;
-    const u64 M = as_basis_change<PK>(s, i, Sp, withG, &di);
+    const u64 M = as_basis_change(s, i, Sp, withG, &di);
     if (c) {
         s.Q = (s.Q + di) & 7;
-        d_add4<PK>(s, M);
+        if (lane_in(M)) s.d ^= 4;
         if (withG) s.h ^= rl64(s.G, i);
     }
     s.act &= ~bit(i);
 }
 
 // Restrict to {x : x . xi = alpha}.  Returns false if the restriction is empty.
-template <bool PK> DEV bool as_restrict(AState &s, u64 xi, int alpha) {
+DEV bool as_restrict(AState &s, u64 xi, int alpha) {
     u64 S = ballot(lane_in(s.act) && par64(s.G & xi));
     int beta = (alpha ^ __popcll(s.h & xi)) & 1;
     if (S == 0) return beta == 0;
     int i = 63 - __clzll(S);
-    as_eliminate<PK>(s, i, S & ~bit(i), beta, true);
+    as_eliminate(s, i, S & ~bit(i), beta, true);
     return true;
 }
 
@@ -442,8 +414,8 @@ template <bool PK> DEV bool as_restrict(AState &s, u64 xi, int alpha) {
 //
 // Packed layout (D_x in bits 61..63 of J_x), the elimination loop scheduled
 // by hand: the compiler's lowering of this loop spends most of its scalar
-// instructions on control-flow bookkeeping, and scalar issue bounds the
-// sweep.  The loop takes, per step, the lowest active variable a:
+// instructions on control-flow bookkeeping, and scalar issue bounds it.  The
+// loop takes, per step, the lowest active variable a:
 //  D_a in {2,6} (bit 62 of J_a): factor sqrt2 w^{s}, s = +1 for 2, -1 for 6;
 //    rows b in eta = J_a & act get J_b ^= eta and D_b -= D_a;
 //  D_a in {0,4}, eta != 0: factor 2 and the constraint eta . z = D_a/4,
@@ -471,9 +443,6 @@ template <bool PK> DEV bool as_restrict(AState &s, u64 xi, int alpha) {
 // v41 = 1 << 31.  A
 // VALU instruction reads an SGPR that v_readlane wrote only two or more
 // instructions later.  Every step clears a bit of act below 60.
-// CSE_ELIM_LOOP_BODY(S, CNEXT) is the loop with its labels suffixed by S
-// (two copies can share an asm block) and CNEXT the instruction that
-// follows a step without a constraint (the branch back to the top).
 #define CSE_END_ROW 60
 // The loop's head: the lowest active variable a leaves act, its row J_a
 // (D_a in the top bits) is read, eta = J_a & act, SCC = D_a in {2,6}.  Each
@@ -487,15 +456,15 @@ template <bool PK> DEV bool as_restrict(AState &s, u64 xi, int alpha) {
     "v_readlane_b32 s63, %[jhi], s56\n\t"                                   \
     "s_and_b64 s[64:65], s[62:63], s[58:59]\n\t"                            \
     "s_bitcmp1_b32 s63, 30\n\t"
-#define CSE_ELIM_NEXT(S)                                                    \
+#define CSE_ELIM_NEXT                                                       \
     CSE_ELIM_HEAD                                                           \
-    "s_cbranch_scc1 L_A" S "%=\n\t"                                          \
-    "s_branch L_nonA" S "%=\n"
-#define CSE_ELIM_LOOP_BODY(S, CNEXT)                                        \
-    "L_top" S "%=:\n\t"                                                     \
+    "s_cbranch_scc1 L_A%=\n\t"                                              \
+    "s_branch L_nonA%=\n"
+#define CSE_ELIM_LOOP                                                       \
+    "L_top%=:\n\t"                                                          \
     CSE_ELIM_HEAD                                                           \
-    "s_cbranch_scc0 L_nonA" S "%=\n"                                        \
-    "L_A" S "%=:\n\t"                                                       \
+    "s_cbranch_scc0 L_nonA%=\n"                                             \
+    "L_A%=:\n\t"                                                            \
     /* D_a in {2,6}: rows in eta take J ^= eta, D -= D_a; m += 1, and       \
        the carry in (SCC = D_a's top bit) counts D_a = 6 in W's low bits */ \
     "v_xor_b32 %[vt0], s64, %[jlo]\n\t"                                     \
@@ -505,11 +474,11 @@ template <bool PK> DEV bool as_restrict(AState &s, u64 xi, int alpha) {
     "s_bitcmp1_b32 s63, 31\n\t"                                             \
     "s_addc_u32 s60, s60, 0x20000000\n\t"                                   \
     CSE_ELIM_HEAD                                                           \
-    "s_cbranch_scc1 L_A" S "%=\n"                                           \
-    "L_nonA" S "%=:\n\t"                                                    \
+    "s_cbranch_scc1 L_A%=\n"                                                \
+    "L_nonA%=:\n\t"                                                         \
     /* eta without bit 63: a constraint? */                                 \
     "s_lshl_b64 s[66:67], s[64:65], 1\n\t"                                  \
-    "s_cbranch_scc0 L_C" S "%=\n\t"                                         \
+    "s_cbranch_scc0 L_C%=\n\t"                                              \
     /* D_a in {0,4} with a constraint: pivot i = min(eta).  Row i and       \
        column i are dead from here on, so eta itself serves as Sp;          \
        its bit 63 is c = D_a / 4, so D += 4 c on the rows of M comes        \
@@ -522,7 +491,7 @@ template <bool PK> DEV bool as_restrict(AState &s, u64 xi, int alpha) {
     "v_cndmask_b32_e64 %[vt0], 0, -1, s[64:65]\n\t"                         \
     "s_and_b32 s56, s67, 0xe0000000\n\t"                                    \
     "s_bitcmp1_b32 s67, 30\n\t"                                             \
-    "s_cbranch_scc1 L_jii" S "%=\n\t"                                       \
+    "s_cbranch_scc1 L_jii%=\n\t"                                            \
     /* D_i in {0,4}: M = Jc, and D += D_i on Sp is bit 63 of Jc. Rows       \
        of M take J ^= Sp with bit 63 flipped where x is in Sp too           \
        (the 4 J_xi of the rows in Sp). */                                   \
@@ -531,15 +500,15 @@ template <bool PK> DEV bool as_restrict(AState &s, u64 xi, int alpha) {
     "v_bitop3_b32 %[jhi], %[jhi], s67, %[vt0] bitop3:0x78\n\t"              \
     "v_bitop3_b32 %[vt1], s65, %[vt0], v41 bitop3:0x78\n\t"                 \
     "s_bitcmp1_b32 s63, 31\n\t"                                             \
-    "s_cbranch_scc0 L_noc0" S "%=\n\t"                                      \
+    "s_cbranch_scc0 L_noc0%=\n\t"                                           \
     "s_add_u32 s60, s60, s56\n"                                             \
-    "L_noc0" S "%=:\n\t"                                                    \
+    "L_noc0%=:\n\t"                                                         \
     "v_bitop3_b32 %[jlo], %[jlo], s64, %[vt3] bitop3:0x78\n\t"              \
     "v_bitop3_b32 %[jhi], %[jhi], %[vt1], %[vt3] bitop3:0x78\n\t"           \
-    CSE_ELIM_NEXT(S)                                                        \
+    CSE_ELIM_NEXT                                                           \
     /* D_i in {2,6}: M = Jc ^ Sp; rows in Sp take J ^= Jc and               \
        D += D_i + 4 J_xi */                                                 \
-    "L_jii" S "%=:\n\t"                                                     \
+    "L_jii%=:\n\t"                                                          \
     "s_and_b32 s67, s67, 0x1fffffff\n\t"                                    \
     "v_cndmask_b32_e64 %[vt3], 0, -1, s[66:67]\n\t"                         \
     "v_bitop3_b32 %[jlo], %[jlo], s66, %[vt0] bitop3:0x78\n\t"              \
@@ -549,20 +518,19 @@ template <bool PK> DEV bool as_restrict(AState &s, u64 xi, int alpha) {
     "v_add_u32 %[jhi], %[jhi], %[vt2]\n\t"                                  \
     "v_xor_b32 %[vt3], %[vt3], %[vt0]\n\t"                                  \
     "s_bitcmp1_b32 s63, 31\n\t"                                             \
-    "s_cbranch_scc0 L_noc1" S "%=\n\t"                                      \
+    "s_cbranch_scc0 L_noc1%=\n\t"                                           \
     "s_add_u32 s60, s60, s56\n"                                             \
-    "L_noc1" S "%=:\n\t"                                                    \
+    "L_noc1%=:\n\t"                                                         \
     "v_bitop3_b32 %[jlo], %[jlo], s64, %[vt3] bitop3:0x78\n\t"              \
     "v_bitop3_b32 %[jhi], %[jhi], s65, %[vt3] bitop3:0x78\n\t"              \
-    CSE_ELIM_NEXT(S)                                                        \
+    CSE_ELIM_NEXT                                                           \
     /* D_a in {0,4} without a constraint: the sum vanishes (D_a = 4,        \
        or the end row) or nC += 1 */                                        \
-    "L_C" S "%=:\n\t"                                                       \
+    "L_C%=:\n\t"                                                            \
     "s_bitcmp1_b32 s63, 31\n\t"                                             \
     "s_cbranch_scc1 L_end%=\n\t"                                            \
     "s_add_u32 s60, s60, 0xffffff80\n\t"                                    \
-    CNEXT
-#define CSE_ELIM_LOOP CSE_ELIM_LOOP_BODY("", "s_branch L_top%=\n")
+    "s_branch L_top%=\n"
 
 // The loop on an AState (records of n <= 60, row 60 the end row); p and m
 // as as_expsum.  W's p field counts down from the base 128 (p = n0 + nC
@@ -597,8 +565,7 @@ DEV int as_expsum_packed(AState &s, int &p, int &m) {
     return 1;
 }
 
-template <bool PK> DEV int as_expsum(AState &s, int &p, int &m) {
-    if (PK) return as_expsum_packed(s, p, m);
+DEV int as_expsum(AState &s, int &p, int &m) {
     int pp = 0, macc = 0, zero = 0;
     u64 act = s.act;
     while (act) {
@@ -606,7 +573,7 @@ template <bool PK> DEV int as_expsum(AState &s, int &p, int &m) {
         act &= ~bit(a);
         const u64 Ja = rl64(s.J, a);
         const u64 eta = Ja & act;
-        const int da = d_of_row<PK>(Ja, s, a);
+        const int da = rl32(s.d, a);
         const int h4 = (da >> 2) & 1;
         if (da & 2) {
             // D_a = 2 (s = +1) or 6 (s = -1): factor sqrt2 w^s; D_b -= 2s
@@ -614,9 +581,7 @@ template <bool PK> DEV int as_expsum(AState &s, int &p, int &m) {
             pp += 1;
             macc += h4 ? 7 : 1;
             const int delta = h4 ? 2 : 6;
-            if (PK) {
-                if (lane_in(eta)) s.J = (s.J ^ eta) + ((u64)delta << 61);
-            } else if (lane_in(eta)) {
+            if (lane_in(eta)) {
                 s.d = (s.d + delta) & 7;
                 s.J ^= eta;
             }
@@ -626,9 +591,9 @@ template <bool PK> DEV int as_expsum(AState &s, int &p, int &m) {
             const int i = 63 - __clzll(eta);
             act &= ~bit(i);
             int di;
-            const u64 M = as_basis_change<PK>(s, i, eta & ~bit(i), false, &di);
+            const u64 M = as_basis_change(s, i, eta & ~bit(i), false, &di);
             s.Q = (s.Q + (di & -h4)) & 7;
-            d_add4<PK>(s, M & allmask(h4));
+            if (lane_in(M & allmask(h4))) s.d ^= 4;
         } else {
             // factor 1 + w^{D_a}: 2 if D_a = 0, the whole sum vanishes if 4
             pp += 2;

@@ -236,14 +236,14 @@ DEV void ip_general(const RState &r1, const RState &r2, int &eps, int &p, int &m
     for (int b = r2.k; b < r2.n; b++) {
         u64 xi = rl64(r2.Gb, b);
         int alpha = par64(r2.h & xi);
-        if (!as_restrict<false>(s, xi, alpha)) {
+        if (!as_restrict(s, xi, alpha)) {
             eps = 0; p = 0; m = 0;
             return;
         }
     }
     as_subtract_general(s, r2);
     int pp, mm;
-    eps = as_expsum<false>(s, pp, mm);
+    eps = as_expsum(s, pp, mm);
     p = eps ? pp - r1.k - r2.k : 0;
     m = mm;
 }
@@ -314,7 +314,6 @@ DEV int rs_project(RState &s, const DevProjector &P) {
     return sexp;
 }
 
-
 DEV u64 shfl64(u64 v, int lane) {
     const unsigned lo = (unsigned)__shfl((int)(unsigned)v, lane, 64);
     const unsigned hi = (unsigned)__shfl((int)(unsigned)(v >> 32), lane, 64);
@@ -324,38 +323,133 @@ DEV u64 shfl64(u64 v, int lane) {
 // slot x at bit 31 - x of each half, as the sweep keeps its words
 DEV u64 brev32x2(u64 v) { return (u64)__brev((unsigned)v) | (u64)__brev((unsigned)(v >> 32)) << 32; }
 
-// The record of a state in reduced row echelon form, rows at their pivot
-// lanes: its form on the instance's slots (cse_tree.h).
-//  * the slot of a pivot column is the coordinate x_a = h_a + z_a itself, so
-//    the rows with h_a = 1 (H) are expanded about z = 1: Q += sum_H D + 4
-//    #edges(J in H), D_a -> -D_a on H, D_x += 4 |J_x & H|;
-//  * the slot of another column q is the multiplier of x_q = h_q + G_.q . z:
-//    J_q = the column of G, D_q = 4 (h_q + |column & H|);
-//  * slots are the columns in the order D.inv.  The matrix is U + U^T with U
-//    the pivot rows' part of it (J below the diagonal, G at the other
-//    columns), and U's rows, then by a transpose its columns move to their
-//    slots.
-DEV void store_form(const AState &s, const InstDesc &D, int sexp, uint64_t *rec) {
+// A state as a form on all n columns (cse_tree.h): the slot of a pivot column
+// is its coordinate x_a, the slot of another column the multiplier of its
+// constraint.  So the state is H on the columns of F applied to the phase
+// state sum_s w^{Q + D.s + 4 s J s} |s>, whatever its dimension.  Lane x holds
+// row x of J, with d1 (D_x = 2 d1_x + 4 d2_x) on its diagonal; the rest is
+// uniform.
+struct FormState {
+    u64 M;
+    u64 d1, d2, F;
+    int Q;
+};
+
+// The form of a state in reduced row echelon form, rows at their pivot lanes.
+//  * x_a = h_a + z_a: the rows with h_a = 1 (H) are expanded about z = 1: Q +=
+//    sum_H D + 4 #edges(J in H), D_a -> -D_a on H, D_x += 4 |J_x & H|;
+//  * x_q = h_q + G_.q . z on another column: J_q = the column of G, D_q =
+//    4 (h_q + |column & H|).  The matrix is U + U^T with U the pivot rows' part
+//    of it (J below the diagonal, G at the other columns).
+DEV void to_form(const AState &s, int n, FormState &f) {
     const int x = lane_id();
-    const int n = D.n;
-    const int src = x < n ? (int)D.inv[x] : x;
     const bool a = lane_in(s.act);
     const u64 H = s.act & s.h, nonact = lowmask(n) & ~s.act;
     const u64 J = a ? s.J & s.act & ~bit(x) : 0ull, Jl = J & lowmask(x);
     int d = a ? (s.d & 6) : 0;
-    const int Q = s.Q + 2 * __popcll(ballot(lane_in(H) && (d & 2))) + 4 * __popcll(ballot(lane_in(H) && (d & 4))) +
-                  4 * __popcll(ballot(lane_in(H) && par64(Jl & H)));
+    f.Q = (s.Q + 2 * __popcll(ballot(lane_in(H) && (d & 2))) + 4 * __popcll(ballot(lane_in(H) && (d & 4))) +
+           4 * __popcll(ballot(lane_in(H) && par64(Jl & H)))) & 7;
     const u64 hq = s.h ^ wave_xor(lane_in(H) ? s.G : 0ull);
     if (lane_in(H)) d = (8 - d) & 7;
     d = (d + 4 * par64(J & H)) & 7;
-    if (!a) d = 4 * (int)((hq & nonact) >> x & 1ull);
-    const u64 Ut = shfl64(transpose64(shfl64(a ? Jl | (s.G & nonact) : 0ull, src)), src);
-    const u64 M = Ut ^ transpose64(Ut);
-    d = __shfl(d, src, 64);
-    const bool f = __shfl((int)((nonact >> x) & 1ull), src, 64) != 0;
-    const u64 d1 = ballot(d & 2), d2 = ballot(d & 4), F = ballot(f);
+    f.d1 = ballot(a && (d & 2));
+    f.d2 = ballot(a && (d & 4)) | (hq & nonact);
+    f.F = nonact;
+    const u64 U = a ? Jl | (s.G & nonact) : 0ull;
+    f.M = U ^ transpose64(U) ^ (f.d1 & bit(x));
+}
+
+// Projection of a form by P; returns the number of 2^-1/2 factors, -1 if it
+// vanishes.  A generator i^m Z(zeta) X(xi) acts on the phase state as i^m'
+// Z(fz) X(fx) with xi and zeta exchanged on F, and multiplies it by w^w
+// (-1)^{eta.s}:
+//   w = 2 m' + sum_{fx} D + 4 #edges(J in fx), eta = J fx + fz (the diagonal
+//   of J is d1).
+//  eta empty: nothing (w = 0) or zero (w = 4);
+//  w in {2,6}: 2^-1/2 w^{+-1}, D -+= 2 on eta, J ^= eta eta^T;
+//  w in {0,4}: the constraint eta . s = w/4, solved for the lowest i in eta,
+//   whose slot becomes its multiplier (or its coordinate again), as in a
+//   tree's step of the third kind; the updates of J keep d1 on its diagonal.
+// Scalar issue bounds it: 63 scalar and 40 vector instructions a generator.
+DEV int project_form(FormState &f, const DevProjector &P) {
+    const int x = lane_id();
+    // generator x in lane x: one load for all instead of one per step
+    const u64 pz = P.zs[x], px = P.xs[x], lowx = lowmask(x);
+    const int pm = P.phase[x];
+    const int ng = P.nstabs;
+    u64 M = f.M, d1 = f.d1, d2 = f.d2, F = f.F;
+    int Q = f.Q, sexp = 0;
+    for (int g = 0; g < ng; g++) {
+        const u64 zeta = rl64(pz, g), xi = rl64(px, g), swap = (zeta ^ xi) & F;
+        const u64 fx = xi ^ swap, in = M & fx;
+        const u64 low = ballot(par64(in & lowx));
+        const u64 eta = ballot(par64(in)) ^ zeta ^ swap;
+        // w / 2, mod 4
+        const int u = rl32(pm, g) + __popcll(d1 & fx) + 2 * (__popcll(zeta & xi & F) + __popcll((low ^ d2) & fx));
+        if (eta == 0) {
+            if (u & 3) return -1;
+            continue;
+        }
+        sexp++;
+        if (u & 1) {
+            if (u & 2) {
+                Q -= 1;
+                d2 ^= eta & d1;
+            } else {
+                Q += 1;
+                d2 ^= eta & ~d1;
+            }
+            d1 ^= eta;
+            if (lane_in(eta)) M ^= eta;
+        } else {
+            const int i = __builtin_ctzll(eta);
+            const u64 o = bit(i), row = rl64(M, i) & ~o, v = eta ^ o;
+            const bool ti = (d2 & o) != 0;
+            u64 al = row ^ o, wm = row;
+            // D_x += +-D_i on v, 4 c on row, 4 on both (c = w / 4)
+            if (d1 & o) {
+                al ^= v;
+                d2 ^= v & d1;
+                d1 ^= eta;
+                if (u & 2) {
+                    Q += ti ? 6 : 2;
+                    d2 ^= (row & ~v) ^ (ti ? 0ull : v);
+                } else {
+                    d2 ^= (row & v) ^ (ti ? v : 0ull);
+                }
+            } else {
+                wm |= o;
+                if (u & 2) {
+                    Q += ti ? 4 : 0;
+                    d2 ^= row & ~v;
+                } else {
+                    d2 ^= row & v;
+                }
+                if (ti) d2 ^= v;
+            }
+            d2 = u & 2 ? d2 | o : d2 & ~o;
+            F ^= o;
+            M ^= (lane_in(eta) ? al : 0ull) ^ (lane_in(wm) ? eta : 0ull);
+        }
+    }
+    f.M = M;
+    f.d1 = d1;
+    f.d2 = d2;
+    f.F = F;
+    f.Q = Q & 7;
+    return sexp;
+}
+
+// The record of a form: rows and, by a transpose, columns of the symmetric
+// matrix move to the instance's slots.
+DEV void store_form(const FormState &f, const InstDesc &D, int sexp, uint64_t *rec) {
+    const int x = lane_id();
+    const int src = x < D.n ? (int)D.inv[x] : x;
+    const u64 M = shfl64(transpose64(shfl64(f.M & ~bit(x), src)), src);
+    const u64 sx = bit(src);
+    const u64 d1 = ballot(f.d1 & sx), d2 = ballot(f.d2 & sx), F = ballot(f.F & sx);
     if (x == 0) {
-        rec[0] = ((uint64_t)n << 8) | ((uint64_t)(Q & 7) << 16) | ((uint64_t)sexp << 24);
+        rec[0] = ((uint64_t)D.n << 8) | ((uint64_t)f.Q << 16) | ((uint64_t)sexp << 24);
         rec[1] = brev32x2(F);
         rec[2] = brev32x2(d1);
         rec[3] = brev32x2(d2);
@@ -397,7 +491,7 @@ DEV void to_rref(AState &s, int k) {
         Pm |= bit(pc);
         const u64 Sp = ballot(x < k && x != a && ((s.G >> pc) & 1ull));
         int dummy;
-        if (Sp) as_basis_change<false>(s, a, Sp, true, &dummy);
+        if (Sp) as_basis_change(s, a, Sp, true, &dummy);
     }
     // lane p's row is row src of the state, and bit p of a row is its bit src
     // (a transpose away from the same move)
@@ -443,84 +537,6 @@ k_random_states(int n, const uint64_t *__restrict__ thr, uint64_t seed, long lon
     if (sexp && lane_id() == 0) sexp[wave] = se;
 }
 
-// The record of Pi prepL(x) built directly in reduced row echelon form,
-// rows at their pivot lanes: the product state (|+> on supp(x), |0>
-// elsewhere) has act = supp(x), G_a = e_a, h = 0 and no form.  Each generator
-// i^m Z(zeta) X(xi) (the cases of measurePauli, stabilizer.c:827-959) works
-// on the coordinates c = xi & act of xi in that basis and the residual
-// rho = xi + sum_{a in c} G_a (zero exactly when xi is in the span):
-//   w = 2m + 4 zeta.h + sum_{a in c} D_a + 4 #edges(J inside c) (mod 8),
-//   eta_b = (J c)_b + zeta.G_b on act (J_bb = [D_b in {2,6}]);
-//  rho = 0, w in {0,4}: the constraint eta . z = w/4 -- nothing (eta empty,
-//    w = 0), zero (eta empty, w = 4), else an elimination of min(eta);
-//  rho = 0, w in {2,6}: a factor 2^-1/2 w^{+-1}: Q += s, D -= 2s and J ^= eta
-//    eta^T on eta (s = 1 for w = 2, -1 for 6);
-//  rho != 0: a new variable at p = min(rho) with G_p = rho, D_p =
-//    w + 4 zeta.rho, J row and column eta, then the basis change that clears
-//    column p from the other rows.
-// Returns the number of 2^-1/2 factors, -1 if the projection vanishes.
-DEV int rs_project_rref(AState &s, const DevProjector &P) {
-    const int x = lane_id();
-    // generator x in lane x: one load for all instead of one per step
-    const u64 pz = P.zs[x], px = P.xs[x];
-    const int pm = P.phase[x];
-    const int ng = P.nstabs;
-    int sexp = 0;
-    for (int g = 0; g < ng; g++) {
-        const int m = rl32(pm, g) & 3;
-        const u64 zeta = rl64(pz, g), xi = rl64(px, g);
-        const u64 c = xi & s.act;
-        const bool inA = lane_in(s.act), inC = lane_in(c);
-        const u64 rho = xi ^ wave_xor(inC ? s.G : 0ull);
-        const u64 vze = ballot(inA && par64(s.G & zeta));
-        const u64 d1 = ballot(inC && (s.d & 2)), d2 = ballot(inC && (s.d & 4));
-        const u64 edg = ballot(inC && par64(s.J & c & lowmask(x)));
-        const int w = (2 * m + 4 * par64(zeta & s.h) + 2 * __popcll(d1) + 4 * __popcll(d2) + 4 * __popcll(edg)) & 7;
-        const u64 jb = (s.J & ~bit(x)) | ((u64)((s.d >> 1) & 1) << x);
-        const u64 eta = ballot(inA && par64(jb & c)) ^ vze;
-        if (rho == 0 && (w & 2) == 0) {
-            if (eta == 0) {
-                if (w) return -1;
-                continue;
-            }
-            const int i = __builtin_ctzll(eta);
-            as_eliminate<false>(s, i, eta & ~bit(i), w >> 2, true);
-        } else if (rho == 0) {
-            const int sg = w == 2 ? 1 : -1;
-            s.Q = (s.Q + sg) & 7;
-            if (lane_in(eta)) {
-                s.d = (s.d - 2 * sg) & 7;
-                s.J ^= eta;
-            }
-        } else {
-            const int p = __builtin_ctzll(rho);
-            const int dp = (w + 4 * par64(zeta & rho)) & 7;
-            if (inA) s.J = (s.J & ~bit(p)) | (((eta >> x) & 1ull) << p);
-            if (x == p) {
-                s.G = rho;
-                s.d = dp;
-                s.J = eta | ((u64)((dp >> 1) & 1) << p);
-            }
-            s.act |= bit(p);
-            const u64 T = ballot(lane_in(s.act) && x != p && ((s.G >> p) & 1ull));
-            if (T) {
-                int dummy;
-                as_basis_change<false>(s, p, T, true, &dummy);
-            }
-        }
-        sexp++;
-    }
-    return sexp;
-}
-
-// Records of projected states, one wave per record g (global index over all
-// instances; instance found from the record prefix).
-// mode 0: theta_s = random stabilizer state s = first + local index of the
-//         instance's Philox stream (seed)
-// mode 1: phi_i = prepH(i) (exact) or prepL(i) (|L>), i = local index
-// then Pi (innerprod.c:95-116 / :218-241), in reduced row echelon form, and
-// the record.  |H^t> instances are taken to the coordinates of to_products
-// first, their projector with them.
 // The instance that holds global index key: the largest i < n with
 // off[i] <= key, for nondecreasing off with off[0] <= key.  The whole wave
 // searches: each round lane x reads off[lo + x*step] and the ballot's highest
@@ -541,6 +557,18 @@ DEV int find_instance(const long long *__restrict__ off, int n, long long key) {
     return lo;
 }
 
+// Records of projected states, one wave per record g (global index over all
+// instances; instance found from the record prefix).
+// mode 0: theta_s = random stabilizer state s = first + local index of the
+//         instance's Philox stream (seed); |H^t> instances take it to the
+//         coordinates of to_products
+// mode 1: phi_i = prepH(i) (exact) or prepL(i) (|L>), i = local index
+// then, as a form, Pi (innerprod.c:95-116 / :218-241) and the record.
+// The state is a form from the start, so a generator needs no constraint
+// solved, no G and no h.  131072 records of t = 40 with 16 generators (mode 1):
+// 0.46 ms as states in echelon form (2151 vector and 1412 scalar instructions
+// each), 0.249 ms as forms (687 and 1025); 4096 sampled ones of t = 40, r = 8:
+// 24.4 and 19.0 us.
 extern "C" __global__ void __launch_bounds__(256)
 k_records(int mode, int ninst, const long long *__restrict__ rec_off, const InstDesc *__restrict__ inst,
           const DevProjector *__restrict__ projs, const uint64_t *__restrict__ thr_table, long long nrec,
@@ -554,7 +582,7 @@ k_records(int mode, int ninst, const long long *__restrict__ rec_off, const Inst
     const long long local = g - rec_off[in];
     const int n = D.n;
     uint64_t *rec = recs + (size_t)REC_WORDS * (size_t)g;
-    AState a;
+    FormState f;
     if (mode == 0) {
         RState s;
         if (!rs_random_state(s, n, thr_table + 65 * n, D.seed, (uint64_t)(D.first + local))) {
@@ -565,27 +593,26 @@ k_records(int mode, int ninst, const long long *__restrict__ rec_off, const Inst
             Rec::store_vanished(rec, n);
             return;
         }
+        AState a;
         to_astate(s, a);
         if (D.exact) to_products(a, n);
         to_rref(a, s.k);
+        to_form(a, n, f);
     } else {
         // the decomposition state, a product of |0>, |+> and (|H^t>) |->
         const int x = lane_id();
-        const u64 row = x < D.k ? D.col[x] : 0ull, sgn = x < D.k && D.exact ? D.sgn[x] : 0ull;
         const bool on = x < D.k && ((local >> x) & 1);
-        const u64 xv = (D.exact ? lowmask(n) : 0ull) ^ wave_xor(on ? row : 0ull);
-        const u64 neg = D.exact ? wave_xor(on ? sgn : 0ull) : 0ull;
-        a.act = xv & lowmask(n);
-        a.G = lane_in(a.act) ? bit(x) : 0ull;
-        a.J = 0;
-        a.d = lane_in(a.act & neg) ? 4 : 0;
-        a.h = 0;
-        a.Q = 0;
+        const u64 xv = (D.exact ? lowmask(n) : 0ull) ^ wave_xor(on ? D.col[x] : 0ull);
+        f.M = 0;
+        f.d1 = 0;
+        f.d2 = D.exact ? wave_xor(on ? D.sgn[x] : 0ull) & xv : 0ull;
+        f.F = lowmask(n) & ~xv;
+        f.Q = 0;
     }
-    const int se = rs_project_rref(a, projs[in]);
+    const int se = project_form(f, projs[in]);
     if (lane_id() == 0) sexp_out[g] = se;
     if (se < 0) Rec::store_vanished(rec, n);
-    else store_form(a, D, se, rec);
+    else store_form(f, D, se, rec);
 }
 
 #include "cse_sweep.h"
