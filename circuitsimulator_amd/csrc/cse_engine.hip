@@ -575,6 +575,13 @@ struct TreeCosts {
     float W[TREE_MAXG + 1], work[TREE_MAXG + 1];
 };
 
+// The terms of index bit 0 are summed in pairs (cse_tree.h) where that bit
+// moves more slots than are looked up, in launches without |H^t> instances
+// (d.pair as make_inst leaves it): those have bits that move one slot and a
+// sign, and the code for pairs next to their own costs them 4 to 20% (exact
+// t = 30 3.26 -> 3.38 ms, 512 samples of t = 40 3.43 -> 4.12 ms).
+bool tree_pairs(const InstDesc &d) { return d.pair && d.ub[1] > TREE_LEAF; }
+
 // lds_only: the stack has to stay in LDS.
 void tree_costs(InstDesc &d, TreeCosts &c, int mode, long long nrec, int simds, bool lds_only, int max_terms) {
     const int lds = mode == 0 ? TREE_LDS_WORDS0 : TREE_LDS_WORDS1;
@@ -588,9 +595,10 @@ void tree_costs(InstDesc &d, TreeCosts &c, int mode, long long nrec, int simds, 
     for (int g = 0; g <= top; g++) {
         if (g > 0) {
             if (d.ub[g] > 32 || (1ll << g) > max_terms) break;
-            if (d.ub[g] > TREE_LEAF) words += TREE_STATE_WORDS + d.ub[g];
+            const bool pair = g == 1 && tree_pairs(d);
+            if (d.ub[g] > TREE_LEAF && !pair) words += TREE_STATE_WORDS + d.ub[g];
             if (lds_only && words > lds) break;
-            below += steps(d.ub[g - 1], d.ub[g]) / (double)(1ll << (g - 1));
+            below += pair ? 0.5 * steps(0, d.ub[1]) : steps(d.ub[g - 1], d.ub[g]) / (double)(1ll << (g - 1));
         }
         const double W = (below + 60.0) * (double)(1ll << g) + steps(d.ub[g], d.n) + 500.0;
         const double lanes = (double)nrec * (double)(d.chi >> g) * (mode == 0 ? 1.0 : 0.5);
@@ -605,11 +613,14 @@ void set_tree(InstDesc &d, int mode, long long nrec, int G) {
     const int lds = mode == 0 ? TREE_LDS_WORDS0 : TREE_LDS_WORDS1;
     d.G = G;
     int words = 0;
-    d.nlds = d.leaf = d.beyond = 0;
+    const bool pairs = tree_pairs(d);
+    d.nlds = d.leaf = d.beyond = d.pair = 0;
     for (int g = 1; g <= d.G; g++) {
         const int w = TREE_STATE_WORDS + d.ub[g];
         if (d.ub[g] <= TREE_LEAF) {
             d.leaf = d.nlds = g;
+        } else if (g == 1 && pairs) {
+            d.leaf = d.nlds = d.pair = 1;
         } else if (d.nlds == g - 1 && words + w <= lds) {
             d.soff[g] = (uint16_t)words;
             words += w;
@@ -669,15 +680,16 @@ double best_bound(const TreeCosts *c, int n) {
 uint64_t slot_word(int x) { return x < 32 ? 1ull << (31 - x) : 1ull << (95 - x); }
 
 // An instance's descriptor but for its tree, and what its trees cost.  mode 0:
-// nsamp records; mode 1: chi records.  max_terms > 0 bounds the terms of a
-// lane (the calls' chunk).
+// nsamp records; mode 1: chi records.  signs: a launch with |H^t> instances.
+// max_terms > 0 bounds the terms of a lane (the calls' chunk).
 void make_inst(InstDesc &d, TreeCosts &c, const cse_ctx *ctx, int mode, int t, int k, int exact, const uint64_t *L,
-               long long nsamp, bool lds_only, int max_terms) {
+               long long nsamp, bool signs, bool lds_only, int max_terms) {
     memset(d.ub, 0, sizeof(d.ub));
     memset(d.soff, 0, sizeof(d.soff));
     d.n = t;
     d.k = exact ? (t + 1) / 2 : k;
     d.exact = exact ? 1 : 0;
+    d.pair = signs ? 0 : 1;
     d.chi = 1ll << d.k;
     uint8_t col[64];
     if (exact) {
@@ -1035,10 +1047,11 @@ static int sampled_batch(cse_ctx *ctx, const cse_sampled_instance *in, int ninst
     bool want_terms = false;
     for (int i = 0; i < ninst; i++) want_terms = want_terms || res[i].terms != nullptr;
     std::vector<TreeCosts> costs((size_t)ninst);
+    const bool signs = std::any_of(in, in + ninst, [](const auto &v) { return v.exact != 0; });
     run_ranges(ninst, [&](int lo, int hi) {
         for (int i = lo; i < hi; i++) {
             make_inst(pl.inst[i], costs[(size_t)i], ctx, 0, in[i].P.nqubits, in[i].k, in[i].exact, in[i].L,
-                      in[i].count, false, chunk);
+                      in[i].count, signs, false, chunk);
             pl.inst[i].seed = in[i].seed;
             pl.inst[i].first = in[i].first;
             to_dev(pl.projs[i], &in[i].P, in[i].exact != 0);
@@ -1167,10 +1180,11 @@ static int exact_batch(cse_ctx *ctx, const cse_instance *in, int ninst, int chun
     TreeCosts one;
     std::vector<TreeCosts> many((size_t)(ninst > 1 ? ninst : 0));
     TreeCosts *const costs = ninst > 1 ? many.data() : &one;
+    const bool signs = std::any_of(in, in + ninst, [](const auto &v) { return v.exact != 0; });
     run_ranges(ninst, [&](int lo, int hi) {
         for (int i = lo; i < hi; i++) {
-            make_inst(pl.inst[i], costs[i], ctx, 1, in[i].P.nqubits, in[i].k, in[i].exact, in[i].L, 0, use_static,
-                      chunk);
+            make_inst(pl.inst[i], costs[i], ctx, 1, in[i].P.nqubits, in[i].k, in[i].exact, in[i].L, 0, signs,
+                      use_static, chunk);
             to_dev(pl.projs[i], &in[i].P, in[i].exact != 0);
         }
     });

@@ -62,9 +62,9 @@ struct InstDesc {
     uint64_t seed;      // mode 0: Philox key of the random states
     long long first;    // mode 0: sample index of the first record
     int nlds;           // levels 1 .. nlds of the stack are in LDS
-    int leaf;           // levels up to this one only move the looked-up slots
+    int leaf;           // levels up to this one only move the looked-up slots, or pair
     int beyond;         // stack words (per lane) outside LDS
-    int spare;
+    int pair;           // leaf is 1, and the terms of index bit 0 are summed in pairs
     uint8_t inv[64];    // column of each slot
     uint8_t ub[TREE_MAXG + 4];    // ub[g]: slots that index bits below g move
     uint16_t soff[TREE_MAXG + 4]; // first word of level g's part of its stack

@@ -270,6 +270,7 @@ template <int NH, bool HT, int MODE> DEV void sweep_body(const SweepArgs &A) {
         const int v_lp = (int)(unsigned)w_lp, v_lt = (int)(unsigned)w_lt;
         const int v_lev = (int)A.inst[inst].ub[gl] | (int)A.inst[inst].soff[gl] << 8;
         const int nlds = D->nlds, leaf = D->leaf;
+        const bool pair = !HT && D->pair;
         // the term within the lane (Gray code of t - 1), and what it toggles
         const unsigned T0 = f.T;
         unsigned gray = 0, ta = 0, tt = 0, tj = 0;
@@ -291,33 +292,9 @@ template <int NH, bool HT, int MODE> DEV void sweep_body(const SweepArgs &A) {
             sr = cr = si = ci = 0.f;
         }
         int lev = G, top = n < 32 ? n : 32;
-        int p0 = 0, m0 = 0;   // the term's exponent and phase without its leaf slots
-        for (int t = 1;; t++) {
-            if (lev >= leaf) {
-                // down from `top` to the leaf slots, saving the form at every
-                // level on the way
-                while (true) {
-                    const int w = __builtin_amdgcn_readlane(v_lev, lev);
-                    const int c = lev > leaf ? w & 0xff : TREE_LEAF;
-                    if (top > c) tree::steps<NH, HT>(f, top, c);
-                    if (lev == leaf) break;
-                    uint32_t *const st = lev <= nlds ? lst : gst;
-                    form_save(f, f.A ^ ta, c, st + 64 * (w >> 8));
-                    top = c;
-                    lev--;
-                }
-                int cnt = cnt0;
-                m0 = ph0;
-                tree::fold<HT>(f.d1, f.d2, f.A, f.T, ~(~0u << (32 - TREE_LEAF)), m0, cnt);
-                p0 = cnt - (int)f.nb;
-                m0 += 2 * (int)f.q1 + 4 * __popc(f.x2);
-            }
-            // the leaf slots from the table: phase, steps of the second kind,
-            // whether the sum is 0
-            const unsigned lf = s_leaf[tree::leaf_index<HT>(f.A, f.T, f.d1, f.d2, f.lo[1])];
-            const int p = p0 + (int)((lf >> 3) & 7u);
-            const int m = (m0 + (int)lf) & 7;
-            const bool nz = valid && (int)f.z >= 0 && lf < 128u;
+        // adds a term: its exponent and phase, whether there is one, its place
+        // within the lane and its index's low part
+        auto term = [&](int p, int m, bool nz, unsigned gy, unsigned jx) {
             if (MODE == 0) {
                 const int row = ((p & 1) << 3) | m;
                 const double s = ldexp(1.0, nz ? 32 + (p >> 1) : -2000);
@@ -328,25 +305,25 @@ template <int NH, bool HT, int MODE> DEV void sweep_body(const SweepArgs &A) {
                 const float e = ldexpf(1.f, nz ? p >> 1 : -2000);
                 kahan1(sr, cr, s_tab.f[row][0] * e);
                 kahan1(si, ci, s_tab.f[row][1] * e);
-            } else if (nz && (int)gray >= rl) {
-                const bool off = (int)gray != rl;
+            } else if (nz && (int)gy >= rl) {
+                const bool off = (int)gy != rl;
                 const int P = p - sexp;
                 kahan1(sr, cr, ldexpf(s_tab.f[((P & 1) << 3) | m][0], (P >> 1) + (off ? 1 : 0)));
                 atomicAdd(&hist[m - 8 * P], off && m == 0 ? 2u : 1u);
             }
             if (A.terms && live) {
-                long long j = jhi ^ tj;
+                long long j = jhi ^ jx;
                 int mm = m;
                 if (MODE == 0) {
                     A.terms[D->term_off + r * D->chi + j] = nz ? (-p) * 8 + mm + 1 : 0;
-                } else if ((int)gray >= rl) {
+                } else if ((int)gy >= rl) {
                     // the pair in the reference's order i <= j, with the
                     // projection's factors of record i left out:
                     // <phi_i| Pi |phi_j> is the conjugate of <phi_j| Pi |phi_i>
                     long long i = ri;
                     int pp = p;
                     if (j < i) {
-                        const long long s = i, rj = (jh << G) | (long long)gray;
+                        const long long s = i, rj = (jh << G) | (long long)gy;
                         i = j;
                         j = s;
                         mm = (8 - m) & 7;
@@ -354,6 +331,50 @@ template <int NH, bool HT, int MODE> DEV void sweep_body(const SweepArgs &A) {
                     }
                     A.terms[D->term_off + i * D->chi - i * (i - 1) / 2 + (j - i)] = nz ? (-pp) * 8 + mm + 1 : 0;
                 }
+            }
+        };
+        const int low = uni(pair ? (int)D->ub[1] : TREE_LEAF);
+        int p0 = 0, m0 = 0;   // the term's exponent and phase without its last slots
+        for (int t = 1;; t++) {
+            if (lev >= leaf) {
+                // down from `top` to the leaf slots, saving the form at every
+                // level on the way
+                while (true) {
+                    const int w = __builtin_amdgcn_readlane(v_lev, lev);
+                    const int c = w & 0xff;
+                    if (top > c) tree::steps<NH, HT>(f, top, c);
+                    if (lev == leaf) break;
+                    uint32_t *const st = lev <= nlds ? lst : gst;
+                    form_save(f, f.A ^ ta, c, st + 64 * (w >> 8));
+                    top = c;
+                    lev--;
+                }
+                int cnt = cnt0;
+                m0 = ph0;
+                tree::fold<HT>(f.d1, f.d2, f.A, f.T, ~(~0u << (32 - low)), m0, cnt);
+                p0 = cnt - (int)f.nb;
+                m0 += 2 * (int)f.q1 + 4 * __popc(f.x2);
+            }
+            if (pair) {
+                tree::PairSums s;
+                int c = low;  // (out of sight of hoisting: a register a slot)
+                asm volatile("" : "+s"(c));
+                tree::pair_sums(f, c, s);
+                const bool some = valid && (int)f.z >= 0;
+                term(p0 + s.cnt[0], (m0 + s.ph[0]) & 7, some && !s.zero[0], gray, tj);
+                gray ^= 1u;
+                ta ^= (unsigned)__builtin_amdgcn_readlane(v_lp, 0);
+                if (A.terms) tj ^= D->jmap[0];
+                term(p0 + s.cnt[1], (m0 + s.ph[1]) & 7, some && !s.zero[1], gray, tj);
+                t++;
+            } else {
+            // the leaf slots from the table: phase, steps of the second kind,
+            // whether the sum is 0
+            const unsigned lf = s_leaf[tree::leaf_index<HT>(f.A, f.T, f.d1, f.d2, f.lo[1])];
+            const int p = p0 + (int)((lf >> 3) & 7u);
+            const int m = (m0 + (int)lf) & 7;
+            const bool nz = valid && (int)f.z >= 0 && lf < 128u;
+            term(p, m, nz, gray, tj);
             }
             if (t == lg) break;
             const int g = __builtin_ctz(t);

@@ -80,6 +80,12 @@ template <u32 K> TREE_DEV void bitk2(u32 v, u32 w, u32 &r, u32 &q) {
         : "=&v"(r), "=&v"(q)
         : "v"(v), "v"(w), "n"(K));
 }
+template <u32 K> TREE_DEV void bitk4(u32 a, u32 b, u32 c, u32 d, u32 *r) {
+    asm("v_and_b32 %0, %8, %4\n\tv_and_b32 %1, %8, %5\n\tv_and_b32 %2, %8, %6\n\tv_and_b32 %3, %8, %7\n\t"
+        TREE_NZ("%0") TREE_NZ("%1") TREE_NZ("%2") TREE_NZ("%3")
+        : "=&v"(r[0]), "=&v"(r[1]), "=&v"(r[2]), "=&v"(r[3])
+        : "v"(a), "v"(b), "v"(c), "v"(d), "n"(K));
+}
 // mask of the top bit, and the next bit moved up
 TREE_DEV u32 pop_mask(u32 &t) {
     u32 m;
@@ -174,6 +180,12 @@ template <u32 K> inline u32 bitk(u32 v) { return nz1(v & K); }
 template <u32 K> inline void bitk2(u32 v, u32 w, u32 &r, u32 &q) {
     r = nz1(v & K);
     q = nz1(w & K);
+}
+template <u32 K> inline void bitk4(u32 a, u32 b, u32 c, u32 d, u32 *r) {
+    r[0] = nz1(a & K);
+    r[1] = nz1(b & K);
+    r[2] = nz1(c & K);
+    r[3] = nz1(d & K);
 }
 inline u32 pop_mask(u32 &t) {
     const u32 m = nz1(t >> 31);
@@ -377,6 +389,86 @@ template <int NH, bool HT, int C> struct StepsHi {
 template <int NH, bool HT> struct StepsHi<NH, HT, -1> {
     static TREE_DEV void run(Form<NH> &, int) {}
 };
+
+// Two terms that differ in every slot left (the lowest index bit moves just
+// these slots): the slots one of them sums are those the other drops, and a
+// dropped slot is at 0, so neither sees the other's part of J.  With J taken
+// as block diagonal, the slots of A and the others, one pass over the slots
+// gives both sums, each step being one of the term that sums its slot.  There
+// is nothing after it, so a slot that is solved for just leaves (`lv` holds
+// the slots still there, `gone` the ones that left); its D stays where the
+// constraint adds it to the phase, and the d2 of a slot of the third kind is
+// cleared, so that d2 without d1 means a sum that is 0.
+template <int NH, int C> TREE_DEV void pair_step(Form<NH> &f, u32 &lv, u32 &gone) {
+    u32 b[4];
+    bitk4<slot_bit(C)>(lv, f.d1, f.d2, f.A, b);
+    const u32 act = b[0], odd = b[1], hi = b[2];
+    lv = andk<~slot_bit(C)>(lv);
+    const u32 own = TREE_B3(lv, f.A, b[3], TA & ~(TB ^ TC));
+    const u32 v = TREE_B3(f.lo[C], own, act, TA & TB & TC), neg = 0u - v;
+    const u32 o = TREE_B3(v, neg, odd, TA & TB & ~TC);
+    const u32 bm = nz1(o);
+    u32 oddi = f.d1 & o, d2i = f.d2 & o;
+    nz2(oddi, d2i);
+    const u32 e = odd | oddi;
+    const u32 u = TREE_XA(d2i, hi, oddi);
+    const u32 h = TREE_B3(odd, hi, u, (TA & ~TB) | (~TA & TC));
+    u32 p[5];
+    picked<index_bits(C)>(o, p);
+    const u32 w = pick<C>(f.lo, p) & TREE_B3(own, bm, o, TA & TB & ~TC);
+    lv = TREE_B3(lv, o, o, TA & ~TB);
+    gone |= o;
+    const u32 vp = TREE_B3(v, o, o, TA & ~TB);
+    const u32 ev = e & vp;
+    const u32 al = w ^ ev;
+    const u32 g = TREE_XA(h, e, f.d1);
+    f.d2 = TREE_XA(f.d2, vp, g);
+    f.d2 ^= TREE_B3(w, hi, vp, TA & (TB ^ TC));
+    f.d2 = TREE_B3(f.d2, o, hi, TA & (~TB | TC));
+    const u32 third = andk<slot_bit(C)>(bm);
+    f.d2 = TREE_B3(f.d2, third, third, TA & ~TB);
+    f.d1 ^= ev;
+    f.d1 = TREE_B3(f.d1, o, hi, TA & (~TB | TC));
+    u32 tv = vp, tw = w;
+    rows<C>(f.lo, tv, tw, al, vp);
+}
+template <int NH, int C, int N> struct PairSteps {
+    static TREE_DEV void run(Form<NH> &f, u32 todo, u32 &lv, u32 &gone) {
+        if (N <= 2 || (todo & (((1u << N) - 1u) << C))) {
+            PairSteps<NH, C + N / 2, N / 2>::run(f, todo, lv, gone);
+            PairSteps<NH, C, N / 2>::run(f, todo, lv, gone);
+        }
+    }
+};
+template <int NH, int C> struct PairSteps<NH, C, 1> {
+    static TREE_DEV void run(Form<NH> &f, u32 todo, u32 &lv, u32 &gone) {
+        if (C > 0 && (todo & (1u << C))) pair_step<NH, (C > 0 ? C : 1)>(f, lv, gone);
+    }
+};
+// The slots below c, 1 <= c <= 32, of both terms: phases and counts as in
+// fold, without a sum where zero is not 0; [0] of the term that sums A.
+struct PairSums {
+    int ph[2], cnt[2];
+    u32 zero[2];
+};
+template <int NH> TREE_DEV void pair_sums(Form<NH> &f, int c, PairSums &s) {
+    const u32 todo = ~0u >> (32 - c), in = ~0u << (32 - c);
+    u32 lv = in, gone = 0;
+    PairSteps<NH, 16, 16>::run(f, todo, lv, gone);
+    PairSteps<NH, 0, 16>::run(f, todo, lv, gone);
+    const u32 odd = TREE_B3(in & f.d1, gone, gone, TA & ~TB);        // first kind
+    const u32 two = in & TREE_B3(f.d1, f.d2, gone, TA & (TB | TC));  // 2 each
+    const u32 four = in & TREE_B3(f.d2, f.d1, gone, TA & (TB | TC)); // 4 each
+    const u32 none = TREE_B3(in & f.d2, f.d1, gone, TA & ~TB & ~TC); // sums that are 0
+#pragma unroll
+    for (int k = 0; k < 2; k++) {
+        const u32 m = in & (k ? ~f.A : f.A);
+        const int na = TREE_POP(odd & m);
+        s.cnt[k] = TREE_POP(m) - na - 2 * TREE_POP(gone & m);
+        s.ph[k] = na + 2 * TREE_POP(two & m) + 4 * TREE_POP(four & m);
+        s.zero[k] = none & m;
+    }
+}
 
 // What finished slots give, those of `in` of a word's 32: phase in units of 1
 // and the count of active slots less the steps of the first kind; the third

@@ -44,6 +44,19 @@ template <int NH, bool HT> static void go(int n, const uint64_t *row, const uint
     out[1] = cnt - (int)f.nb - n;
     out[2] = (ph + 2 * (int)f.q1 + 4 * TREE_POP(f.x2)) & 7;
 }
+extern "C" void pair_eval(int c, const uint64_t *row, const uint64_t *w, int *out) {
+    Form<0> f;
+    memset(&f, 0, sizeof f);
+    for (int x = 0; x < c; x++) f.lo[x] = (u32)row[x];
+    f.d1 = (u32)w[0]; f.d2 = (u32)w[1]; f.A = (u32)w[2];
+    PairSums s;
+    pair_sums(f, c, s);
+    for (int k = 0; k < 2; k++) {
+        out[3 * k] = s.zero[k] ? 0 : 1;
+        out[3 * k + 1] = s.cnt[k];
+        out[3 * k + 2] = s.ph[k] & 7;
+    }
+}
 extern "C" void tree_eval(int nh, int ht, int n, const uint64_t *row, const uint64_t *w, int *out) {
     if (nh == 0) ht ? go<0, true>(n, row, w, out) : go<0, false>(n, row, w, out);
     else if (nh == 16) ht ? go<16, true>(n, row, w, out) : go<16, false>(n, row, w, out);
@@ -119,6 +132,40 @@ def test_form_sums_match_brute_force(tree, nh, n, signs):
         # the n - nv empty slots are pivots without a sum: 2^{-1/2} each
         got = out[0] * 2.0 ** ((out[1] + n - nv) / 2) * cmath.exp(1j * math.pi * out[2] / 4)
         assert abs(got - brute(J, d1, d2, A, F, T)) <= 1e-9
+
+
+@pytest.mark.parametrize("c", [1, 2, 3, 4, 5, 8, 9, 12, 16, 17, 18, 31, 32])
+def test_two_complementary_terms_match_brute_force(tree, c):
+    # up to 9 coupled slots, on both sides of the cut, among the c
+    rnd = random.Random(77 * c)
+    for _ in range(300):
+        nv = min(c, rnd.randint(1, 9))
+        pos = sorted(rnd.sample(range(c), nv))
+        dens = rnd.random()
+        J = [0] * nv
+        for a in range(nv):
+            for b in range(a):
+                if rnd.random() < dens:
+                    J[a] |= 1 << b
+                    J[b] |= 1 << a
+        d1, d2, A = (rnd.getrandbits(nv) for _ in range(3))
+        if rnd.random() < 0.5:
+            d1 = 0
+
+        def up(v):
+            return sum((v >> i & 1) << p for i, p in enumerate(pos))
+
+        rows = (ctypes.c_uint64 * 64)()
+        for i, p in enumerate(pos):
+            rows[p] = words(up(J[i]))
+        out = (ctypes.c_int * 6)()
+        tree.pair_eval(c, rows, (ctypes.c_uint64 * 4)(*[words(up(v)) for v in (d1, d2, A, 0)]), out)
+        for k in range(2):
+            a = ~A & ((1 << nv) - 1) if k else A
+            # the c - nv empty slots: 2^{-1/2} each where dropped, 1 where summed
+            got = out[3 * k] * 2.0 ** ((out[3 * k + 1] - c) / 2) * cmath.exp(1j * math.pi * out[3 * k + 2] / 4)
+            want = brute(J, d1, d2, a, 0, 0) * (1.0 if k else 2.0 ** (-(c - nv) / 2))
+            assert abs(got - want) <= 1e-9
 
 
 @pytest.mark.parametrize("t,k", [(1, 0), (1, 1), (2, 3), (13, 5), (24, 11), (48, 12), (64, 14), (60, 20)])
