@@ -580,7 +580,15 @@ struct TreeCosts {
 // (d.pair as make_inst leaves it): those have bits that move one slot and a
 // sign, and the code for pairs next to their own costs them 4 to 20% (exact
 // t = 30 3.26 -> 3.38 ms, 512 samples of t = 40 3.43 -> 4.12 ms).
-bool tree_pairs(const InstDesc &d) { return d.pair && d.ub[1] > TREE_LEAF; }
+bool tree_pairs(const InstDesc &d) { return d.pair && d.ub[1] > TREE_LEAF && d.ub[1] <= 32; }
+
+// Levels of a tree have at most 32 slots, but in launches with states of more
+// than 48 and no |H^t> instances (whose bits move two slots at a time: none
+// gets that far): 8192 samples of t = 63, k = 10 1.26 -> 0.86 ms, 4096 of t =
+// 56, k = 12 1.26 -> 0.98 ms (means of four).  The kernel of 33 to 48 slots
+// has 128 registers, and with the code for such levels in it 2^28 terms of t =
+// 48 take 10.0 -> 10.6 ms and 2000 samples of t = 37 101 -> 108 us.
+int tree_levels(int nmax, bool signs) { return nmax > 48 && !signs ? 64 : 32; }
 
 // lds_only: the stack has to stay in LDS.
 void tree_costs(InstDesc &d, TreeCosts &c, int mode, long long nrec, int simds, bool lds_only, int max_terms) {
@@ -594,9 +602,9 @@ void tree_costs(InstDesc &d, TreeCosts &c, int mode, long long nrec, int simds, 
     double below = 0.0;  // steps of the slots below ub[g], per term
     for (int g = 0; g <= top; g++) {
         if (g > 0) {
-            if (d.ub[g] > 32 || (1ll << g) > max_terms) break;
+            if (d.ub[g] > d.levels || (1ll << g) > max_terms) break;
             const bool pair = g == 1 && tree_pairs(d);
-            if (d.ub[g] > TREE_LEAF && !pair) words += TREE_STATE_WORDS + d.ub[g];
+            if (d.ub[g] > TREE_LEAF && !pair) words += tree_words(d.ub[g]);
             if (lds_only && words > lds) break;
             below += pair ? 0.5 * steps(0, d.ub[1]) : steps(d.ub[g - 1], d.ub[g]) / (double)(1ll << (g - 1));
         }
@@ -616,7 +624,7 @@ void set_tree(InstDesc &d, int mode, long long nrec, int G) {
     const bool pairs = tree_pairs(d);
     d.nlds = d.leaf = d.beyond = d.pair = 0;
     for (int g = 1; g <= d.G; g++) {
-        const int w = TREE_STATE_WORDS + d.ub[g];
+        const int w = tree_words(d.ub[g]);
         if (d.ub[g] <= TREE_LEAF) {
             d.leaf = d.nlds = g;
         } else if (g == 1 && pairs) {
@@ -680,16 +688,18 @@ double best_bound(const TreeCosts *c, int n) {
 uint64_t slot_word(int x) { return x < 32 ? 1ull << (31 - x) : 1ull << (95 - x); }
 
 // An instance's descriptor but for its tree, and what its trees cost.  mode 0:
-// nsamp records; mode 1: chi records.  signs: a launch with |H^t> instances.
+// nsamp records; mode 1: chi records.  signs: a launch with |H^t> instances;
+// levels: tree_levels of the launch.
 // max_terms > 0 bounds the terms of a lane (the calls' chunk).
 void make_inst(InstDesc &d, TreeCosts &c, const cse_ctx *ctx, int mode, int t, int k, int exact, const uint64_t *L,
-               long long nsamp, bool signs, bool lds_only, int max_terms) {
+               long long nsamp, bool signs, int levels, bool lds_only, int max_terms) {
     memset(d.ub, 0, sizeof(d.ub));
     memset(d.soff, 0, sizeof(d.soff));
     d.n = t;
     d.k = exact ? (t + 1) / 2 : k;
     d.exact = exact ? 1 : 0;
     d.pair = signs ? 0 : 1;
+    d.levels = levels;
     d.chi = 1ll << d.k;
     uint8_t col[64];
     if (exact) {
@@ -1047,11 +1057,17 @@ static int sampled_batch(cse_ctx *ctx, const cse_sampled_instance *in, int ninst
     bool want_terms = false;
     for (int i = 0; i < ninst; i++) want_terms = want_terms || res[i].terms != nullptr;
     std::vector<TreeCosts> costs((size_t)ninst);
-    const bool signs = std::any_of(in, in + ninst, [](const auto &v) { return v.exact != 0; });
+    bool signs = false;
+    int nmax = 0;
+    for (int i = 0; i < ninst; i++) {
+        signs = signs || in[i].exact;
+        nmax = std::max(nmax, in[i].P.nqubits);
+    }
+    const int levels = tree_levels(nmax, signs);
     run_ranges(ninst, [&](int lo, int hi) {
         for (int i = lo; i < hi; i++) {
             make_inst(pl.inst[i], costs[(size_t)i], ctx, 0, in[i].P.nqubits, in[i].k, in[i].exact, in[i].L,
-                      in[i].count, signs, false, chunk);
+                      in[i].count, signs, levels, false, chunk);
             pl.inst[i].seed = in[i].seed;
             pl.inst[i].first = in[i].first;
             to_dev(pl.projs[i], &in[i].P, in[i].exact != 0);
@@ -1180,11 +1196,17 @@ static int exact_batch(cse_ctx *ctx, const cse_instance *in, int ninst, int chun
     TreeCosts one;
     std::vector<TreeCosts> many((size_t)(ninst > 1 ? ninst : 0));
     TreeCosts *const costs = ninst > 1 ? many.data() : &one;
-    const bool signs = std::any_of(in, in + ninst, [](const auto &v) { return v.exact != 0; });
+    bool signs = false;
+    int nmax = 0;
+    for (int i = 0; i < ninst; i++) {
+        signs = signs || in[i].exact;
+        nmax = std::max(nmax, in[i].P.nqubits);
+    }
+    const int levels = tree_levels(nmax, signs);
     run_ranges(ninst, [&](int lo, int hi) {
         for (int i = lo; i < hi; i++) {
             make_inst(pl.inst[i], costs[i], ctx, 1, in[i].P.nqubits, in[i].k, in[i].exact, in[i].L, 0, signs,
-                      use_static, chunk);
+                      levels, use_static, chunk);
             to_dev(pl.projs[i], &in[i].P, in[i].exact != 0);
         }
     });

@@ -289,9 +289,9 @@ static uint64_t lightest(const uint64_t *w, int m, uint64_t U, uint32_t *best) {
 
 /* Combinations are searched among at most this many rows at a time. */
 #define CHAIN_SEARCH 12
-/* ... and no more once this many columns have moved: a tree has no levels of
- * its own beyond 32 slots. */
-#define CHAIN_MOVED 32
+/* ... and no more once this many columns have moved: levels so wide are
+ * entered too rarely to matter. */
+#define CHAIN_MOVED 48
 
 void cse_chain_basis(int t, int k, const uint64_t *L, int levels, uint64_t *rows, uint32_t *jmap, uint8_t *ub,
                      uint8_t *col) {

@@ -40,8 +40,11 @@ inline __host__ __device__ long long tri_before(long long ch, long long nch, lon
 // blocks of four waves on a CU (160 KB), next to the exact sweep's histogram
 #define TREE_LDS_WORDS0 38
 #define TREE_LDS_WORDS1 34
-// words of a saved form besides its rows
+// words of a saved form besides its rows, those it has beyond 32 slots, and all
+// of one on c slots
 #define TREE_STATE_WORDS 5
+#define TREE_HIGH_WORDS 3
+constexpr int tree_words(int c) { return TREE_STATE_WORDS + (c <= 32 ? c : TREE_HIGH_WORDS + 2 * c - 32); }
 
 // largest flush_terms (and the default): 2^30 terms keep every 32-bit bin
 // below 2^32
@@ -64,6 +67,8 @@ struct InstDesc {
     int nlds;           // levels 1 .. nlds of the stack are in LDS
     int leaf;           // levels up to this one only move the looked-up slots, or pair
     int beyond;         // stack words (per lane) outside LDS
+    int levels;         // most slots of a level (tree_levels)
+    int spare;
     int pair;           // leaf is 1, and the terms of index bit 0 are summed in pairs
     uint8_t inv[64];    // column of each slot
     uint8_t ub[TREE_MAXG + 4];    // ub[g]: slots that index bits below g move

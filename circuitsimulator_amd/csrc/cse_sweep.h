@@ -94,6 +94,36 @@ template <int NH> DEV void form_load(tree::Form<NH> &f, int c, const uint32_t *p
     f.nb = w & 0xffu;
     rows_load<NH, 0>(f, c, p);
 }
+// the rest of a form on c > 32 slots, after the first 32 rows
+constexpr int kHigh = TREE_STATE_WORDS + 32;
+template <int NH, int X> DEV void rows_save_high(const tree::Form<NH> &f, int c, uint32_t *p) {
+    if constexpr (X < NH) {
+        if (c <= 32 + X) return;
+        p[64 * (kHigh + TREE_HIGH_WORDS + 2 * X)] = f.lo[32 + X];
+        p[64 * (kHigh + TREE_HIGH_WORDS + 2 * X + 1)] = f.hi[X];
+        rows_save_high<NH, X + 1>(f, c, p);
+    }
+}
+template <int NH> DEV void form_save_high(const tree::Form<NH> &f, unsigned a, int c, uint32_t *p) {
+    p[64 * kHigh] = f.d1h;
+    p[64 * (kHigh + 1)] = f.d2h;
+    p[64 * (kHigh + 2)] = a;
+    rows_save_high<NH, 0>(f, c, p);
+}
+template <int NH> DEV void form_load_high(tree::Form<NH> &f, int c, const uint32_t *p) {
+    f.d1h = p[64 * kHigh];
+    f.d2h = p[64 * (kHigh + 1)];
+    f.Ah = p[64 * (kHigh + 2)];
+#pragma unroll
+    for (int x = 0; x < NH; x++) {
+        // (every row gets a value, so none has to be kept from before)
+        f.lo[32 + x] = f.hi[x] = 0;
+        if (c > 32 + x) {
+            f.lo[32 + x] = p[64 * (kHigh + TREE_HIGH_WORDS + 2 * x)];
+            f.hi[x] = p[64 * (kHigh + TREE_HIGH_WORDS + 2 * x + 1)];
+        }
+    }
+}
 
 // What a term adds, by (p odd) 8 + m: 2^{(p odd)/2} w^m in the basis 1, w,
 // w^2, w^3 and as an FP32 pair, to be scaled by 2^{p >> 1}.
@@ -136,6 +166,8 @@ struct TermTables {
 // moves to another one and at its exit.  NH: slots beyond 32 (n <= 32 + NH).
 // HT: some instance has |H^t> terms.
 template <int NH, bool HT, int MODE> DEV void sweep_body(const SweepArgs &A) {
+    // levels beyond 32 slots: only where instances may have them (tree_levels)
+    constexpr bool DEEP = NH > 16 && !HT;
     constexpr int LW = MODE == 0 ? TREE_LDS_WORDS0 : TREE_LDS_WORDS1;
     __shared__ uint32_t lstack[4][LW * 64];
     __shared__ unsigned int hist[MODE == 1 ? HIST_STRIDE : 1];
@@ -260,20 +292,20 @@ template <int NH, bool HT, int MODE> DEV void sweep_body(const SweepArgs &A) {
                 }
             }
         int ph0 = (int)((w0 >> 16) & 7), cnt0 = -n;
-        if (NH > 0) {
+        if (NH > 0 && !DEEP) {
             tree::StepsHi<NH, HT, NH - 1>::run(f, n);
             tree::fold<HT>(f.d1h, f.d2h, f.Ah, f.Th, ~0u, ph0, cnt0);
         }
         // by index bit g (in lane g): the slots it toggles, their signs, the
         // index j; by level: slots and place of the saved form
         const int gl = x < TREE_MAXG ? x : TREE_MAXG;
-        const int v_lp = (int)(unsigned)w_lp, v_lt = (int)(unsigned)w_lt;
+        const int v_lp = (int)(unsigned)w_lp, v_lph = (int)(unsigned)(w_lp >> 32), v_lt = (int)(unsigned)w_lt;
         const int v_lev = (int)A.inst[inst].ub[gl] | (int)A.inst[inst].soff[gl] << 8;
         const int nlds = D->nlds, leaf = D->leaf;
         const bool pair = !HT && D->pair;
         // the term within the lane (Gray code of t - 1), and what it toggles
         const unsigned T0 = f.T;
-        unsigned gray = 0, ta = 0, tt = 0, tj = 0;
+        unsigned gray = 0, ta = 0, tah = 0, tt = 0, tj = 0;
         // MODE 1: the lane's block holds the diagonal at term rl
         const int rl = MODE == 1 && jh == (r >> G) ? (int)(r & (lg - 1)) : -1;
         unsigned jhi = 0, ri = 0;
@@ -291,7 +323,6 @@ template <int NH, bool HT, int MODE> DEV void sweep_body(const SweepArgs &A) {
             c0 = c1 = c2 = c3 = 0.0;
             sr = cr = si = ci = 0.f;
         }
-        int lev = G, top = n < 32 ? n : 32;
         // adds a term: its exponent and phase, whether there is one, its place
         // within the lane and its index's low part
         auto term = [&](int p, int m, bool nz, unsigned gy, unsigned jx) {
@@ -335,68 +366,95 @@ template <int NH, bool HT, int MODE> DEV void sweep_body(const SweepArgs &A) {
         };
         const int low = uni(pair ? (int)D->ub[1] : TREE_LEAF);
         int p0 = 0, m0 = 0;   // the term's exponent and phase without its last slots
-        for (int t = 1;; t++) {
-            if (lev >= leaf) {
-                // down from `top` to the leaf slots, saving the form at every
-                // level on the way
+        int t = 1, lev = G, top = DEEP || n < 32 ? n : 32;
+        while (true) {
+            if (DEEP && top > 32) {
+                // the levels beyond 32 slots, and what their slots give
                 while (true) {
                     const int w = __builtin_amdgcn_readlane(v_lev, lev);
                     const int c = w & 0xff;
-                    if (top > c) tree::steps<NH, HT>(f, top, c);
-                    if (lev == leaf) break;
-                    uint32_t *const st = lev <= nlds ? lst : gst;
-                    form_save(f, f.A ^ ta, c, st + 64 * (w >> 8));
+                    tree::StepsHi<NH, HT, NH - 1>::run(f, top, c);
+                    if (c <= 32) break;
+                    uint32_t *const st = gst + 64 * (w >> 8);
+                    form_save(f, f.A ^ ta, c, st);
+                    form_save_high(f, f.Ah ^ tah, c, st);
                     top = c;
                     lev--;
                 }
-                int cnt = cnt0;
-                m0 = ph0;
-                tree::fold<HT>(f.d1, f.d2, f.A, f.T, ~(~0u << (32 - low)), m0, cnt);
-                p0 = cnt - (int)f.nb;
-                m0 += 2 * (int)f.q1 + 4 * __popc(f.x2);
+                ph0 = (int)((w0 >> 16) & 7);
+                cnt0 = -n;
+                tree::fold<HT>(f.d1h, f.d2h, f.Ah, f.Th, ~0u, ph0, cnt0);
+                top = 32;
             }
-            if (pair) {
-                tree::PairSums s;
-                int c = low;  // (out of sight of hoisting: a register a slot)
-                asm volatile("" : "+s"(c));
-                tree::pair_sums(f, c, s);
-                const bool some = valid && (int)f.z >= 0;
-                term(p0 + s.cnt[0], (m0 + s.ph[0]) & 7, some && !s.zero[0], gray, tj);
-                gray ^= 1u;
-                ta ^= (unsigned)__builtin_amdgcn_readlane(v_lp, 0);
-                if (A.terms) tj ^= D->jmap[0];
-                term(p0 + s.cnt[1], (m0 + s.ph[1]) & 7, some && !s.zero[1], gray, tj);
-                t++;
-            } else {
-            // the leaf slots from the table: phase, steps of the second kind,
-            // whether the sum is 0
-            const unsigned lf = s_leaf[tree::leaf_index<HT>(f.A, f.T, f.d1, f.d2, f.lo[1])];
-            const int p = p0 + (int)((lf >> 3) & 7u);
-            const int m = (m0 + (int)lf) & 7;
-            const bool nz = valid && (int)f.z >= 0 && lf < 128u;
-            term(p, m, nz, gray, tj);
+            while (true) {
+                if (lev >= leaf) {
+                    // down from `top` to the leaf slots, saving the form at every
+                    // level on the way
+                    while (true) {
+                        const int w = __builtin_amdgcn_readlane(v_lev, lev);
+                        const int c = w & 0xff;
+                        if (top > c) tree::steps<NH, HT>(f, top, c);
+                        if (lev == leaf) break;
+                        uint32_t *const st = lev <= nlds ? lst : gst;
+                        form_save(f, f.A ^ ta, c, st + 64 * (w >> 8));
+                        top = c;
+                        lev--;
+                    }
+                    int cnt = cnt0;
+                    m0 = ph0;
+                    tree::fold<HT>(f.d1, f.d2, f.A, f.T, ~(~0u << (32 - low)), m0, cnt);
+                    p0 = cnt - (int)f.nb;
+                    m0 += 2 * (int)f.q1 + 4 * __popc(f.x2);
+                }
+                if (pair) {
+                    tree::PairSums s;
+                    int c = low;  // (out of sight of hoisting: a register a slot)
+                    asm volatile("" : "+s"(c));
+                    tree::pair_sums(f, c, s);
+                    const bool some = valid && (int)f.z >= 0;
+                    term(p0 + s.cnt[0], (m0 + s.ph[0]) & 7, some && !s.zero[0], gray, tj);
+                    gray ^= 1u;
+                    ta ^= (unsigned)__builtin_amdgcn_readlane(v_lp, 0);
+                    if (A.terms) tj ^= D->jmap[0];
+                    term(p0 + s.cnt[1], (m0 + s.ph[1]) & 7, some && !s.zero[1], gray, tj);
+                    t++;
+                } else {
+                    // the leaf slots from the table: phase, steps of the second
+                    // kind, whether the sum is 0
+                    const unsigned lf = s_leaf[tree::leaf_index<HT>(f.A, f.T, f.d1, f.d2, f.lo[1])];
+                    term(p0 + (int)((lf >> 3) & 7u), (m0 + (int)lf) & 7, valid && (int)f.z >= 0 && lf < 128u, gray,
+                         tj);
+                }
+                if (t == lg) goto summed;
+                const int g = __builtin_ctz(t++);
+                gray ^= 1u << g;
+                if (A.terms) tj ^= D->jmap[g];
+                const unsigned la = (unsigned)__builtin_amdgcn_readlane(v_lp, g);
+                const unsigned lt = HT ? (unsigned)__builtin_amdgcn_readlane(v_lt, g) : 0u;
+                ta ^= la;
+                tt ^= lt;
+                if (DEEP) tah ^= (unsigned)__builtin_amdgcn_readlane(v_lph, g);
+                lev = g;
+                if (g < leaf) {
+                    // only leaf slots change
+                    f.A ^= la;
+                    if (HT) f.T ^= lt;
+                } else {
+                    const int w = __builtin_amdgcn_readlane(v_lev, g + 1);
+                    top = w & 0xff;
+                    if (DEEP && top > 32) break;
+                    form_load(f, top, (g + 1 <= nlds ? lst : gst) + 64 * (w >> 8));
+                    f.A ^= ta;
+                    if (HT) f.T = T0 ^ tt;
+                }
             }
-            if (t == lg) break;
-            const int g = __builtin_ctz(t);
-            gray ^= 1u << g;
-            if (A.terms) tj ^= D->jmap[g];
-            const unsigned la = (unsigned)__builtin_amdgcn_readlane(v_lp, g);
-            const unsigned lt = HT ? (unsigned)__builtin_amdgcn_readlane(v_lt, g) : 0u;
-            ta ^= la;
-            tt ^= lt;
-            lev = g;
-            if (g < leaf) {
-                // only leaf slots change
-                f.A ^= la;
-                if (HT) f.T ^= lt;
-            } else {
-                const int w = __builtin_amdgcn_readlane(v_lev, g + 1);
-                top = w & 0xff;
-                form_load(f, top, (g + 1 <= nlds ? lst : gst) + 64 * (w >> 8));
-                f.A ^= ta;
-                if (HT) f.T = T0 ^ tt;
-            }
+            const uint32_t *const st = gst + 64 * (__builtin_amdgcn_readlane(v_lev, lev + 1) >> 8);
+            form_load(f, top, st);
+            form_load_high(f, top, st);
+            f.A ^= ta;
+            f.Ah ^= tah;
         }
+    summed:
         if (MODE == 0) {
             if (valid) ips += (unsigned long long)lg;
             // the record's sums over the lanes that share it (integers below

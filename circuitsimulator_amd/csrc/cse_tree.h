@@ -380,14 +380,15 @@ template <int NH, bool HT> TREE_DEV void steps(Form<NH> &f, int c0, int c1) {
     Steps<NH, HT, 16, 16>::run(f, todo);
     Steps<NH, HT, 0, 16>::run(f, todo);
 }
+// Steps of the slots c0 - 1 .. c1 that are 32 or more.
 template <int NH, bool HT, int C> struct StepsHi {
-    static TREE_DEV void run(Form<NH> &f, int c0) {
-        if (c0 > 32 + C) step_hi<NH, HT, C>(f);
-        StepsHi<NH, HT, C - 1>::run(f, c0);
+    static TREE_DEV void run(Form<NH> &f, int c0, int c1 = 32) {
+        if (c0 > 32 + C && c1 <= 32 + C) step_hi<NH, HT, C>(f);
+        StepsHi<NH, HT, C - 1>::run(f, c0, c1);
     }
 };
 template <int NH, bool HT> struct StepsHi<NH, HT, -1> {
-    static TREE_DEV void run(Form<NH> &, int) {}
+    static TREE_DEV void run(Form<NH> &, int, int = 32) {}
 };
 
 // Two terms that differ in every slot left (the lowest index bit moves just

@@ -247,3 +247,42 @@ def test_every_exact_term_at_the_kernels_widths(E, t, k, exact):
         print(f"exact t={t} k={k} exact={exact} chunk={chunk}", flush=True)
         _, terms, _ = E.batch_exact([inst], chunk=chunk, want_terms=True, nterms=nl)
         assert want == list(terms)
+
+
+# levels beyond 32 slots: rows that reach them one, two and many slots at a
+# time, next to narrower instances in the same launch
+@pytest.mark.gpu
+@pytest.mark.parametrize("t,steps", [(49, [30, 2, 1, 16]), (56, [8, 20, 10, 9, 8]), (64, [33, 1, 15, 15]),
+                                     (63, [3, 28, 1, 1, 17]), (64, [2, 40, 21])])
+def test_levels_beyond_32_slots(E, t, steps):
+    from circuitsimulator_amd.engine import Instance, Projector
+    rng = np.random.default_rng(41 * t + len(steps))
+    order = rng.permutation(t)
+    L, at = [], 0
+    for s in steps:
+        # s new columns and some of the ones before
+        L.append(sum(1 << int(q) for q in order[at:at + s]) ^ (orc.rand_bits(rng, t) & sum(1 << int(q) for q in order[:at])))
+        at += s
+    k = len(L)
+    ph, xs, zs = random_commuting_projector(rng, t, t // 3)
+    se, zsum, terms = oracle_sampled(t, k, L, 0, ph, xs, zs, 5, 0, 3, 1 << k)
+    P = Projector.make(ph, xs, zs, t)
+    for chunk in (0, 4, 1 << k):
+        print(f"t={t} steps={steps} chunk={chunk}", flush=True)
+        _, ex = E.sampled_projector(P, L, k, 0, 5, 0, 3, chunk=chunk, want_terms=True)
+        assert np.array_equal(ex["sexp"], se)
+        assert np.array_equal(ex["terms"], terms)
+        assert np.array_equal(ex["zsum"], zsum)
+    inst, want = [], []
+    for n, rows in ((t, L), (9, [3, 500, 77])):
+        i = Instance()
+        p = (ph, xs, zs) if n == t else random_commuting_projector(rng, n, 3)
+        i.P = Projector.make(*p, n)
+        i.exact, i.k = 0, len(rows)
+        for q, v in enumerate(rows):
+            i.L[q] = v
+        inst.append(i)
+        want += [w[0] for w in oracle_exact_terms(n, len(rows), rows, 0, *p)]
+    for chunk in (0, 1 << k):
+        _, got, _ = E.batch_exact(inst, chunk=chunk, want_terms=True, nterms=len(want))
+        assert want == list(got)
