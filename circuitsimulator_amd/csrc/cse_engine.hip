@@ -48,7 +48,6 @@ struct cse_ctx {
     // a batch's results (sums, Kahan pairs, histograms, counts, error flag) in
     // one allocation, laid out as the pinned stage they are copied into
     DevBuf outb;
-    size_t out_bytes = 0;
     long long *d_zsum = nullptr;
     double *d_kahan = nullptr;
     unsigned long long *d_hist = nullptr, *d_ips = nullptr;
@@ -248,6 +247,7 @@ struct Plan {
     long long stack_words = 0;  // per lane and wave, beyond LDS
     int nmax = 0;
     bool anyH = false;
+    bool values = false;  // exact mode: sums go to the host, not histograms
     // counts the instances, whose descriptors are complete but for their
     // offsets: instance i has nr(i) records and nt(i) terms
     template <class R, class T> void finish(int n, R &&nr, T &&nt) {
@@ -323,12 +323,18 @@ int run_records(cse_ctx *ctx, const Plan &pl, int mode) {
 }
 
 // Layout of a batch's results block, the same on the device and in the
-// pinned stage.  Sampled mode (0): per-sample Z[omega] sums (32 B), Kahan
-// pairs (16 B) and projection exponents (4 B), then per-instance counts and
-// the error flag.  Exact mode (1): per-instance histograms, Kahan pairs and
-// counts, then the error flag; both end with the clock readings.
+// pinned stage, but for the exact mode's sums, which the device has no room
+// for, and its histograms where only their sums are wanted, which stay there.
+// Sampled mode (0): per-sample Z[omega] sums (32 B), Kahan pairs (16 B) and
+// projection exponents (4 B), then per-instance counts and the error flag.
+// Exact mode (1): per-instance histograms or sums (Plan::values), Kahan pairs
+// and counts, then the error flag; both end with the clock readings.  (With
+// the histograms after the counts, their atomics in one cache line with those
+// of the counts, 2^22 terms of one instance take 3 us more.)
 struct OutLayout {
-    size_t zsum, kahan, sexp, hist, ips, err, clock, total;
+    size_t vals, zsum, kahan, sexp, hist, ips, err, clock;
+    size_t copied;  // the end of what comes back
+    size_t total;
 };
 
 OutLayout out_layout(const Plan &pl, int mode) {
@@ -340,16 +346,17 @@ OutLayout out_layout(const Plan &pl, int mode) {
         o.kahan = 32 * n;
         o.sexp = 48 * n;
         o.ips = (52 * n + 7) & ~(size_t)7;
-        o.err = o.ips + 8 * ni;
     } else {
-        const size_t nh = (size_t)HIST_STRIDE * ni;
-        o.hist = 0;
-        o.kahan = 8 * nh;
+        o.kahan = pl.values ? 64 * ni : 8 * (size_t)HIST_STRIDE * ni;
         o.ips = o.kahan + 16 * ni;
-        o.err = o.ips + 8 * ni;
     }
+    o.err = o.ips + 8 * ni;
     o.clock = o.err + 8;  // three readings, see BatchTimes
-    o.total = (o.clock + 3 * 8 + 15) & ~(size_t)15;
+    o.copied = o.total = (o.clock + 3 * 8 + 15) & ~(size_t)15;
+    if (pl.values) {
+        o.hist = (o.copied + 255) & ~(size_t)255;
+        o.total = o.hist + 8 * (size_t)HIST_STRIDE * ni;
+    }
     return o;
 }
 
@@ -388,11 +395,11 @@ int bind_ctx_mem(cse_ctx *ctx, const Plan &pl, int mode, bool want_terms) {
     ENSURE(plan, pbytes);
     ENSURE(outb, o.total);
     ENSURE(recs, (size_t)REC_WORDS * 8 * (size_t)pl.nrec);
-    ENSURE(queue, 8);
+    ENSURE(queue, 16);
     ENSURE(stack, (size_t)pl.stack_words * 64 * 4 * 4 * (size_t)sweep_grid(ctx, pl, sweep_choice(pl, mode)));
     if (mode == 1) ENSURE(sexp, 4 * (size_t)pl.nrec);
     if (want_terms) ENSURE(terms, 4 * (size_t)(pl.nterms > 0 ? pl.nterms : 1));
-    int rc = ensure_host(ctx, ctx->hstage, o.total);
+    int rc = ensure_host(ctx, ctx->hstage, o.copied);
     if (rc) return rc;
     ctx->b_pinned = true;
     ctx->b_plan = (char *)ctx->plan.p;
@@ -441,7 +448,6 @@ int bind_static_mem(cse_ctx *ctx, const Plan &pl, char *hup, char *hstage) {
 int prep_batch(cse_ctx *ctx, const Plan &pl, int mode, size_t plan_bytes) {
     const OutLayout o = out_layout(pl, mode);
     char *b = ctx->b_out;
-    ctx->out_bytes = o.total;
     ctx->d_zsum = mode == 0 ? (long long *)(b + o.zsum) : nullptr;
     ctx->d_kahan = (double *)(b + o.kahan);
     ctx->d_sexp = mode == 0 ? (int32_t *)(b + o.sexp) : ctx->b_sexp1;
@@ -490,11 +496,12 @@ int run_sweep(cse_ctx *ctx, const Plan &pl, int mode, bool want_terms) {
     return CSE_OK;
 }
 
-// Results of at most this size come back in one block's stores, followed by
-// the call's number, which the host polls: 4 us less than a wait for the
-// stream.  Larger ones take a grid of blocks (faster than a copy call at 64 KB
-// to 1 MB: 14 to 32 us against 21 to 39).
-constexpr size_t kPollBytes = 16384;
+// Results come back in kernel stores (at 64 KB to 1 MB 14 to 32 us against 21
+// to 39 of a copy call), followed by the call's number, which the host polls:
+// 2 to 4 us less than a wait for the stream.  Results of more than kPollBytes
+// belong to calls of milliseconds, which outlast the polling; beyond
+// kGridBytes they come back in a copy call.
+constexpr size_t kPollBytes = 1 << 20;
 constexpr size_t kGridBytes = 64 << 20;
 
 // Runs a bound, staged batch, in stream order: plan and clear, records,
@@ -505,21 +512,29 @@ template <class F> int run_batch(cse_ctx *ctx, const Plan &pl, int mode, bool wa
     if (!rc) rc = run_records(ctx, pl, mode);
     if (!rc) rc = run_sweep(ctx, pl, mode, want_terms);
     if (rc) return rc;
-    const bool poll = ctx->b_pinned && ctx->out_bytes <= kPollBytes && !want_terms;
+    const OutLayout o = out_layout(pl, mode);
+    const size_t first = pl.values ? o.kahan : 0;  // the sums are written by the kernel itself
+    const size_t bytes = o.copied - first;
+    const bool dma = !ctx->b_pinned || bytes > kGridBytes;
+    const bool poll = !dma && bytes <= kPollBytes && !want_terms;
     ResultArgs a;
-    a.src = (const uint4 *)ctx->b_out;
-    a.dst = (uint4 *)ctx->b_hstage;
-    a.n = (long long)(ctx->out_bytes / 16);
+    a.src = (const uint4 *)(ctx->b_out + first);
+    a.dst = (uint4 *)(ctx->b_hstage + first);
+    a.n = dma ? 0 : (long long)(bytes / 16);
     a.clock = ctx->d_clock + 2;
+    a.hist = ctx->d_hist;
+    a.vals = (double *)(ctx->b_hstage + o.vals);
+    a.nvals = pl.values ? pl.ninst : 0;
+    a.left = (unsigned *)(ctx->b_queue + 1);
     a.done = poll ? (uint32_t *)ctx->hdone.p : nullptr;
     a.call = ++ctx->calls;
-    const bool dma = !ctx->b_pinned || ctx->out_bytes > kGridBytes;
-    if (dma) a.n = 0;
-    const long long blocks = poll ? 1 : std::min<long long>(1024, (a.n + 255) / 256);
+    // small results in one block: no count to wait for
+    const long long blocks =
+        std::min<long long>(1024, std::max((a.nvals + 3ll) / 4, bytes <= 16384 ? 1 : (a.n + 255) / 256));
     hipLaunchKernelGGL(k_results, dim3((unsigned)std::max(1ll, blocks)), dim3(256), 0, ctx->stream, a);
     HIPCHK(hipGetLastError());
     if (dma)
-        HIPCHK(hipMemcpyAsync(ctx->b_hstage, ctx->b_out, ctx->out_bytes, hipMemcpyDeviceToHost, ctx->stream));
+        HIPCHK(hipMemcpyAsync(ctx->b_hstage + first, ctx->b_out + first, bytes, hipMemcpyDeviceToHost, ctx->stream));
     if (want_terms) {
         rc = copy();
         if (rc) return rc;
@@ -1193,6 +1208,8 @@ static int exact_batch(cse_ctx *ctx, const cse_instance *in, int ninst, int chun
     int rc = use_static ? CSE_OK : ensure_host(ctx, ctx->hup, pbytes);
     if (rc) return rc;
     Plan pl = plan_in(use_static ? hup : (char *)ctx->hup.p, ninst);
+    pl.values = !use_static;
+    for (int i = 0; i < ninst; i++) pl.values = pl.values && !res[i].hist;
     TreeCosts one;
     std::vector<TreeCosts> many((size_t)(ninst > 1 ? ninst : 0));
     TreeCosts *const costs = ninst > 1 ? many.data() : &one;
@@ -1222,9 +1239,7 @@ static int exact_batch(cse_ctx *ctx, const cse_instance *in, int ninst, int chun
         return CSE_OK;
     });
     if (rc) return rc;
-    // the results block came back in one copy, into a pinned stage of the
-    // same layout: histograms (HIST_STRIDE words per instance), the Kahan
-    // pairs, the inner-product counts, the error flag
+    // the results block came back into a host stage of the same layout
     const OutLayout o = out_layout(pl, 1);
     char *hs = ctx->b_hstage;
     const unsigned long long *hist = (const unsigned long long *)(hs + o.hist);
@@ -1233,15 +1248,19 @@ static int exact_batch(cse_ctx *ctx, const cse_instance *in, int ninst, int chun
     const BatchTimes bt = batch_times(ctx, o);
     const double kms = bt.sweep, tms = bt.records + bt.sweep;
     if (kernel_ms) *kernel_ms = kms;
-    // each instance's exact value from its histogram (a few microseconds
-    // each): split over host threads for large batches
+    // each instance's exact value, from its sums or from its histogram (2.5 us
+    // each: split over host threads for large batches)
     auto convert = [&](int lo, int hi) {
         for (int i = lo; i < hi; i++) {
             cse_exact_result *r = &res[i];
-            const int64_t *h = (const int64_t *)&hist[(size_t)HIST_STRIDE * i];
             r->pmin = CSE_HIST_PMIN;
-            if (r->hist) memcpy(r->hist, h, 8 * (size_t)HIST_STRIDE);
-            cse_hist_value(h, CSE_HIST_PMIN, &r->re, &r->im);
+            if (pl.values) {
+                cse_hist_finish((const cse_dd *)(hs + o.vals) + 4 * (size_t)i, &r->re, &r->im);
+            } else {
+                const int64_t *h = (const int64_t *)&hist[(size_t)HIST_STRIDE * i];
+                if (r->hist) memcpy(r->hist, h, 8 * (size_t)HIST_STRIDE);
+                cse_hist_value(h, CSE_HIST_PMIN, &r->re, &r->im);
+            }
             r->value = hypot(r->re, r->im);
             r->kahan_re = kz[2 * i];
             r->kahan_im = kz[2 * i + 1];
@@ -1252,7 +1271,7 @@ static int exact_batch(cse_ctx *ctx, const cse_instance *in, int ninst, int chun
         }
     };
     const unsigned hw = std::thread::hardware_concurrency();
-    const int nthr = ninst >= 512 ? (int)std::min(8u, hw ? hw : 1u) : 1;
+    const int nthr = ninst >= 512 && !pl.values ? (int)std::min(8u, hw ? hw : 1u) : 1;
     if (nthr > 1) {
         const int per = (ninst + nthr - 1) / nthr;
         run_jobs(nthr, [&](int w) { convert(std::min(ninst, w * per), std::min(ninst, (w + 1) * per)); });

@@ -127,6 +127,14 @@ static cse_dd dd_scale(cse_dd a, int e)
 static const cse_dd SQRT2 = {1.4142135623730951, -9.667293313452913e-17};
 
 /* ------------------------------------------------ exact -> FP64 */
+void cse_hist_finish(const cse_dd s[4], double *re, double *im)
+{
+    cse_dd r = cse_dd_add(s[0], cse_dd_mul(s[2], SQRT2));
+    cse_dd im_ = cse_dd_add(s[1], cse_dd_mul(s[3], SQRT2));
+    *re = r.hi + r.lo;
+    *im = im_.hi + im_.lo;
+}
+
 void cse_hist_value(const int64_t *hist, int pmin, double *re, double *im)
 {
     /* bin (P, M) = hist[8 (-P) + M], P in [pmin, 0]: count * 2^{P/2} w^M.
@@ -173,10 +181,7 @@ void cse_hist_value(const int64_t *hist, int pmin, double *re, double *im)
         for (int q = 0; q < 4; q++)
             if (acc[q][i]) s[q] = cse_dd_add(s[q], dd_scale(cse_dd_from_i128(acc[q][i]), i + emin));
     }
-    cse_dd r = cse_dd_add(s[0], cse_dd_mul(s[2], SQRT2));
-    cse_dd im_ = cse_dd_add(s[1], cse_dd_mul(s[3], SQRT2));
-    *re = r.hi + r.lo;
-    *im = im_.hi + im_.lo;
+    cse_hist_finish(s, re, im);
 }
 
 /* (hi * 2^64 + lo) * 2^e in double-double; the carry of lo joins hi

@@ -57,6 +57,9 @@ typedef struct {
 cse_dd cse_dd_add(cse_dd a, cse_dd b);
 cse_dd cse_dd_mul(cse_dd a, cse_dd b);
 cse_dd cse_dd_from_i128(__int128 v);
+/* a histogram's value from its sums: real, imaginary, and both in units of
+ * sqrt2 */
+void cse_hist_finish(const cse_dd s[4], double *re, double *im);
 
 #ifdef __cplusplus
 }

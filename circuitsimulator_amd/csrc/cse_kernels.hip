@@ -660,32 +660,123 @@ struct PrepArgs {
     const uint4 *src;
     uint4 *dst, *zero;
     long long ncopy, nzero;  // 16-byte words
-    unsigned long long *queue;
+    unsigned long long *queue;  // and the count of k_results
 };
 extern "C" __global__ void k_prep(PrepArgs a) {
     const long long stride = (long long)gridDim.x * blockDim.x;
     const long long i0 = (long long)blockIdx.x * blockDim.x + threadIdx.x;
     for (long long i = i0; i < a.ncopy; i += stride) a.dst[i] = a.src[i];
     for (long long i = i0; i < a.nzero; i += stride) a.zero[i] = make_uint4(0, 0, 0, 0);
-    if (i0 == 0) *a.queue = 0;
+    if (i0 == 0) a.queue[0] = a.queue[1] = 0;
 }
 
-// A batch's results block to pinned host memory, grid-stride; with `done`
-// (one block), the call's number after them.
+// A batch's results block to pinned host memory, grid-stride; with `done`, the
+// call's number after them, by the last block to finish.
+//
+// nvals > 0: no caller wants the histograms of the exact instances, so their
+// Z[w] sums go to the host instead: 64 bytes an instance for 8,256, and what
+// the host needs 2.5 us an instance for takes a wave 2 to 3.  The sums and the
+// order of the additions are cse_hist_value's, so the values are the same
+// bits.  (A count is at most chi^2 <= 2^60, so 64-bit integers hold every sum
+// that is kept in 128 bits there.)
 struct ResultArgs {
     const uint4 *src;
     uint4 *dst;
     long long n;             // 16-byte words
     unsigned long long *clock;
+    const unsigned long long *hist;
+    double *vals;            // 8 per instance, pinned
+    int nvals;
+    unsigned *left;          // blocks that have finished
     uint32_t *done;
     uint32_t call;
 };
-extern "C" __global__ void k_results(ResultArgs a) {
+namespace {
+
+constexpr int kValueExps = (HIST_STRIDE / 8) / 2 + 2;  // powers of two: 0, -1 .. -65
+
+struct Dd {
+    double hi, lo;
+};
+DEV Dd dd_two_sum(double a, double b) {
+    const double s = a + b, bb = s - a;
+    return {s, (a - (s - bb)) + (b - bb)};
+}
+DEV Dd dd_quick_sum(double a, double b) {
+    const double s = a + b;
+    return {s, b - (s - a)};
+}
+DEV Dd dd_add(Dd a, Dd b) {
+    Dd s = dd_two_sum(a.hi, b.hi);
+    const Dd t = dd_two_sum(a.lo, b.lo);
+    s.lo += t.hi;
+    s = dd_quick_sum(s.hi, s.lo);
+    s.lo += t.lo;
+    return dd_quick_sum(s.hi, s.lo);
+}
+DEV Dd dd_int(long long v, int e) {
+    const double hi = (double)v;
+    const Dd r = dd_quick_sum(hi, (double)(v - (long long)hi));
+    return {ldexp(r.hi, e), ldexp(r.lo, e)};
+}
+
+// Row P = -r of a histogram: the sums of its even phases (real, imaginary)
+// and of its odd ones, the latter in units of sqrt(1/2).
+struct HistRow {
+    long long er = 0, ei = 0, orr = 0, oi = 0;
+    DEV HistRow(const unsigned long long *h, int r) {
+        if (r < 0 || r >= HIST_STRIDE / 8) return;
+        const long long *b = (const long long *)h + 8 * r;
+        er = b[0] - b[4];
+        ei = b[2] - b[6];
+        orr = (b[1] - b[3]) - (b[5] - b[7]);
+        oi = (b[1] + b[3]) - (b[5] + b[7]);
+    }
+};
+
+}  // namespace
+extern "C" __global__ void __launch_bounds__(256) k_results(ResultArgs a) {
+    const unsigned long long now = wall_clock64();
+    __shared__ Dd s_acc[4][4][kValueExps];
+    // an instance a wave: lane j adds up what has the power -j of two (rows
+    // 2j, 2j - 1 and 2j - 2), four lanes then add the powers from the lowest
+    const int x = lane_id(), wv = (int)threadIdx.x >> 6;
+    for (int at = 4 * (int)blockIdx.x; at < a.nvals; at += 4 * (int)gridDim.x) {
+        const int i = at + wv;
+        u64 used = 0;
+        if (i < a.nvals) {
+            const unsigned long long *h = a.hist + (size_t)HIST_STRIDE * (size_t)i;
+            for (int j0 = 0; j0 < kValueExps; j0 += 64) {
+                const int j = j0 + x;
+                const bool in = j < kValueExps;
+                const HistRow r0(h, in ? 2 * j : -1), r1(h, in ? 2 * j - 1 : -1), r2(h, in ? 2 * j - 2 : -1);
+                const long long v[4] = {r0.er + r1.orr, r0.ei + r1.oi, r1.er + r2.orr, r1.ei + r2.oi};
+                if (in)
+                    for (int q = 0; q < 4; q++) s_acc[wv][q][j] = dd_int(v[q], -j);
+                const u64 some = ballot((v[0] | v[1] | v[2] | v[3]) != 0);
+                if (j0 == 0) used = some;
+                else if (some) used |= 1ull << 63;  // 63 stands for the rest as well
+            }
+        }
+        __syncthreads();
+        if (i < a.nvals && x < 4) {
+            Dd s = {0.0, 0.0};
+            if (used >> 63)
+                for (int j = kValueExps - 1; j >= 63; j--) s = dd_add(s, s_acc[wv][x][j]);
+            for (used &= ~(1ull << 63); used;) {
+                const int j = 63 - __clzll((long long)used);
+                used &= ~(1ull << j);
+                s = dd_add(s, s_acc[wv][x][j]);
+            }
+            a.vals[8 * (size_t)i + 2 * x] = s.hi;
+            a.vals[8 * (size_t)i + 2 * x + 1] = s.lo;
+        }
+        __syncthreads();
+    }
     const long long stride = (long long)gridDim.x * blockDim.x;
     const long long i0 = (long long)blockIdx.x * blockDim.x + threadIdx.x;
     // the clock is part of the block's last words: its 16 bytes are put
     // together by the thread that copies them
-    const unsigned long long now = wall_clock64();
     const long long off = (const char *)a.clock - (const char *)a.src, at = off >> 4;
     const int half = (int)(off >> 3) & 1;
     if (i0 == 0 && a.n == 0) *a.clock = now;
@@ -703,8 +794,14 @@ extern "C" __global__ void k_results(ResultArgs a) {
         a.dst[i] = v;
     }
     if (a.done) {
+        // a block's stores have reached the host before it counts itself (a
+        // block of its own has nobody to count: the atomic costs 1 us), and
+        // the last one tells the host
         __threadfence_system();
         __syncthreads();
-        if (threadIdx.x == 0) __hip_atomic_store(a.done, a.call, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+        if (threadIdx.x == 0 &&
+            (gridDim.x == 1 ||
+             __hip_atomic_fetch_add(a.left, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == gridDim.x - 1))
+            __hip_atomic_store(a.done, a.call, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
     }
 }
