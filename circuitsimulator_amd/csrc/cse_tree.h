@@ -103,29 +103,46 @@ TREE_DEV u32 push_nz(u32 w, u32 t) {
 // and b start as the same value.)
 // N rows r: r ^= a where tv's next bit is set, ^= b where tw's is.  One asm
 // block for several rows: between blocks the compiler pads with s_nop.
-#define TREE_ROW(r)                                                                        \
+//
+// From four rows on a bit leaves its word as the carry of word + word, and the
+// carry selects a or 0: five instructions a row.  A carry must not be read in
+// the next two instructions after the one that writes it, so a row's selects
+// wait behind the update of the row before.  The second carry is in a fixed
+// pair below s64: with carries in s64 or above the same stream runs at 2.4
+// instead of 3.7 wave instructions per ns and CU (the register allocator took
+// s64 in the exact kernels, which then lost 10%).  One or two rows, where the
+// wait is not filled, take masks: six a row.  2^28 terms of t = 48 with masks
+// throughout 10.1 ms, with carries from eight rows on 9.5, from four 9.3.
+#define TREE_CARRY "v_add_co_u32 %[tv], vcc, %[tv], %[tv]\n\tv_add_co_u32 %[tw], s[46:47], %[tw], %[tw]\n\t"
+#define TREE_SEL "v_cndmask_b32 %[m], 0, %[a], vcc\n\tv_cndmask_b32 %[q], 0, %[b], s[46:47]\n\t"
+#define TREE_UPD(r) "v_bitop3_b32 " r ", " r ", %[m], %[q] bitop3:0x96\n\t"
+#define TREE_ROW0 TREE_CARRY "s_nop 0\n\t" TREE_SEL
+#define TREE_ROW(r) TREE_CARRY TREE_UPD(r) TREE_SEL
+#define TREE_ROWS_IO                                                                     \
+    [tv] "+&v"(tv), [tw] "+&v"(tw), [m] "=&v"(m), [q] "=&v"(q) : [a] "v"(a), [b] "v"(b) : "vcc", "s46", "s47"
+#define TREE_FEW(r)                                                                        \
     "v_ashrrev_i32 %[m], 31, %[tv]\n\tv_add_u32 %[tv], %[tv], %[tv]\n\t"                  \
     "v_bitop3_b32 " r ", " r ", %[m], %[a] bitop3:0x78\n\t"                                \
     "v_ashrrev_i32 %[m], 31, %[tw]\n\tv_add_u32 %[tw], %[tw], %[tw]\n\t"                  \
     "v_bitop3_b32 " r ", " r ", %[m], %[b] bitop3:0x78\n\t"
-#define TREE_ROWS_IO [tv] "+&v"(tv), [tw] "+&v"(tw), [m] "=&v"(m) : [a] "v"(a), [b] "v"(b)
+#define TREE_FEW_IO [tv] "+&v"(tv), [tw] "+&v"(tw), [m] "=&v"(m) : [a] "v"(a), [b] "v"(b)
 template <int N> TREE_DEV void rows(u32 *r, u32 &tv, u32 &tw, u32 a, u32 b) {
-    u32 m;
+    u32 m, q;
     if constexpr (N >= 8) {
-        asm(TREE_ROW("%0") TREE_ROW("%1") TREE_ROW("%2") TREE_ROW("%3") TREE_ROW("%4") TREE_ROW("%5") TREE_ROW("%6")
-                TREE_ROW("%7")
+        asm(TREE_ROW0 TREE_ROW("%0") TREE_ROW("%1") TREE_ROW("%2") TREE_ROW("%3") TREE_ROW("%4") TREE_ROW("%5")
+                TREE_ROW("%6") TREE_UPD("%7")
             : "+&v"(r[0]), "+&v"(r[1]), "+&v"(r[2]), "+&v"(r[3]), "+&v"(r[4]), "+&v"(r[5]), "+&v"(r[6]), "+&v"(r[7]),
               TREE_ROWS_IO);
         rows<N - 8>(r + 8, tv, tw, a, b);
     } else if constexpr (N >= 4) {
-        asm(TREE_ROW("%0") TREE_ROW("%1") TREE_ROW("%2") TREE_ROW("%3")
+        asm(TREE_ROW0 TREE_ROW("%0") TREE_ROW("%1") TREE_ROW("%2") TREE_UPD("%3")
             : "+&v"(r[0]), "+&v"(r[1]), "+&v"(r[2]), "+&v"(r[3]), TREE_ROWS_IO);
         rows<N - 4>(r + 4, tv, tw, a, b);
     } else if constexpr (N >= 2) {
-        asm(TREE_ROW("%0") TREE_ROW("%1") : "+&v"(r[0]), "+&v"(r[1]), TREE_ROWS_IO);
+        asm(TREE_FEW("%0") TREE_FEW("%1") : "+&v"(r[0]), "+&v"(r[1]), TREE_FEW_IO);
         rows<N - 2>(r + 2, tv, tw, a, b);
     } else if constexpr (N == 1) {
-        asm(TREE_ROW("%0") : "+&v"(r[0]), TREE_ROWS_IO);
+        asm(TREE_FEW("%0") : "+&v"(r[0]), TREE_FEW_IO);
     }
 }
 // the same for rows of two words
