@@ -247,6 +247,7 @@ struct Plan {
     long long stack_words = 0;  // per lane and wave, beyond LDS
     int nmax = 0;
     bool anyH = false;
+    int copies = 1;       // of the results block, see spread_sums
     bool values = false;  // exact mode: sums go to the host, not histograms
     // counts the instances, whose descriptors are complete but for their
     // offsets: instance i has nr(i) records and nt(i) terms
@@ -334,7 +335,7 @@ int run_records(cse_ctx *ctx, const Plan &pl, int mode) {
 struct OutLayout {
     size_t vals, zsum, kahan, sexp, hist, ips, err, clock;
     size_t copied;  // the end of what comes back
-    size_t total;
+    size_t total;   // of one copy, a multiple of 256 bytes where there are several
 };
 
 OutLayout out_layout(const Plan &pl, int mode) {
@@ -357,6 +358,7 @@ OutLayout out_layout(const Plan &pl, int mode) {
         o.hist = (o.copied + 255) & ~(size_t)255;
         o.total = o.hist + 8 * (size_t)HIST_STRIDE * ni;
     }
+    if (pl.copies > 1) o.total = (o.total + 255) & ~(size_t)255;
     return o;
 }
 
@@ -366,7 +368,6 @@ OutLayout out_layout(const Plan &pl, int mode) {
 // instructions a step).
 typedef void (*SweepFn)(SweepArgs);
 struct SweepKernel {
-    int id;
     SweepFn fn;
     int blocks_per_cu;
 };
@@ -375,8 +376,9 @@ SweepKernel sweep_choice(const Plan &pl, int mode) {
                                         {{k_sweep_e32, k_sweep_e48, k_sweep_e64}, {k_sweep_eh32, k_sweep_eh48, k_sweep_eh64}}};
     const int w = pl.nmax <= 32 ? 0 : pl.nmax <= 48 ? 1 : 2, h = pl.anyH ? 1 : 0;
     SweepKernel k;
-    k.id = (mode * 2 + h) * 3 + w;
     k.fn = fn[mode][h][w];
+    static const SweepFn copies[3] = {k_sweep_c32, k_sweep_c48, k_sweep_c64};
+    if (pl.copies > 1) k.fn = copies[w];
     k.blocks_per_cu = w == 2 ? 3 : 4;
     return k;
 }
@@ -386,6 +388,17 @@ int sweep_grid(const cse_ctx *ctx, const Plan &pl, const SweepKernel &k) {
     return (int)std::max(1ll, std::min((long long)ctx->cus * k.blocks_per_cu, pl.nitems));
 }
 
+// The blocks of a launch of one exact instance all add their sums to the same
+// 8 KB at their end.  From 256 blocks on they add to TREE_COPIES copies, which
+// the results kernel adds up: calls of t = 24, k = 11 take 88.8 us with one
+// copy, 80.6 with 4 or 8, 82.2 with 16, those of k = 10 58.9 and 56.0.  Below
+// (t = 20, k = 8) the copies cost 1 us, and |H^t> sums, which fall into fewer
+// bins, gain nothing (t = 24: 114.7 us with one copy, 116.8 with 8).
+void spread_sums(const cse_ctx *ctx, Plan &pl) {
+    if (pl.anyH || sweep_grid(ctx, pl, sweep_choice(pl, 1)) < 256) return;
+    pl.copies = TREE_COPIES;
+}
+
 // Binds a batch to the context's own buffers, grown on demand (device memory
 // and the pinned host stage of the results; the plan is in ctx->hup).
 int bind_ctx_mem(cse_ctx *ctx, const Plan &pl, int mode, bool want_terms) {
@@ -393,7 +406,7 @@ int bind_ctx_mem(cse_ctx *ctx, const Plan &pl, int mode, bool want_terms) {
     const size_t pbytes = plan_layout(pl.ninst, off);
     const OutLayout o = out_layout(pl, mode);
     ENSURE(plan, pbytes);
-    ENSURE(outb, o.total);
+    ENSURE(outb, o.total * (size_t)pl.copies);
     ENSURE(recs, (size_t)REC_WORDS * 8 * (size_t)pl.nrec);
     ENSURE(queue, 16);
     ENSURE(stack, (size_t)pl.stack_words * 64 * 4 * 4 * (size_t)sweep_grid(ctx, pl, sweep_choice(pl, mode)));
@@ -460,7 +473,7 @@ int prep_batch(cse_ctx *ctx, const Plan &pl, int mode, size_t plan_bytes) {
     a.dst = (uint4 *)ctx->b_plan;
     a.ncopy = ctx->b_pinned ? (long long)(plan_bytes / 16) : 0;
     a.zero = (uint4 *)b;
-    a.nzero = (long long)(o.total / 16);
+    a.nzero = (long long)(o.total * (size_t)pl.copies / 16);
     a.queue = ctx->b_queue;
     if (!ctx->b_pinned)
         HIPCHK(hipMemcpyAsync(ctx->b_plan, ctx->b_hup, plan_bytes, hipMemcpyHostToDevice, ctx->stream));
@@ -490,6 +503,7 @@ int run_sweep(cse_ctx *ctx, const Plan &pl, int mode, bool want_terms) {
     A.hist = ctx->d_hist;
     A.ips = ctx->d_ips;
     A.clock = ctx->d_clock;
+    A.copy_words = (unsigned)(out_layout(pl, mode).total / 8);
     const SweepKernel k = sweep_choice(pl, mode);
     hipLaunchKernelGGL(k.fn, dim3(sweep_grid(ctx, pl, k)), dim3(256), 0, ctx->stream, A);
     HIPCHK(hipGetLastError());
@@ -525,13 +539,17 @@ template <class F> int run_batch(cse_ctx *ctx, const Plan &pl, int mode, bool wa
     a.hist = ctx->d_hist;
     a.vals = (double *)(ctx->b_hstage + o.vals);
     a.nvals = pl.values ? pl.ninst : 0;
+    a.copies = pl.copies;
+    a.tail = (int)((o.kahan - first) / 8);
+    a.copy_words = (long long)(o.total / 8);
     a.left = (unsigned *)(ctx->b_queue + 1);
     a.done = poll ? (uint32_t *)ctx->hdone.p : nullptr;
     a.call = ++ctx->calls;
     // small results in one block: no count to wait for
     const long long blocks =
         std::min<long long>(1024, std::max((a.nvals + 3ll) / 4, bytes <= 16384 ? 1 : (a.n + 255) / 256));
-    hipLaunchKernelGGL(k_results, dim3((unsigned)std::max(1ll, blocks)), dim3(256), 0, ctx->stream, a);
+    hipLaunchKernelGGL(pl.copies > 1 ? k_results_copies : k_results, dim3((unsigned)std::max(1ll, blocks)), dim3(256),
+                       0, ctx->stream, a);
     HIPCHK(hipGetLastError());
     if (dma)
         HIPCHK(hipMemcpyAsync(ctx->b_hstage + first, ctx->b_out + first, bytes, hipMemcpyDeviceToHost, ctx->stream));
@@ -1232,6 +1250,7 @@ static int exact_batch(cse_ctx *ctx, const cse_instance *in, int ninst, int chun
     pl.finish(ninst, [&](int i) { return pl.inst[i].chi; },
               [&](int i) { return pl.inst[i].chi * (pl.inst[i].chi + 1) / 2; });
     if (terms_out && pl.nterms > (1ll << 31)) return fail(ctx, CSE_ERR_ARG, "per-term output too large");
+    if (ninst == 1 && !use_static) spread_sums(ctx, pl);
     rc = use_static ? bind_static_mem(ctx, pl, hup, hstage) : bind_ctx_mem(ctx, pl, 1, terms_out != nullptr);
     if (rc) return rc;
     rc = run_batch(ctx, pl, 1, terms_out != nullptr, stage_plan(ctx, pl), [&]() -> int {

@@ -50,6 +50,9 @@ constexpr int tree_words(int c) { return TREE_STATE_WORDS + (c <= 32 ? c : TREE_
 // below 2^32
 #define CSE_FLUSH_TERMS_MAX (1ll << 30)
 
+// copies of an instance's sums where there are several (spread_sums)
+#define TREE_COPIES 8
+
 // Histogram bins per instance: P in [-(64 + 64), 0], 8 phases (the public
 // CSE_HIST_BINS).
 #define HIST_STRIDE (129 * 8)
@@ -102,6 +105,9 @@ struct SweepArgs {
     unsigned long long *hist; // HIST_STRIDE per instance
     unsigned long long *ips;  // per instance
     unsigned long long *clock; // readings: records, sweep, results start
+    // k_sweep_c*: the sums above are those of copy 0; block b adds to copy
+    // b mod TREE_COPIES, copies being copy_words 8-byte words apart
+    unsigned copy_words;
 };
 
 #ifdef __HIPCC__

@@ -687,6 +687,10 @@ struct ResultArgs {
     const unsigned long long *hist;
     double *vals;            // 8 per instance, pinned
     int nvals;
+    // one exact instance whose sums come in copies (SweepArgs): of the
+    // histogram, and from word `tail` of src of the Kahan pair and the count
+    int copies, tail;
+    long long copy_words;
     unsigned *left;          // blocks that have finished
     uint32_t *done;
     uint32_t call;
@@ -735,9 +739,29 @@ struct HistRow {
 };
 
 }  // namespace
-extern "C" __global__ void __launch_bounds__(256) k_results(ResultArgs a) {
+template <bool COPIES> DEV void results_body(const ResultArgs &a) {
     const unsigned long long now = wall_clock64();
     __shared__ Dd s_acc[4][4][kValueExps];
+    __shared__ unsigned long long s_sum[COPIES ? HIST_STRIDE + 3 : 1];
+    const unsigned long long *hist = a.hist;
+    if (COPIES) {
+        for (int w = (int)threadIdx.x; w < HIST_STRIDE + 3; w += 256) {
+            const int t = w - HIST_STRIDE;
+            const unsigned long long *p = t < 0 ? a.hist + w : (const unsigned long long *)a.src + a.tail + t;
+            unsigned long long v[TREE_COPIES], s = 0;
+            double k = 0.0;
+#pragma unroll
+            for (int c = 0; c < TREE_COPIES; c++) v[c] = c < a.copies ? p[(size_t)c * (size_t)a.copy_words] : 0ull;
+#pragma unroll
+            for (int c = 0; c < TREE_COPIES; c++) {
+                s += v[c];
+                k += __longlong_as_double((long long)v[c]);
+            }
+            s_sum[w] = t == 0 || t == 1 ? (unsigned long long)__double_as_longlong(k) : s;
+        }
+        __syncthreads();
+        hist = s_sum;
+    }
     // an instance a wave: lane j adds up what has the power -j of two (rows
     // 2j, 2j - 1 and 2j - 2), four lanes then add the powers from the lowest
     const int x = lane_id(), wv = (int)threadIdx.x >> 6;
@@ -745,7 +769,7 @@ extern "C" __global__ void __launch_bounds__(256) k_results(ResultArgs a) {
         const int i = at + wv;
         u64 used = 0;
         if (i < a.nvals) {
-            const unsigned long long *h = a.hist + (size_t)HIST_STRIDE * (size_t)i;
+            const unsigned long long *h = hist + (size_t)HIST_STRIDE * (size_t)i;
             for (int j0 = 0; j0 < kValueExps; j0 += 64) {
                 const int j = j0 + x;
                 const bool in = j < kValueExps;
@@ -782,6 +806,14 @@ extern "C" __global__ void __launch_bounds__(256) k_results(ResultArgs a) {
     if (i0 == 0 && a.n == 0) *a.clock = now;
     for (long long i = i0; i < a.n; i += stride) {
         uint4 v = a.src[i];
+        if (COPIES) {
+            const int w = (int)(2 * i), u = w - a.tail + HIST_STRIDE;
+            unsigned long long lo = v.x | (u64)v.y << 32, hi = v.z | (u64)v.w << 32;
+            if (a.nvals == 0 && w < HIST_STRIDE) lo = s_sum[w], hi = s_sum[w + 1];
+            if (u >= HIST_STRIDE && u < HIST_STRIDE + 3) lo = s_sum[u];
+            if (u + 1 >= HIST_STRIDE && u + 1 < HIST_STRIDE + 3) hi = s_sum[u + 1];
+            v = make_uint4((unsigned)lo, (unsigned)(lo >> 32), (unsigned)hi, (unsigned)(hi >> 32));
+        }
         if (i == at) {
             if (half) {
                 v.z = (unsigned)now;
@@ -805,3 +837,5 @@ extern "C" __global__ void __launch_bounds__(256) k_results(ResultArgs a) {
             __hip_atomic_store(a.done, a.call, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
     }
 }
+extern "C" __global__ void __launch_bounds__(256) k_results(ResultArgs a) { results_body<false>(a); }
+extern "C" __global__ void __launch_bounds__(256) k_results_copies(ResultArgs a) { results_body<true>(a); }

@@ -164,8 +164,10 @@ struct TermTables {
 // histogram; a block keeps its partial histogram and Kahan sums from item to
 // item of one instance and adds them to the instance's global sums when it
 // moves to another one and at its exit.  NH: slots beyond 32 (n <= 32 + NH).
-// HT: some instance has |H^t> terms.
-template <int NH, bool HT, int MODE> DEV void sweep_body(const SweepArgs &A) {
+// HT: some instance has |H^t> terms.  COPIES: one instance, its sums in copies
+// (kernels of their own: the address alone cost the others 1 to 2% of a call
+// of 40 us).
+template <int NH, bool HT, int MODE, bool COPIES> DEV void sweep_body(const SweepArgs &A) {
     // levels beyond 32 slots: only where instances may have them (tree_levels)
     constexpr bool DEEP = NH > 16 && !HT;
     constexpr int LW = MODE == 0 ? TREE_LDS_WORDS0 : TREE_LDS_WORDS1;
@@ -203,9 +205,10 @@ template <int NH, bool HT, int MODE> DEV void sweep_body(const SweepArgs &A) {
             s_k[wv] = wk;
         }
         __syncthreads();
+        const unsigned copy = COPIES ? (blockIdx.x % TREE_COPIES) * A.copy_words : 0u;
         if (tid == 0) {
-            atomicAdd(&A.ips[cur], s_ips[0] + s_ips[1] + s_ips[2] + s_ips[3]);
-            if (MODE == 1) atomicAdd(&A.kahan[2 * (size_t)cur], (s_k[0] + s_k[1]) + (s_k[2] + s_k[3]));
+            atomicAdd(&(A.ips + copy)[cur], s_ips[0] + s_ips[1] + s_ips[2] + s_ips[3]);
+            if (MODE == 1) atomicAdd(&(A.kahan + copy)[2 * (size_t)cur], (s_k[0] + s_k[1]) + (s_k[2] + s_k[3]));
         }
         if (MODE == 1) {
             // an off-diagonal term counts as z + conj(z): phases 0 and 4 are
@@ -215,7 +218,7 @@ template <int NH, bool HT, int MODE> DEV void sweep_body(const SweepArgs &A) {
                 if (!v) continue;
                 hist[b] = 0;
                 const int m = b & 7;
-                unsigned long long *h = A.hist + (size_t)cur * HIST_STRIDE;
+                unsigned long long *h = A.hist + copy + (size_t)cur * HIST_STRIDE;
                 atomicAdd(&h[b], (unsigned long long)v << (m == 4 ? 1 : 0));
                 if (m & 3) atomicAdd(&h[(b & ~7) | (8 - m)], (unsigned long long)v);
             }
@@ -526,19 +529,22 @@ extern "C" __global__ void k_leaf_table(uint8_t *plain, uint8_t *sign) {
     if (i < 1u << tree::LeafBits<true>::value) leaf_entry<true>(i, sign);
 }
 
-#define SWEEP_KERNEL(NAME, NH, HT, MODE, WAVES)                                            \
+#define SWEEP_KERNEL(NAME, NH, HT, MODE, COPIES, WAVES)                                    \
     extern "C" __global__ void __launch_bounds__(256, WAVES) NAME(SweepArgs A) {           \
-        sweep_body<NH, HT, MODE>(A);                                                       \
+        sweep_body<NH, HT, MODE, COPIES>(A);                                               \
     }
-SWEEP_KERNEL(k_sweep_s32, 0, false, 0, 4)
-SWEEP_KERNEL(k_sweep_s48, 16, false, 0, 4)
-SWEEP_KERNEL(k_sweep_s64, 32, false, 0, 3)
-SWEEP_KERNEL(k_sweep_e32, 0, false, 1, 4)
-SWEEP_KERNEL(k_sweep_e48, 16, false, 1, 4)
-SWEEP_KERNEL(k_sweep_e64, 32, false, 1, 3)
-SWEEP_KERNEL(k_sweep_sh32, 0, true, 0, 4)
-SWEEP_KERNEL(k_sweep_sh48, 16, true, 0, 4)
-SWEEP_KERNEL(k_sweep_sh64, 32, true, 0, 3)
-SWEEP_KERNEL(k_sweep_eh32, 0, true, 1, 4)
-SWEEP_KERNEL(k_sweep_eh48, 16, true, 1, 4)
-SWEEP_KERNEL(k_sweep_eh64, 32, true, 1, 3)
+SWEEP_KERNEL(k_sweep_s32, 0, false, 0, false, 4)
+SWEEP_KERNEL(k_sweep_s48, 16, false, 0, false, 4)
+SWEEP_KERNEL(k_sweep_s64, 32, false, 0, false, 3)
+SWEEP_KERNEL(k_sweep_e32, 0, false, 1, false, 4)
+SWEEP_KERNEL(k_sweep_e48, 16, false, 1, false, 4)
+SWEEP_KERNEL(k_sweep_e64, 32, false, 1, false, 3)
+SWEEP_KERNEL(k_sweep_sh32, 0, true, 0, false, 4)
+SWEEP_KERNEL(k_sweep_sh48, 16, true, 0, false, 4)
+SWEEP_KERNEL(k_sweep_sh64, 32, true, 0, false, 3)
+SWEEP_KERNEL(k_sweep_eh32, 0, true, 1, false, 4)
+SWEEP_KERNEL(k_sweep_eh48, 16, true, 1, false, 4)
+SWEEP_KERNEL(k_sweep_eh64, 32, true, 1, false, 3)
+SWEEP_KERNEL(k_sweep_c32, 0, false, 1, true, 4)
+SWEEP_KERNEL(k_sweep_c48, 16, false, 1, true, 4)
+SWEEP_KERNEL(k_sweep_c64, 32, false, 1, true, 3)

@@ -74,3 +74,18 @@ def test_batches(E, count):
     vals, _ = E.batch_exact_values(A)
     assert np.array_equal(vals[:40], want[:40])
     assert vals[1] == 0.0
+
+
+@pytest.mark.parametrize("t,k", [(24, 9), (24, 10), (40, 10), (50, 11)])
+def test_copies_of_the_sums(E, t, k):
+    """Calls of 256 blocks and more add to copies of the histogram: the same
+    histogram, count and value as the call in the library's static array,
+    which has one copy."""
+    (ph, xs, zs), L = drawn(t, k, t // 3, t + k)
+    P = Projector.make(ph, xs, zs, t)
+    a, ha = E.exact_projector(P, L, k, 0, want_hist=True)
+    b, hb = E.exact_projector_noalloc(P, L, k, 0, want_hist=True)
+    c, _ = E.exact_projector(P, L, k, 0)
+    assert np.array_equal(ha, hb) and a.ips == b.ips == c.ips == a.terms
+    assert (a.re, a.im) == (b.re, b.im) == (c.re, c.im) == host_value(ha)
+    assert abs(a.kahan_re - b.kahan_re) <= 1e-5 * abs(a.re)
