@@ -20,15 +20,13 @@ import time
 ROOT = os.path.dirname(os.path.abspath(__file__))
 sys.path.insert(0, ROOT)
 
-# Algorithmic work per inner product of the elimination algorithm the sweep
-# runs (fixation of the pivot coordinates outside supp(x_j), restrictions on
-# non-pivot columns, A/B/C elimination steps), in 64-bit word operations of a
-# dense-row formulation: the mean over 64 projected random states x 512
-# seeded j of this workload, from the register-level model of the kernel
-# (tests/test_sweep_model.py, algorithmic_work), which checks it.  Two int32
-# lane operations per word operation.
+# Work per inner product when every term is eliminated by itself (fixation of
+# the pivot coordinates outside supp(x_j), restrictions on non-pivot columns,
+# A/B/C elimination steps), in 64-bit word operations of a dense-row
+# formulation: the mean over 64 projected random states x 512 seeded j of this
+# workload, from the model in tests/test_sweep_model.py (algorithmic_work),
+# which checks it.  The sweep shares eliminations between terms.
 ALG_WORDOPS_PER_IP = 982.0
-ALG_LANE_OPS_PER_IP = 2 * ALG_WORDOPS_PER_IP
 # The canonical dense-row algorithm's count (the reference's shrink /
 # basis-alignment / exponential-sum sequence, oracle/cse_oracle.c
 # orc_ip_wordops), mean over the same workload
@@ -36,15 +34,17 @@ CANONICAL_WORDOPS_PER_IP = 14743
 
 # Per inner product of the sweep kernel on this workload, from rocprofv3
 # --pmc over one dispatch of 2^28 inner products
-# (profiles/k_sweep_norm_estimation_t48_r24_k12_M65536.md):
-VALU_INSTS_PER_IP = 163.8    # SQ_INSTS_VALU / inner products (wave64 instructions)
-SALU_INSTS_PER_IP = 159.1    # SQ_INSTS_SALU / inner products
+# (profiles/sweep_cases.md):
+VALU_INSTS_PER_IP = 36.0     # SQ_INSTS_VALU / inner products (wave64 instructions)
+SALU_INSTS_PER_IP = 1.5      # SQ_INSTS_SALU / inner products
 VALU_LANE_OPS_PER_IP = VALU_INSTS_PER_IP * 64
 # HBM bytes per inner product of the sweep: (FETCH_SIZE x 2.000 + WRITE_SIZE x
 # 1.000) KiB, factors from a 1 GiB copy kernel, / inner products
-SWEEP_BYTES_PER_IP = 2.80
-CLOCK_GHZ = 2.38             # GRBM_GUI_ACTIVE / kernel time / 8 XCDs
-PEAK_INT_TOPS = 39.3  # 256 CU x 4 SIMD x 16 lanes x 2.4 GHz, int32 lane-ops/s
+SWEEP_BYTES_PER_IP = 53.7
+CLOCK_GHZ = 2.28             # GRBM_GUI_ACTIVE / kernel time / 8 XCDs
+# 256 CU x 2 wave64 instructions per cycle x 2.4 GHz, int32 lane-ops/s: the
+# rate of and, xor, or, bitop3, add, sub and right shifts
+PEAK_INT_TOPS = 78.6
 
 
 def exact_mean(t, sexp, zsum):
@@ -711,23 +711,22 @@ def main():
     }
     if "tune_s" in tuning:
         out["tuning"] = tuning
-    # integer-VALU roofline of the sweep kernel: the algorithm's own work
-    # (int32 lane-operations per inner product of the elimination algorithm
-    # it runs) at the kernel's rate, against the VALU peak
-    achieved = kernel_ips * ALG_LANE_OPS_PER_IP / 1e12
+    # integer-VALU roofline of the sweep kernel: its executed int32 lane
+    # operations per inner product at the kernel's rate, against the VALU peak
+    achieved = kernel_ips * VALU_LANE_OPS_PER_IP / 1e12
     out["roofline"] = {"bound": "valu", "achieved": achieved, "peak": PEAK_INT_TOPS, "unit": "Tops/s",
                        "frac": achieved / PEAK_INT_TOPS,
                        "traffic": SWEEP_BYTES_PER_IP * M * chi,
                        "traffic_source": "rocprofv3 FETCH_SIZE/WRITE_SIZE of one sweep dispatch, calibrated",
-                       "kernel": "k_sweep_packed",
-                       "per_unit": f"{ALG_LANE_OPS_PER_IP:.0f} int32 lane-ops ({ALG_WORDOPS_PER_IP:.0f} 64-bit "
-                                   f"word-ops) per inner product of the fixation/elimination algorithm",
+                       "kernel": "k_sweep_s48",
+                       "per_unit": f"{VALU_LANE_OPS_PER_IP:.0f} executed int32 lane-ops per inner product",
+                       "unshared_wordops_per_ip": ALG_WORDOPS_PER_IP,
                        "canonical_wordops_per_ip": CANONICAL_WORDOPS_PER_IP}
-    # the binding limit: instruction issue (one SALU per CU per cycle, one
-    # wave64 VALU per SIMD per 4 cycles), from the executed instruction counts
+    # the binding limit: instruction issue (one SALU per CU per cycle, two
+    # wave64 VALU), from the executed instruction counts
     out["issue"] = {
         "salu_frac": kernel_ips * SALU_INSTS_PER_IP / (cus * CLOCK_GHZ * 1e9),
-        "valu_frac": kernel_ips * VALU_INSTS_PER_IP / (cus * 4 * CLOCK_GHZ * 1e9 / 4),
+        "valu_frac": kernel_ips * VALU_INSTS_PER_IP / (cus * 2 * CLOCK_GHZ * 1e9),
         "salu_per_ip": SALU_INSTS_PER_IP, "valu_per_ip": VALU_INSTS_PER_IP,
         "executed_valu_lane_ops_per_ip": VALU_LANE_OPS_PER_IP,
         "hbm_GBps": kernel_ips * SWEEP_BYTES_PER_IP / 1e9,
