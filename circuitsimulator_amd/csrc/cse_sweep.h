@@ -194,6 +194,9 @@ template <int NH, bool HT, int MODE, bool COPIES> DEV void sweep_body(const Swee
     for (int b = tid; b < 1 << tree::LeafBits<HT>::value; b += 256) s_leaf[b] = A.leaf[b];
     if (MODE == 1)
         for (int b = tid; b < HIST_STRIDE; b += 256) hist[b] = 0;
+    // Other waves read the tables and add to the histogram, and no barrier of
+    // the first item comes before that.
+    __syncthreads();
 
     // adds the block's sums of instance cur to the global ones (whole block)
     auto flush = [&]() {
