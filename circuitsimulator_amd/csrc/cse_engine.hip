@@ -503,6 +503,7 @@ int run_sweep(cse_ctx *ctx, const Plan &pl, int mode, bool want_terms) {
     A.hist = ctx->d_hist;
     A.ips = ctx->d_ips;
     A.clock = ctx->d_clock;
+    A.err = ctx->d_err;
     A.copy_words = (unsigned)(out_layout(pl, mode).total / 8);
     const SweepKernel k = sweep_choice(pl, mode);
     hipLaunchKernelGGL(k.fn, dim3(sweep_grid(ctx, pl, k)), dim3(256), 0, ctx->stream, A);
@@ -1138,6 +1139,7 @@ static int sampled_batch(cse_ctx *ctx, const cse_sampled_instance *in, int ninst
     int *errp = (int *)(hs + o.err);
     const int errv = *errp;
     if (errv & 1) return fail(ctx, CSE_ERR_RNG, "random state draw exceeded its shrink cap");
+    if (errv & 2) return fail(ctx, CSE_ERR_HIP, "internal: an inner product exponent left [-64, 0]");
     const BatchTimes bt = batch_times(ctx, o);
     const double pms = bt.records, kms = bt.sweep;
     if (kernel_ms) *kernel_ms = kms;
@@ -1266,6 +1268,8 @@ static int exact_batch(cse_ctx *ctx, const cse_instance *in, int ninst, int chun
     const unsigned long long *hist = (const unsigned long long *)(hs + o.hist);
     const double *kz = (const double *)(hs + o.kahan);
     const unsigned long long *nips = (const unsigned long long *)(hs + o.ips);
+    if (*(const int *)(hs + o.err) & 2)
+        return fail(ctx, CSE_ERR_HIP, "internal: an inner product exponent left [-64, 0]");
     const BatchTimes bt = batch_times(ctx, o);
     const double kms = bt.sweep, tms = bt.records + bt.sweep;
     if (kernel_ms) *kernel_ms = kms;

@@ -105,6 +105,7 @@ struct SweepArgs {
     unsigned long long *hist; // HIST_STRIDE per instance
     unsigned long long *ips;  // per instance
     unsigned long long *clock; // readings: records, sweep, results start
+    int *err;                 // bit 1: an inner product left [-64, 0]
     // k_sweep_c*: the sums above are those of copy 0; block b adds to copy
     // b mod TREE_COPIES, copies being copy_words 8-byte words apart
     unsigned copy_words;

@@ -332,17 +332,21 @@ template <int NH, bool HT, int MODE, bool COPIES> DEV void sweep_body(const Swee
         // adds a term: its exponent and phase, whether there is one, its place
         // within the lane and its index's low part
         auto term = [&](int p, int m, bool nz, unsigned gy, unsigned jx) {
+            // an inner product has -64 <= p <= 0; another one is not added (its
+            // place in the histogram may not exist) and fails the call
+            const bool sum = nz && (unsigned)-p <= 64u;
+            if (nz && !sum) atomicOr(A.err, 2);
             if (MODE == 0) {
                 const int row = ((p & 1) << 3) | m;
-                const double s = ldexp(1.0, nz ? 32 + (p >> 1) : -2000);
+                const double s = ldexp(1.0, sum ? 32 + (p >> 1) : -2000);
                 c0 = fma(s_tab.z[row][0], s, c0);
                 c1 = fma(s_tab.z[row][1], s, c1);
                 c2 = fma(s_tab.z[row][2], s, c2);
                 c3 = fma(s_tab.z[row][3], s, c3);
-                const float e = ldexpf(1.f, nz ? p >> 1 : -2000);
+                const float e = ldexpf(1.f, sum ? p >> 1 : -2000);
                 kahan1(sr, cr, s_tab.f[row][0] * e);
                 kahan1(si, ci, s_tab.f[row][1] * e);
-            } else if (nz && (int)gy >= rl) {
+            } else if (sum && (int)gy >= rl) {
                 const bool off = (int)gy != rl;
                 const int P = p - sexp;
                 kahan1(sr, cr, ldexpf(s_tab.f[((P & 1) << 3) | m][0], (P >> 1) + (off ? 1 : 0)));

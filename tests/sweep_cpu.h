@@ -211,8 +211,8 @@ int sweep_add(int mode, int n, int k, int exact, int G, const uint8_t *ub, const
     item_off.push_back(item_off.back() + (d.lanes + 255) / 256);
     return (int)item_off.back();
 }
-// Runs it with `grid` blocks whose waves run in the order given.
-void sweep_run(int mode, int nh, int ht, int copies, int grid, const int *order, long long flush_terms, int32_t *terms,
+// Runs it with `grid` blocks whose waves run in the order given; the error flags.
+int sweep_run(int mode, int nh, int ht, int copies, int grid, const int *order, long long flush_terms, int32_t *terms,
                long long *zsum, double *kahan, unsigned long long *hist, unsigned long long *ips, int copy_words) {
     static void (*const fn[2][2][3])(SweepArgs) = {
         {{k_sweep_s32, k_sweep_s48, k_sweep_s64}, {k_sweep_sh32, k_sweep_sh48, k_sweep_sh64}},
@@ -224,6 +224,7 @@ void sweep_run(int mode, int nh, int ht, int copies, int grid, const int *order,
     for (blockIdx.x = 0; blockIdx.x < (unsigned)sign / 64; blockIdx.x++)
         for (threadIdx.x = 0; threadIdx.x < 64; threadIdx.x++) k_leaf_table(leaf.data(), leaf.data() + plain);
     unsigned long long queue[2] = {0, 0}, clock[3];
+    int err = 0;
     std::vector<uint32_t> stack((size_t)stack_words * 256 * (size_t)grid);
     memset(&args, 0, sizeof args);
     args.ninst = (int)inst.size();
@@ -242,6 +243,7 @@ void sweep_run(int mode, int nh, int ht, int copies, int grid, const int *order,
     args.hist = hist;
     args.ips = ips;
     args.clock = clock;
+    args.err = &err;
     args.copy_words = (unsigned)copy_words;
     kernel = copies ? cp[nh / 16] : fn[mode][ht][nh / 16];
     blockDim.x = 256;
@@ -250,6 +252,7 @@ void sweep_run(int mode, int nh, int ht, int copies, int grid, const int *order,
         blockIdx.x = (unsigned)b;
         fiber::run_block(call, order);
     }
+    return err;
 }
 // Adds q to the phase of record r of instance i.
 void sweep_phase(int i, int r, int q) {

@@ -119,7 +119,7 @@ def launch(S, mode, insts, nh, ht, grid, order, flush=1 << 30, copies=0):
     hist, kah, cnt = out["hist"], out["kahan"], ips
     if copies:
         hist, kah, cnt = block[:HIST], block[HIST:HIST + 2].view(np.float64), block[HIST + 2:HIST + 3]
-    S.sweep_run(mode, nh, ht, copies, grid, (ctypes.c_int * 4)(*order), ctypes.c_longlong(flush),
+    out["err"] = S.sweep_run(mode, nh, ht, copies, grid, (ctypes.c_int * 4)(*order), ctypes.c_longlong(flush),
                 ptr(out["terms"], ctypes.c_int32), ptr(out["zsum"], ctypes.c_longlong), ptr(kah, ctypes.c_double),
                 ptr(hist, ctypes.c_ulonglong), ptr(cnt, ctypes.c_ulonglong), words if copies else 0)
     if copies:
@@ -151,6 +151,7 @@ def packed(t):
 
 
 def check_sampled(out, insts, ref):
+    assert out["err"] == 0
     at = tat = 0
     for d, t in zip(insts, ref):
         chi = 1 << d["k"]
@@ -176,6 +177,7 @@ def hist_of(d, t):
 
 
 def check_exact(out, insts, ref):
+    assert out["err"] == 0
     terms = [packed(t)[np.triu_indices(1 << d["k"])] for d, t in zip(insts, ref)]
     assert np.array_equal(out["terms"], np.concatenate(terms))
     for i, (d, t) in enumerate(zip(insts, ref)):
@@ -234,3 +236,27 @@ def test_copies_add_up(S):
     d = [instance(S, rnd, 1, 12, 6, 0)]
     ref = terms_of(S, d, exact=True)
     check_exact(launch(S, 1, d, 0, 0, d[0]["items"], ORDERS[1], copies=1), d, ref)
+
+
+# a record that no projection gives, with more summed slots than its state has
+@pytest.mark.parametrize("mode", [0, 1])
+@pytest.mark.parametrize("n,extra", [(3, 3), (3, 29)])
+def test_an_exponent_out_of_range_is_flagged_and_not_added(S, mode, n, extra):
+    rnd = random.Random(9)
+    S.sweep_begin()
+    # every summed slot a factor 2: the term of index 0 has p = extra
+    bad = [n << 8, word((1 << n + extra) - 1), 0, 0] + [0] * 64
+    ok = record(rnd, n)
+    d = [instance(S, rnd, mode, n, 1, 0, count=2, first=n, rec=[bad, ok])]
+    ref = terms_of(S, d, exact=mode == 1)
+    assert tuple(ref[0][0, 0][:2]) == (1, extra)
+    out = launch(S, mode, d, 0, 0, 1, ORDERS[0])
+    assert out["err"] == 2
+    ref[0][0, ref[0][0, :, 1] > 0, 0] = 0
+    if mode == 0:
+        for r in range(2):
+            want = np.sum([zomega(int(p), int(m)) for e, p, m in ref[0][r] if e] or [[0] * 4], axis=0)
+            assert np.array_equal(out["zsum"][r], want)
+    else:
+        got = out["hist"][0].astype(np.int64)
+        assert got.sum() == sum(2 * (j > r) + (j == r) for r in range(2) for j in range(r, 2) if ref[0][r, j, 0])
