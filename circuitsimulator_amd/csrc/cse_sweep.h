@@ -37,11 +37,16 @@ DEV void tri_item(long long l, long long ch, long long nch, long long &r, long l
     c = g + off % per;
 }
 
-// Kahan step: sum s with compensation c, plus v
+// Compensated FP32 sum s - c, plus v.  The rounding error of s + v is taken by
+// Knuth's two-sum, exact whichever of the two is larger, and only summed up in
+// c: what is lost is of the order of n eps^2, so a lane's sum has the error of
+// its FP32 terms alone, however many it adds.  (Kahan's own step loses part of
+// the error wherever a term is larger than the sum so far: over random terms
+// the relative error is 3.0e-8 with runs of 4, 3.7e-8 with runs of 32, 3.9e-8
+// with runs of 256; this one 3.0e-8.)
 DEV void kahan1(float &s, float &c, float v) {
-    const float y = v - c;
-    const float t = s + y;
-    c = (t - s) - y;
+    const float t = s + v, b = t - s;
+    c -= (s - (t - b)) + (v - b);
     s = t;
 }
 
@@ -147,11 +152,11 @@ struct TermTables {
             }
             z[t][k] = v;
         }
-        const float mag = t < 8 ? 1.f : 1.41421356237309505f;
-        const float c = m == 0 ? 1.f : m == 4 ? -1.f : m == 2 || m == 6 ? 0.f : m == 1 || m == 7 ? r : -r;
-        const float s = m == 2 ? 1.f : m == 6 ? -1.f : m == 0 || m == 4 ? 0.f : m == 1 || m == 3 ? r : -r;
-        f[t][0] = mag * c;
-        f[t][1] = mag * s;
+        // the nearest FP32 numbers (sqrt2 sqrt1/2 is 1, its FP32 product is not:
+        // that alone is half of the sums' error)
+        const float one = t < 8 ? 1.f : 1.41421356237309505f, half = t < 8 ? r : 1.f;
+        f[t][0] = m == 0 ? one : m == 4 ? -one : m == 2 || m == 6 ? 0.f : m == 1 || m == 7 ? half : -half;
+        f[t][1] = m == 2 ? one : m == 6 ? -one : m == 0 || m == 4 ? 0.f : m == 1 || m == 3 ? half : -half;
     }
 };
 
@@ -186,14 +191,17 @@ template <int NH, bool HT, int MODE, bool COPIES> DEV void sweep_body(const Swee
     long long pend = 0;         // MODE 1: terms counted since the last flush
     unsigned long long ips = 0; // per lane, of instance cur
     // the lane's sums: Z[w] coefficients at scale 2^32 as integers in FP64
-    // (at most 2^G 2^32 <= 2^44, exact), Kahan FP32 pair
+    // (at most 2^G 2^32 <= 2^44, exact) and the compensated FP32 pair of an
+    // item's terms; MODE 1 adds the items' real parts up in s_k, a wave each
     double c0 = 0.0, c1 = 0.0, c2 = 0.0, c3 = 0.0;
     float sr = 0.f, cr = 0.f, si = 0.f, ci = 0.f;
     if (blockIdx.x == 0 && tid == 0) A.clock[1] = wall_clock64();
     s_tab.fill(tid);
     for (int b = tid; b < 1 << tree::LeafBits<HT>::value; b += 256) s_leaf[b] = A.leaf[b];
-    if (MODE == 1)
+    if (MODE == 1) {
         for (int b = tid; b < HIST_STRIDE; b += 256) hist[b] = 0;
+        if (x == 0) s_k[wv] = 0.0;
+    }
     // Other waves read the tables and add to the histogram, and no barrier of
     // the first item comes before that.
     __syncthreads();
@@ -201,12 +209,7 @@ template <int NH, bool HT, int MODE, bool COPIES> DEV void sweep_body(const Swee
     // adds the block's sums of instance cur to the global ones (whole block)
     auto flush = [&]() {
         const unsigned long long wi = (unsigned long long)wave_sum64((long long)ips);
-        double wk = 0.0;
-        if (MODE == 1) wk = wave_sumf64((double)sr - (double)cr);
-        if (x == 0) {
-            s_ips[wv] = wi;
-            s_k[wv] = wk;
-        }
+        if (x == 0) s_ips[wv] = wi;
         __syncthreads();
         const unsigned copy = COPIES ? (blockIdx.x % TREE_COPIES) * A.copy_words : 0u;
         if (tid == 0) {
@@ -225,11 +228,11 @@ template <int NH, bool HT, int MODE, bool COPIES> DEV void sweep_body(const Swee
                 atomicAdd(&h[b], (unsigned long long)v << (m == 4 ? 1 : 0));
                 if (m & 3) atomicAdd(&h[(b & ~7) | (8 - m)], (unsigned long long)v);
             }
-            sr = cr = 0.f;
         }
         ips = 0;
         pend = 0;
         __syncthreads();
+        if (MODE == 1 && x == 0) s_k[wv] = 0.0;
     };
 
     auto run_item = [&](long long item) {
@@ -325,10 +328,8 @@ template <int NH, bool HT, int MODE, bool COPIES> DEV void sweep_body(const Swee
             // the one lane that holds its diagonal
             if (valid && rl >= 0) ips += (unsigned long long)(D->chi - (long long)ri);
         }
-        if (MODE == 0) {
-            c0 = c1 = c2 = c3 = 0.0;
-            sr = cr = si = ci = 0.f;
-        }
+        if (MODE == 0) c0 = c1 = c2 = c3 = 0.0;
+        sr = cr = si = ci = 0.f;
         // adds a term: its exponent and phase, whether there is one, its place
         // within the lane and its index's low part
         auto term = [&](int p, int m, bool nz, unsigned gy, unsigned jx) {
@@ -465,6 +466,12 @@ template <int NH, bool HT, int MODE, bool COPIES> DEV void sweep_body(const Swee
             f.Ah ^= tah;
         }
     summed:
+        if (MODE == 1) {
+            // (a lane's own sum across its items would take two registers that
+            // the loop has not got: scratch of the 32-slot kernel 20 -> 56 bytes)
+            const double wk = wave_sumf64((double)sr - (double)cr);
+            if (x == 0) s_k[wv] += wk;
+        }
         if (MODE == 0) {
             if (valid) ips += (unsigned long long)lg;
             // the record's sums over the lanes that share it (integers below

@@ -4,6 +4,7 @@ eliminated by itself: a block's shared tables are complete before any wave
 reads them, in whatever order its waves run; the claim loop takes every item
 once; partial sums are flushed whole; a lane's FP32 sums are short."""
 import ctypes
+import math
 import os
 import random
 import shutil
@@ -260,3 +261,36 @@ def test_an_exponent_out_of_range_is_flagged_and_not_added(S, mode, n, extra):
     else:
         got = out["hist"][0].astype(np.int64)
         assert got.sum() == sum(2 * (j > r) + (j == r) for r in range(2) for j in range(r, 2) if ref[0][r, j, 0])
+
+
+# What the FP32 sums may be off: a term is the FP32 number nearest to its value
+# (2^-24 of it), and n additions lose at most about n^2 2^-48 of the sum of
+# magnitudes besides.
+@pytest.mark.parametrize("mode", [0, 1])
+@pytest.mark.parametrize("n,k,G,signs", [(20, 8, 8, 0), (16, 8, 7, 1), (52, 7, 6, 0)])
+def test_fp32_sums_carry_only_their_terms_rounding(S, mode, n, k, G, signs):
+    rnd = random.Random(31 * n + k)
+    S.sweep_begin()
+    d = [instance(S, rnd, mode, n, k, G, signs, count=4, first=1)]
+    ref = terms_of(S, d, exact=mode == 1)[0]
+    out = launch(S, mode, d, nh_of(n), signs, 1, ORDERS[0])
+
+    def of(p, m):  # the nearest FP32 numbers
+        zero = (m % 4 == 2, m % 4 == 0)
+        return tuple(0.0 if z else float(np.float32(2.0 ** (p / 2) * f(math.pi * m / 4)))
+                     for z, f in zip(zero, (math.cos, math.sin)))
+
+    tot = [0.0, 0.0, 0.0]
+    for r in range(d[0]["count"]):
+        if mode == 0:
+            tot = [0.0, 0.0, 0.0]
+        sexp = int(d[0]["recs"][r][0] >> 24 & 0xffff) if mode == 1 else 0
+        vals = [tuple((1 + (mode == 1 and j > r)) * c for c in of(int(p) - sexp, int(m)))
+                for j, (e, p, m) in enumerate(ref[r]) if e and (mode == 0 or j >= r)]
+        tot = [math.fsum([tot[0]] + [v[0] for v in vals]), math.fsum([tot[1]] + [v[1] for v in vals]),
+               math.fsum([tot[2]] + [max(map(abs, v)) for v in vals])]
+        if mode == 0:
+            for q in range(2):
+                assert abs(out["kahan"][r, q] - tot[q]) <= (1 << 2 * G) * 2.0 ** -48 * tot[2]
+    if mode == 1:
+        assert abs(out["kahan"][0, 0] - tot[0]) <= (1 << 2 * G) * 2.0 ** -48 * tot[2]
