@@ -25,7 +25,9 @@ struct DevBuf {
 };
 
 // pinned host memory: device-to-host copies into it are single DMA
-// transfers instead of chunked staging through a driver buffer
+// transfers instead of chunked staging through a driver buffer.  Coherent,
+// whatever the process's environment says (HIP_HOST_COHERENT): the host reads
+// results and the call's number while the device may still run.
 struct HostBuf {
     void *p = nullptr;
     size_t cap = 0;
@@ -160,7 +162,7 @@ int ensure_host(cse_ctx *ctx, HostBuf &b, size_t bytes) {
     b.p = nullptr;
     b.cap = 0;
     size_t want = bytes + bytes / 4;
-    hipError_t e = hipHostMalloc(&b.p, want, hipHostMallocDefault);
+    hipError_t e = hipHostMalloc(&b.p, want, hipHostMallocCoherent);
     if (e != hipSuccess) {
         (void)hipGetLastError();
         return fail(ctx, CSE_ERR_NOMEM, "hipHostMalloc(%zu): %s", want, hipGetErrorString(e));
