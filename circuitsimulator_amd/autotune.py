@@ -5,12 +5,13 @@ work is cut, never the results.
 more of their elimination, shallower ones give more lanes.  The engine's rule
 (0) prices both for the launch at hand; the candidates bound it further.  The
 sweep kernels that a call may name (cse_set_sweep_kernel) are one per mode and
-width, so the kernel half of a candidate changes nothing.
+width, so the kernel half of a candidate changes nothing and each bound is
+timed once per name; bounds between two powers of two act as the lower one.
 
 Every setting gives the same terms and the same exact results (integer sums,
 independent of order), so the choice is a timing question only.
 tune_exact / tune_sampled time each candidate on the device (the
-sweep's HIP-event time, best of `reps`) on a proxy of the workload, together
+sweep's time by the device's clock, best of `reps`) on a proxy of the workload, together
 with the engine's own rule, and return the fastest, cached per (device, kind,
 shape key) for the process.  The engine's rule stays unless a candidate
 beats it by more than `tol`.
@@ -33,10 +34,12 @@ CANDIDATES = (128, 192, 256, 384, 512, 1024)
 KERNELS = (1, 2)
 # exact mode: bounds on a lane's terms
 EXACT_CAPS = (256, 512, 1024, 2048, 4096)
-# waves per CU that a launch is sized by for the proxy
+# waves per CU that the proxy is sized by (resident are 16, beyond 48 qubits 12:
+# the proxy is that much longer than it has to be)
 _WAVES_PER_CU = {"exact": 7 * 4, "sampled": 8 * 4}
-# widths up to this share a cache key
-_PACKED_MAX_T = 60
+# the sweep has a kernel each for states up to these widths and one beyond; a
+# choice made for one does not hold for another
+_WIDTHS = (32, 48)
 
 _cache = {}
 _lock = threading.Lock()
@@ -68,12 +71,12 @@ def _exact_fields(instances):
 
 def _key(E, kind, ts, hdec, chis, items):
     cus, name = E.device_info()
-    packed = max(ts) <= _PACKED_MAX_T
+    width = sum(max(ts) > w for w in _WIDTHS)
     waves = cus * _WAVES_PER_CU[kind]
     # items per wave in octaves, saturating where the launch is throughput-bound
     load = min(int(math.log2(max(1.0, items / waves))), 6)
     mean_chi = sum(chis) / len(chis)
-    return (name, cus, kind, packed, bool(hdec), load, int(round(math.log2(mean_chi))))
+    return (name, cus, kind, width, bool(hdec), load, int(round(math.log2(mean_chi))))
 
 
 def _best(run, candidates, reps, tol, rule=0):

@@ -146,6 +146,21 @@ def test_exact_key_separates_shapes():
     assert len(E.runs) == 3 * n
 
 
+@pytest.mark.parametrize("kind", ["exact", "sampled"])
+def test_widths_of_different_kernels_do_not_share_a_choice(kind):
+    autotune.clear_cache()
+    E = FakeEngine(exact_cost() if kind == "exact" else sampled_cost())
+    for t, new in [(24, True), (32, False), (33, True), (48, False), (49, True), (64, False)]:
+        n = len(E.runs)
+        if kind == "exact":
+            autotune.tune_exact(E, exact_array([4] * 3, t=t))
+        else:
+            A = sampled_instance_array(2)
+            A["P"]["nqubits"], A["P"]["nstabs"], A["k"], A["count"] = t, 1, 6, 10
+            autotune.tune_sampled(E, A)
+        assert (len(E.runs) > n) == new, t
+
+
 def sampled_cost(best=(2, 384), **kw):
     return cost_table(autotune.CANDIDATES, best, **kw)
 
