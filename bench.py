@@ -35,13 +35,15 @@ CANONICAL_WORDOPS_PER_IP = 14743
 # Per inner product of the sweep kernel on this workload, from rocprofv3
 # --pmc over one dispatch of 2^28 inner products
 # (profiles/sweep_cases.md):
-VALU_INSTS_PER_IP = 36.0     # SQ_INSTS_VALU / inner products (wave64 instructions)
-SALU_INSTS_PER_IP = 1.5      # SQ_INSTS_SALU / inner products
+VALU_INSTS_PER_IP = 34.0     # SQ_INSTS_VALU / inner products (wave64 instructions)
+SALU_INSTS_PER_IP = 1.55     # SQ_INSTS_SALU / inner products
 VALU_LANE_OPS_PER_IP = VALU_INSTS_PER_IP * 64
 # HBM bytes per inner product of the sweep: (FETCH_SIZE x 2.000 + WRITE_SIZE x
 # 1.000) KiB, factors from a 1 GiB copy kernel, / inner products
-SWEEP_BYTES_PER_IP = 53.7
-CLOCK_GHZ = 2.28             # GRBM_GUI_ACTIVE / kernel time / 8 XCDs
+SWEEP_BYTES_PER_IP = 52.0
+# a term's exact addition to four integers and its FP32 addition to a pair
+NEEDED_LANE_OPS_PER_IP = 12
+CLOCK_GHZ = 2.37             # GRBM_GUI_ACTIVE / time of a kernel among others / 8 XCDs
 # 256 CU x 2 wave64 instructions per cycle x 2.4 GHz, int32 lane-ops/s: the
 # rate of and, xor, or, bitop3, add, sub and right shifts
 PEAK_INT_TOPS = 78.6
@@ -712,7 +714,10 @@ def main():
     if "tune_s" in tuning:
         out["tuning"] = tuning
     # integer-VALU roofline of the sweep kernel: its executed int32 lane
-    # operations per inner product at the kernel's rate, against the VALU peak
+    # operations per inner product at the kernel's rate, against the VALU peak.
+    # It says how busy the vector units are, not how much of that work a better
+    # method would need: what every method has to do is a term's addition to
+    # its sums (needed_lane_ops_per_ip).
     achieved = kernel_ips * VALU_LANE_OPS_PER_IP / 1e12
     out["roofline"] = {"bound": "valu", "achieved": achieved, "peak": PEAK_INT_TOPS, "unit": "Tops/s",
                        "frac": achieved / PEAK_INT_TOPS,
@@ -720,6 +725,7 @@ def main():
                        "traffic_source": "rocprofv3 FETCH_SIZE/WRITE_SIZE of one sweep dispatch, calibrated",
                        "kernel": "k_sweep_s48",
                        "per_unit": f"{VALU_LANE_OPS_PER_IP:.0f} executed int32 lane-ops per inner product",
+                       "needed_lane_ops_per_ip": NEEDED_LANE_OPS_PER_IP,
                        "unshared_wordops_per_ip": ALG_WORDOPS_PER_IP,
                        "canonical_wordops_per_ip": CANONICAL_WORDOPS_PER_IP}
     # the binding limit: instruction issue (one SALU per CU per cycle, two

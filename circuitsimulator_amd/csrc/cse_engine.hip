@@ -78,7 +78,6 @@ struct cse_ctx {
     char *scratch = nullptr;
     char scratch_err[160] = {0};
     bool thr_ready = false;
-    int sweep_kernel[2] = {0, 0};  // per mode (cse_set_sweep_kernel)
     // exact mode: terms of one instance after which a wave flushes its
     // partial histogram (CSE_FLUSH_TERMS in the environment, at most and by
     // default CSE_FLUSH_TERMS_MAX)
@@ -589,9 +588,9 @@ BatchTimes batch_times(const cse_ctx *ctx, const OutLayout &o) {
 // Cost model of a lane's tree, in VALU instructions: a step of slot c takes
 // about 58 for its own state (a signed one, |H^t>, 8 more) and 7 for every
 // slot below it, a slot beyond 32 14 for those beyond; a term's sums take
-// about 60.  (Since rows are updated through carries it is 6 for every slot
-// below; with 6 here t = 63, k = 10, 512 samples take 138 us for 126 and the
-// others what they took.)
+// about 60.  The 7 is a fit: a row takes 6, but the kernels of wide states also
+// wait for their scratch, which the model has no term for (with 6 t = 63, k =
+// 10, 512 samples take 138 us for 126, and the others what they took).
 double step_cost(int c, bool h) {
     return c < 32 ? 58.0 + (h ? 8 : 0) + 7.0 * c : 90.0 + (h ? 10 : 0) + 7.0 * 32 + 14.0 * (c - 32);
 }
@@ -915,8 +914,7 @@ int cse_set_sweep_kernel(cse_ctx *ctx, int mode, int kernel) {
     if (!ctx) return CSE_ERR_ARG;
     if (mode < 0 || mode > 1) return fail(ctx, CSE_ERR_ARG, "sweep mode %d outside [0, 1]", mode);
     if (kernel < 0 || kernel > 2) return fail(ctx, CSE_ERR_ARG, "sweep kernel %d outside [0, 2]", kernel);
-    ctx->sweep_kernel[mode] = kernel;
-    return CSE_OK;
+    return CSE_OK;  // there is one a mode and width
 }
 
 int cse_set_graphs(cse_ctx *ctx, int enable) {
@@ -1054,8 +1052,10 @@ static void run_jobs(int nw, F &&job) {
     for (std::thread &th : pool) th.join();
 }
 
-// job(lo, hi) over [0, n): on several threads from 128 on (a thread takes
-// about 15 us to start, an instance of a plan about 1 us)
+// job(lo, hi) over [0, n): on several threads from 128 on, where the instances
+// of most launches of that many pay for a thread's start (15 us): one takes 1
+// us at t = 13, k = 5, 2 at t = 40, k = 8, 14 at t = 48, k = 12 and 100 at t =
+// 64, k = 30 (whose 2^30 terms take milliseconds)
 extern "C++" template <class F>
 static void run_ranges(int n, F &&job) {
     const unsigned hw = std::thread::hardware_concurrency();

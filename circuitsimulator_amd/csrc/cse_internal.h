@@ -71,7 +71,6 @@ struct InstDesc {
     int leaf;           // levels up to this one only move the looked-up slots, or pair
     int beyond;         // stack words (per lane) outside LDS
     int levels;         // most slots of a level (tree_levels)
-    int spare;
     int pair;           // leaf is 1, and the terms of index bit 0 are summed in pairs
     uint8_t inv[64];    // column of each slot
     uint8_t ub[TREE_MAXG + 4];    // ub[g]: slots that index bits below g move

@@ -125,9 +125,8 @@ DEV void as_subtract_general(AState &s, const RState &s2) {
 // layout (D_x in bits 61..63 of J_x, n <= 60), one asm block: for each row b
 // of Gbar2 from k2 to n - 1, xi = that row and the right side alpha =
 // h2 . xi; the column is the ballot of the parity of G & xi over the active
-// rows, c = (h2 ^ h) . xi, and the elimination of i = min(S) over S is the
-// exact-mode sweep's (PHIL_RESTRICT_ALL): rows of S take J_i, D_i + 4 J_xi
-// and G_i, the rows of M = J_i (^ S when D_i is in {2,6}) take S, and c = 1
+// rows, c = (h2 ^ h) . xi, and i = min(S) is eliminated over S: rows of S take
+// J_i, D_i + 4 J_xi and G_i, the rows of M = J_i (^ S when D_i is in {2,6}) take S, and c = 1
 // adds D_i to Q (bits 29..31 of s60), 4 to D on M and G_i to h.  Returns 0
 // when a restriction is empty with right side 1 (the product is 0).
 DEV int pk_restrict_general(unsigned &jlo, unsigned &jhi, unsigned &glo, unsigned &ghi, u64 &h, u64 &act,

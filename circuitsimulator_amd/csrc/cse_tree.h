@@ -37,8 +37,9 @@
 // from a bit is and, sub, ashr (not v_bfe_i32), successive row masks are ashr
 // and add (not v_bfe_i32 at each bit), the row of a slot that differs from
 // lane to lane is picked by a tree of bitop3 selects, and counts are sums of
-// masks (not v_bcnt).  With v_bfe_i32 masks a step of slot 10 takes 93
-// instructions at 2.4 per ns and CU, this way 125 at 4.4.
+// masks (not v_bcnt).  With row updates through masks (rows, below, has what
+// they are now) a step of slot 10 took 93 instructions at 2.4 per ns and CU
+// with v_bfe_i32, 125 at 4.4 this way.
 #pragma once
 #include <stdint.h>
 
