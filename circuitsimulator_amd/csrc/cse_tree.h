@@ -56,6 +56,8 @@ constexpr unsigned TA = 0xF0, TB = 0xCC, TC = 0xAA;
 // the three-operand boolean function of truth table F in one instruction
 #define TREE_B3(a, b, c, F) ((cse::tree::u32)__builtin_amdgcn_bitop3_b32((a), (b), (c), (F) & 0xffu))
 #define TREE_POP(v) __popc(v)
+// v is 0 in every lane
+#define TREE_NONE(v) (__builtin_amdgcn_ballot_w64((v) != 0) == 0)
 // the top n bits of v shifted in below i
 #define TREE_SHIN(i, v, n) ((cse::tree::u32)__builtin_amdgcn_alignbit((i), (v), 32 - (n)))
 template <u32 K> TREE_DEV u32 andk(u32 v) {
@@ -180,6 +182,7 @@ template <int K> TREE_DEV void picked(u32 o, u32 *w) {
 #else
 #define TREE_DEV inline
 #define TREE_POP(v) __builtin_popcount(v)
+#define TREE_NONE(v) ((v) == 0)
 inline u32 tree_b3(u32 a, u32 b, u32 c, unsigned F) {
     u32 r = 0;
     for (int i = 0; i < 8; i++)
@@ -319,6 +322,12 @@ template <int NH, bool HT, int C> TREE_DEV void step_hi(Form<NH> &f) {
     const u32 nh = vh | negh;               // top bit: vh is not empty
     const u32 iso = TREE_B3(act, odd, TREE_B3(nh, vl, negl, TA | TB | TC), TA & ~TB & ~TC);
     f.z = TREE_B3(f.z, iso, hi, TA | (TB & TC));
+    // Slots without a row in any lane have no more to do.  The chain of 64 steps
+    // is all that a launch of few terms takes: exact t = 64, k = 0, 5 generators
+    // 72 -> 48 us (one wave a term, rows in lanes: 50 to 58), 20 generators 77 ->
+    // 64 (58 to 62), and 2^28 terms of t = 48 take what they took.  (Below slot
+    // 32 the test gains 3 us more there and costs |H^t> calls 1%.)
+    if (TREE_NONE(vl | vh)) return;
     // the slot solved for, among those from 32 on if there is one
     u32 nhm = nh;
     const u32 ol = TREE_B3(TREE_B3(vl, negl, odd, TA & TB & ~TC), pop_mask(nhm), odd, TA & ~TB);

@@ -7,6 +7,7 @@ import pytest
 from circuitsimulator_amd import Engine
 from circuitsimulator_amd.engine import Instance, Projector
 from circuitsimulator_amd.workloads import commuting_paulis, random_L
+from gpu_util import oracle_exact_terms
 
 pytestmark = pytest.mark.gpu
 
@@ -42,6 +43,26 @@ def test_flushes_within_an_instance(monkeypatch):
         # FP32 terms of at most 2^-24 relative error, signs at random
         assert abs(r.kahan_re - r.re) <= 1e-5 * abs(r.re)
     assert len(set(got.values())) == 1
+
+
+@pytest.mark.parametrize("t,r,k", [(33, 1, 0), (49, 3, 1), (64, 1, 0), (64, 5, 2), (64, 40, 1)])
+def test_slots_without_rows(t, r, k):
+    """Few generators leave most slots without a row in any lane, whose steps
+    end early: every pair term against the oracle."""
+    rng = np.random.default_rng(10 * t + r)
+    ph, xs, zs = commuting_paulis(rng, t, r)
+    L = random_L(rng, t, k) if k else []
+    inst = Instance()
+    inst.P = Projector.make(ph, xs, zs, t)
+    inst.k = k
+    for i, v in enumerate(L):
+        inst.L[i] = v
+    chi = 1 << k
+    with Engine(0) as E:
+        (res,), terms, _ = E.batch_exact([inst], want_terms=True, nterms=chi * (chi + 1) // 2)
+    want = oracle_exact_terms(t, k, L, 0, ph, xs, zs)
+    assert [w[0] for w in want] == list(terms)
+    assert res.im == 0.0
 
 
 def test_results_of_every_size_on_one_context():
